@@ -262,7 +262,7 @@ struct Timer {
 void enqueue_cycle(ArmonBatch* b, int64_t cycle, Timer* t)
 {
     if (t) t->begin();
-    launch_batch_time_step(b->d_states, b->d_cfgs, (int) b->p.size(), b->stream);
+    launch_batch_time_step(b->d_states, b->d_states, b->d_cfgs, (int) b->p.size(), b->stream);
     if (t) t->end(2);
     ArmonParams pc = b->common;
     pc.cycle = (int) cycle;
@@ -617,7 +617,7 @@ ARMON_EXPORT int armon_batch_autotune(ArmonBatch* b, ArmonBatchTuning* out)
             s.active = 1;
             s.current_dt = 1e-7;
             s.next_dt = 1e-7;
-            s.dt_min_bits = 0x7FEFFFFFFFFFFFFFull;   // DBL_MAX
+            for (auto& slot : s.dt_min) slot.bits = kNoBound;
         }
         hip_check(hipMemcpyAsync(b->d_tune, tune.data(), sizeof(DeviceState) * tune.size(), hipMemcpyHostToDevice,
                                  b->stream),

@@ -91,8 +91,7 @@ ARMON_HD bool recip_div_ok(double x)
 // signed zero of a / b. Any operand outside the ranges sends every quotient of the group back
 // to a / b. The rcp instruction runs at a quarter of the FMA rate, so a shared divisor saves
 // about 9 FMA issue slots per extra quotient.
-#if defined(__HIP_DEVICE_COMPILE__)
-ARMON_HD double refined_recip(double b)
+__device__ __forceinline__ double refined_recip(double b)
 {
     double y = __builtin_amdgcn_rcp(b);
     double e = __builtin_fma(-b, y, 1.0);
@@ -101,13 +100,12 @@ ARMON_HD double refined_recip(double b)
     return __builtin_fma(y, e, y);
 }
 
-ARMON_HD double refined_quot(double a, double b, double y)
+__device__ __forceinline__ double refined_quot(double a, double b, double y)
 {
     const double q = a * y;
     const double r = __builtin_fma(b, q, -a);
     return __builtin_fma(-r, y, q);
 }
-#endif
 
 ARMON_HD int shared_divisor_ok(double b) { return (int) (b >= 0x1p-200) & (int) (b <= 0x1p200); }
 
@@ -150,6 +148,40 @@ ARMON_HD void with_divisor_t(T b, Body&& body)
         body([&](T a) { return dv<T>(a, b); });
 }
 
+// Reciprocals that several stages of a sweep share (over the cell's density, its Lagrangian
+// length, the sum of two neighbouring lengths), kept in a register or in LDS and used by quot().
+// FP64: refined_recip for a divisor in [2^-200, 2^200], else NaN, which quot() hands on, so that
+// whoever uses the quotient finds out with one comparison and divides instead. A divisor outside
+// the range, a zero, an infinity or a NaN all come out as NaN. With a divisor in the range the
+// quotient has the bits of a / b for a = +-0 and for every finite |a| >= 2^-700 whose quotient is
+// finite (the quotient is then at least 2^-900 and the remainder exact; an overflow on the way, or
+// an infinite a, gives NaN). FP32-mixed: the native reciprocal.
+template <class T> __device__ __forceinline__ T shared_recip(T b);
+template <> __device__ __forceinline__ double shared_recip<double>(double b)
+{
+    const double y = refined_recip(b);
+    const uint64_t bits = __builtin_bit_cast(uint64_t, y);   // the low half of a NaN may be anything
+    const uint32_t high = (int) (y >= 0x1p-200) & (int) (y <= 0x1p200) ? (uint32_t) (bits >> 32) : 0x7FF80000u;
+    return __builtin_bit_cast(double, (uint64_t) high << 32 | (uint32_t) bits);
+}
+template <> __device__ __forceinline__ float shared_recip<float>(float b) { return __builtin_amdgcn_rcpf(b); }
+
+template <class T> __device__ __forceinline__ T quot(T a, T b, T y);
+template <> __device__ __forceinline__ double quot<double>(double a, double b, double y) { return refined_quot(a, b, y); }
+template <> __device__ __forceinline__ float quot<float>(float a, float, float y) { return a * y; }
+
+// Whether quotients through `y`, or of the numerator `a`, have to be divided instead (FP64 only).
+template <class T> __device__ __forceinline__ int unusable(T y)
+{
+    if constexpr (sizeof(T) == 8) return (int) !(y == y);
+    else return 0;
+}
+template <class T> __device__ __forceinline__ int too_small(T a)
+{
+    if constexpr (sizeof(T) == 8) return (int) (__builtin_fabs(a) < 0x1p-700) & (int) (a != 0);
+    else return 0;
+}
+
 // The compiler's correctly rounded FP64 square root on gfx950 is rsq followed by two corrections
 // (sqrt_core's 10 operations), wrapped by a scaling (operands below 2^-767 are multiplied by
 // 2^256 and the root by 2^-128) and a final select that returns the operand itself for +-0 and
@@ -157,8 +189,7 @@ ARMON_HD void with_divisor_t(T b, Body&& body)
 // unchanged, so sqrt_t runs the 10 operations alone there, with the bits of the library square
 // root, and the library square root for every other operand (zero, subnormal, tiny, infinite,
 // negative or NaN), out of line.
-#if defined(__HIP_DEVICE_COMPILE__)
-ARMON_HD double sqrt_core(double x)
+__device__ __forceinline__ double sqrt_core(double x)
 {
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y;
@@ -171,7 +202,6 @@ ARMON_HD double sqrt_core(double x)
     d = __builtin_fma(-g, g, x);
     return __builtin_fma(d, h, g);
 }
-#endif
 
 ARMON_HD int sqrt_core_ok(double x) { return (int) (x >= 0x1p-767) & (int) (x < __builtin_huge_val()); }
 
@@ -410,6 +440,205 @@ ARMON_HD void projection(T dx, T inv_dx, T dt, T us_i, T us_ip,
         v = div(n_vrho);
         E = div(n_Erho);
     });
+}
+
+// ---- the fused sweeps' form of the arithmetic above -----------------------------------------
+// The same expressions, in the same order, on values that the sweeps keep (rho c, rho dx, the
+// Lagrangian lengths and the refined reciprocals), with the minima and maxima as single
+// instructions. In FP64 each result has the bits of the functions above for all operands (where
+// a shared reciprocal does not serve, the operands are divided); in FP32-mixed likewise.
+//
+// kmin and kmax as v_min / v_max: these return the other operand for a NaN and order -0 below +0.
+// kmax(0, kmin(1, r)) is then max(min(r, 1), 0) for every r (a NaN gives 1, zeros give +0).
+template <class T> __device__ __forceinline__ T fmin_t(T a, T b)
+{
+    if constexpr (sizeof(T) == 8) return __builtin_fmin(a, b);
+    else return __builtin_fminf(a, b);
+}
+template <class T> __device__ __forceinline__ T fmax_t(T a, T b)
+{
+    if constexpr (sizeof(T) == 8) return __builtin_fmax(a, b);
+    else return __builtin_fmaxf(a, b);
+}
+
+template <int L, class T> __device__ __forceinline__ T limiter_t(T r)
+{
+    if constexpr (L == LIM_MINMOD) {
+        return fmax_t(fmin_t(r, T(1)), T(0));
+    } else if constexpr (L == LIM_SUPERBEE) {
+        return fmax_t(fmax_t(fmin_t(2 * r, T(1)), T(0)), fmin_t(r, T(2)));
+    } else {
+        (void) r;
+        return T(1);
+    }
+}
+
+// slope_minmod. For s = +-1 the product s D is D with its sign flipped or not, so the larger
+// difference is |D_p|. max(min(max(|D_p|, 0), s D_m), 0) is kmax(0, kmin(|D_p|, s D_m)) also where
+// one of them is a NaN: 0 for a NaN D_p, |D_p| for a NaN D_m.
+template <class T> __device__ __forceinline__ T slope_minmod_t(T D_p, T D_m)
+{
+    const T s = copysign_t<T>(T(1), D_p);
+    const T m = fmax_t(fmin_t(fmax_t(abs_t<T>(D_p), T(0)), s * D_m), T(0));
+    return copysign_t<T>(m, D_p);
+}
+
+// perfect_gas without g, with y = shared_recip(rho). A quotient of at least 2^-400 over a density in
+// shared_recip's range has a numerator of at least 2^-600, and it lies in sqrt_core's range.
+template <class T> __device__ __forceinline__ void perfect_gas_pc(T gamma, T rho, T E, T u, T v, T y, T& p, T& c)
+{
+    T e = E - T(0.5) * (u * u + v * v);
+    p = (gamma - 1) * rho * e;
+    if constexpr (sizeof(T) == 8) {
+        const double cc = refined_quot(gamma * p, rho, y);
+        c = sqrt_core(cc);
+        if (__builtin_expect(!((int) (cc >= 0x1p-400) & (int) (cc < __builtin_huge_val())), 0))
+            c = sqrt_t<double>(gamma * p / rho);
+    } else {
+        (void) y;
+        c = sqrt_t<T>(dv<T>(gamma * p, rho));
+    }
+}
+
+// dt / dm for dm = rho dx, from y = shared_recip(rho) where that serves (else NaN in FP64): 1 / dm is
+// y / dx exactly for a power of two; for another dx the product y * RN(1 / dx) is within 2^-51 of it
+// and one Newton step refines it.
+template <int DXM, class T> __device__ __forceinline__ T mass_quotient(T dt, T dm, T y, T inv_dx)
+{
+    if constexpr (sizeof(T) == 8) {
+        double z = y * inv_dx;
+        if constexpr (DXM != DX_POW2) z = __builtin_fma(z, __builtin_fma(-dm, z, 1.0), z);
+        const double r = refined_quot(dt, dm, z);
+        return too_small(dt) ? __builtin_nan("") : r;   // dt is the same for all lanes
+    } else if constexpr (DXM == DX_POW2) {
+        return dt * (y * inv_dx);
+    } else {
+        return dv<T>(dt, dm);
+    }
+}
+
+// godunov from the impedances rho c of both cells.
+template <class T>
+__device__ __forceinline__ void face_godunov(T rc_l, T rc_r, T u_im, T u_i, T p_im, T p_i, T& ustar, T& pstar)
+{
+    const T sum = rc_l + rc_r;
+    const T y = shared_recip<T>(sum);
+    const T a = rc_l * u_im + rc_r * u_i + (p_im - p_i);
+    const T b = rc_r * p_im + rc_l * p_i + rc_l * rc_r * (u_im - u_i);
+    ustar = quot<T>(a, sum, y);
+    pstar = quot<T>(b, sum, y);
+    if (__builtin_expect(unusable(ustar) | unusable(pstar) | too_small(a) | too_small(b), 0)) {
+        ustar = dv<T>(a, sum);
+        pstar = dv<T>(b, sum);
+    }
+}
+
+// gad_correct in parts. The differences A = u* - u_left and B = u_right - u* of a face (u or p) are its
+// own terms and, over the neighbouring faces' differences, the limiters' numerators: the face above's
+// A over A + 1e-6, the face below's B over B + 1e-6. theta depends on the masses dm = rho dx and the
+// impedances rho c of both cells.
+template <class T> __device__ __forceinline__ T gad_theta(T dt, T dm_l, T dm_r, T rc_l, T rc_r)
+{
+    T Dm = (dm_l + dm_r) / 2;
+    return T(0.5) * (1 - (rc_l + rc_r) / 2 * dv<T>(dt, Dm));
+}
+
+template <int L, class T> __device__ __forceinline__ T gad_star(T theta, T star, T A, T A_above, T B, T B_below)
+{
+    const T r_m = limiter_t<L>(dv<T>(A_above, A + T(1e-6)));
+    const T r_p = limiter_t<L>(dv<T>(B_below, B + T(1e-6)));
+    return star + theta * (r_p * B - r_m * A);
+}
+
+// The signed upwind length of a face: -(dx - dt u*) with the face below's u* for a donor below, else
+// dx + dt u* with the face above's (a vanishing length keeps its sign).
+template <class T> __device__ __forceinline__ T donor_length(T dx, T dt, T disp, T us_m, T us_p)
+{
+    const T us = disp > 0 ? -us_m : us_p;
+    const T d = dx + dt * us;
+    return disp > 0 ? -d : d;
+}
+
+template <class T> __device__ __forceinline__ void donor_flux_1(T disp, const T (&q)[4], T (&f)[4])
+{
+    f[0] = disp * q[0];
+    for (int k = 1; k < 4; k++) f[k] = sizeof(T) == 8 ? disp * q[k] : disp * (q[0] * q[k]);
+}
+
+// advection_flux_2 in parts: what a cell's slopes scale its differences by (slope_ratios, from its
+// length L, its sums with the neighbours' lengths, S below and S_p above, and their reciprocals),
+// the share of a slope that a face takes (length_factor) and the fluxes. L is dx and an increment:
+// where it is not zero it is at least 2^-53 dx, and so are the sums and Dx, so that the numerators are
+// in quot()'s range. q: rho and, in FP64, its products with u, v and E; in FP32 u, v and E themselves,
+// as the flux fuses their product with rho.
+template <class T>
+__device__ __forceinline__ void slope_ratios(T L, T S, T yS, T S_p, T yS_p, T& r_m, T& r_p)
+{
+    const T two_L = 2 * L;
+    r_m = quot<T>(two_L, S, yS);
+    r_p = quot<T>(two_L, S_p, yS_p);
+    if (__builtin_expect(unusable(r_m) | unusable(r_p), 0)) {
+        r_m = dv<T>(two_L, S);
+        r_p = dv<T>(two_L, S_p);
+    }
+}
+
+template <class T> __device__ __forceinline__ T length_factor(T Dx, T L, T yL)
+{
+    T lf = quot<T>(Dx, 2 * L, T(0.5) * yL);
+    if (__builtin_expect(unusable(lf), 0)) lf = dv<T>(Dx, 2 * L);
+    return lf;
+}
+
+template <class T>
+__device__ __forceinline__ void donor_flux_2(T disp, T lf, const T (&q)[4], const T (&slope)[4], T (&f)[4])
+{
+    f[0] = disp * (q[0] - slope[0] * lf);
+#pragma unroll
+    for (int k = 1; k < 4; k++)
+        f[k] = sizeof(T) == 8 ? disp * (q[k] - slope[k] * lf) : disp * (q[0] * q[k] - slope[k] * lf);
+}
+
+// What the slopes take differences of, from a cell's rho, u, v and E.
+template <class T> __device__ __forceinline__ T carried(const T (&c)[4], int k) { return k == 0 ? c[0] : c[0] * c[k]; }
+
+// projection from the cell's Lagrangian length.
+template <int DXM, class T>
+__device__ __forceinline__ void project(T dx, T inv_dx, T dX, const T (&f)[4], const T (&fp)[4], T& rho, T& u, T& v, T& E)
+{
+    T n[4];
+    if constexpr (DXM == DX_POW2) {
+        n[0] = (dX * rho - (fp[0] - f[0])) * inv_dx;
+        n[1] = (dX * rho * u - (fp[1] - f[1])) * inv_dx;
+        n[2] = (dX * rho * v - (fp[2] - f[2])) * inv_dx;
+        n[3] = (dX * rho * E - (fp[3] - f[3])) * inv_dx;
+    } else if constexpr (sizeof(T) == 8) {
+        const T a[4] = {dX * rho - (fp[0] - f[0]), dX * rho * u - (fp[1] - f[1]), dX * rho * v - (fp[2] - f[2]),
+                        dX * rho * E - (fp[3] - f[3])};
+        if (__builtin_expect((int) recip_div_ok(a[0]) & (int) recip_div_ok(a[1]) & (int) recip_div_ok(a[2]) &
+                                     (int) recip_div_ok(a[3]),
+                             1)) {
+            for (int k = 0; k < 4; k++) n[k] = div_by_recip(a[k], dx, inv_dx);
+        } else {
+            for (int k = 0; k < 4; k++) n[k] = dv<T>(a[k], dx);
+        }
+    } else {
+        n[0] = dv<T>(dX * rho - (fp[0] - f[0]), dx);
+        n[1] = dv<T>(dX * rho * u - (fp[1] - f[1]), dx);
+        n[2] = dv<T>(dX * rho * v - (fp[2] - f[2]), dx);
+        n[3] = dv<T>(dX * rho * E - (fp[3] - f[3]), dx);
+    }
+    rho = n[0];
+    const T y = shared_recip<T>(n[0]);
+    u = quot<T>(n[1], n[0], y);
+    v = quot<T>(n[2], n[0], y);
+    E = quot<T>(n[3], n[0], y);
+    if (__builtin_expect(unusable(u) | unusable(v) | unusable(E) | too_small(n[1]) | too_small(n[2]) | too_small(n[3]),
+                         0)) {
+        u = dv<T>(n[1], n[0]);
+        v = dv<T>(n[2], n[0]);
+        E = dv<T>(n[3], n[0]);
+    }
 }
 
 // reductions.cpp:18-20: CFL bound of one cell (mask 1 for real cells).

@@ -136,7 +136,7 @@ struct ArmonSolver {
     hipStream_t stream = nullptr;
 
     // fused engine
-    DeviceState* st = nullptr;
+    DeviceState* st = nullptr;       // two: the cycles step from one to the other, from st[0]
     float* f32[10] = {};             // FP32-mixed buffers: A rho,u,v,E | B rho,u,v,E | stale p, c
     int sweeps_per_cycle = 2;
     int64_t cycles_enqueued = 0;
@@ -400,7 +400,6 @@ SweepArgs<T> sweep_args(ArmonSolver* s, int axis, double factor, bool reduce, T*
     a.out_rho = out[0]; a.out_u = out[1]; a.out_v = out[2]; a.out_E = out[3];
     a.stale_p = stale_p;
     a.stale_c = stale_c;
-    a.st = s->st;
     a.nx = p.nx;
     a.ny = p.ny;
     a.row_length = p.row_length;
@@ -449,16 +448,20 @@ struct Timer {
 void fused_enqueue_cycle(ArmonSolver* s, int64_t cycle, Timer* timer)
 {
     const ArmonParams& p = s->p;
-    TimeStepConfig tc{p.cfl, p.Dt, p.max_time, p.max_cycles, p.cst_dt, p.dt_on_even_cycles};
-    if (timer) timer->begin();
-    launch_time_step(s->st, tc, s->stream);
-    if (timer) timer->end(2);
-
+    const TimeStepConfig tc{p.cfl, p.Dt, p.max_time, p.max_cycles, p.cst_dt, p.dt_on_even_cycles};
+    const DeviceState* prev = s->st + (cycle & 1);
+    DeviceState* st = s->st + ((cycle + 1) & 1);
     ArmonParams pc = p;
     pc.cycle = (int) cycle;
     int axes[3];
     double factors[3];
     const int n = armon_split_axes(&pc, axes, factors);
+    // the last sweep adds to the bounds that the first one clears, so the two must be apart
+    const bool folded = n > 1 && p.y_run_rows <= 0 && (int64_t) p.nx * p.ny <= kFoldedCells;
+    if (timer) timer->begin();
+    if (!folded) launch_time_step(prev, st, tc, s->stream);
+    if (timer) timer->end(2);
+
     const SweepVariant var = variant_of(p);
     // buffer parity at the start of this cycle
     int64_t parity = (cycle * s->sweeps_per_cycle) & 1;
@@ -472,12 +475,18 @@ void fused_enqueue_cycle(ArmonSolver* s, int64_t cycle, Timer* timer)
                             s->arr[ARMON_FIELD_WORK4]};
             auto a = sweep_args<double>(s, axes[k], factors[k], reduce, parity ? B : A, parity ? A : B,
                                         s->arr[ARMON_FIELD_PMAT], s->arr[ARMON_FIELD_CMAT]);
+            a.st = st;
+            a.prev = folded && k == 0 ? prev : nullptr;
+            a.step = tc;
             launch_sweep<double>(axes[k], var, a, s->stream);
         } else {
             float* A[4] = {s->f32[0], s->f32[1], s->f32[2], s->f32[3]};
             float* B[4] = {s->f32[4], s->f32[5], s->f32[6], s->f32[7]};
             auto a = sweep_args<float>(s, axes[k], factors[k], reduce, parity ? B : A, parity ? A : B, s->f32[8],
                                        s->f32[9]);
+            a.st = st;
+            a.prev = folded && k == 0 ? prev : nullptr;
+            a.step = tc;
             launch_sweep<float>(axes[k], var, a, s->stream);
         }
         if (timer) timer->end(axes[k] == ARMON_AXIS_X ? 0 : 1);
@@ -532,7 +541,8 @@ void fused_advance(ArmonSolver* s, int64_t n)
 DeviceState read_state(ArmonSolver* s)
 {
     DeviceState h{};
-    hip_check(hipMemcpyAsync(&h, s->st, sizeof h, hipMemcpyDeviceToHost, s->stream), "read device state");
+    hip_check(hipMemcpyAsync(&h, s->st + (s->cycles_enqueued & 1), sizeof h, hipMemcpyDeviceToHost, s->stream),
+              "read device state");
     hip_check(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
     return h;
 }
@@ -993,7 +1003,7 @@ ARMON_EXPORT ArmonSolver* armon_solver_create(const ArmonParams* params)
         for (int f = 0; f < ARMON_FIELD_COUNT; f++)
             hip_check(hipMemsetAsync(s->arr[f], 0xFF, bytes, s->stream), "hipMemset");
         void* st = nullptr;
-        hip_check(hipMalloc(&st, sizeof(DeviceState)), "hipMalloc(state)");
+        hip_check(hipMalloc(&st, 2 * sizeof(DeviceState)), "hipMalloc(states)");
         s->st = static_cast<DeviceState*>(st);
         if (s->p.engine == ARMON_ENGINE_FUSED && s->p.precision == ARMON_PREC_FP32_MIXED) {
             for (int k = 0; k < 10; k++) {

@@ -13,58 +13,20 @@ using namespace sweep;
 
 namespace {
 
-// ---------------------------------------------------------------------------------------
-// Time step (armon_2D.cpp:212-252 and the loop condition of :347)
-// ---------------------------------------------------------------------------------------
-
-__device__ __forceinline__ void time_step(DeviceState* st, const TimeStepConfig& c)
+__global__ void k_time_step(const DeviceState* prev, DeviceState* st, TimeStepConfig c)
 {
-    if (st->error || !(st->time < c.max_time && st->cycle < c.max_cycles)) {
-        st->active = 0;
-        return;
-    }
-    double current = st->next_dt;
-    double next;
-    if (c.cst_dt) {
-        next = c.Dt;
-    } else if (!c.dt_on_even_cycles || (st->cycle % 2 == 0) || current == 0) {
-        const double dt = bits_to_double(st->dt_min_bits);
-        double local;
-        if (!finite_d(dt) || dt <= 0) local = dt;
-        else if (current == 0) local = c.cfl * dt;
-        else local = kmin(c.cfl * dt, 1.05 * current);
-        if (!finite_d(local) || local <= 0) {
-            st->error = 1;
-            st->error_cycle = st->cycle;
-            st->error_dt = local;
-            st->active = 0;
-            return;
-        }
-        next = local;
-    } else {
-        next = current;
-    }
-    if (st->cycle == 0) current = next;
-    st->current_dt = current;
-    st->next_dt = next;
-    st->dt_min_bits = double_to_bits(DBL_MAX);
-    st->time += current;
-    st->cycle += 1;
-    st->active = 1;
+    write_step(st, next_step(prev, c));
 }
 
-__global__ void k_time_step(DeviceState* st, TimeStepConfig c)
+// One wave per domain.
+__global__ void __launch_bounds__(256) k_batch_time_step(const DeviceState* prev, DeviceState* states,
+                                                         const TimeStepConfig* cfgs, int n)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) time_step(st, c);
+    const int d = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    if (d < n) write_step(states + d, next_step(prev + d, cfgs[d]));
 }
 
-__global__ void k_batch_time_step(DeviceState* states, const TimeStepConfig* cfgs, int n)
-{
-    const int d = blockIdx.x * blockDim.x + threadIdx.x;
-    if (d < n) time_step(states + d, cfgs[d]);
-}
-
-__global__ void k_reset_min(DeviceState* st) { st->dt_min_bits = double_to_bits(DBL_MAX); }
+__global__ void k_reset_min(DeviceState* st) { st->dt_min[threadIdx.x].bits = kNoBound; }
 
 template <class T>
 __global__ void __launch_bounds__(256) k_cfl_real(DeviceState* st, const T* u, const T* v, const T* c, int nx, int ny,
@@ -119,15 +81,16 @@ template int batch_resident_blocks<double>(int, const SweepVariant&, int);
 
 int x_tile_outputs(const SweepVariant& v, int tile) { return tile - 2 * read_extent(v.flux, v.proj); }
 
-void launch_time_step(DeviceState* st, const TimeStepConfig& c, hipStream_t s)
+void launch_time_step(const DeviceState* prev, DeviceState* st, const TimeStepConfig& c, hipStream_t s)
 {
-    k_time_step<<<1, 64, 0, s>>>(st, c);
+    k_time_step<<<1, 64, 0, s>>>(prev, st, c);
     check_launch("time_step");
 }
 
-void launch_batch_time_step(DeviceState* states, const TimeStepConfig* cfgs, int n, hipStream_t s)
+void launch_batch_time_step(const DeviceState* prev, DeviceState* states, const TimeStepConfig* cfgs, int n,
+                            hipStream_t s)
 {
-    k_batch_time_step<<<(unsigned) ((n + 63) / 64), 64, 0, s>>>(states, cfgs, n);
+    k_batch_time_step<<<(unsigned) ((n + 3) / 4), 256, 0, s>>>(prev, states, cfgs, n);
     check_launch("batch_time_step");
 }
 
@@ -135,7 +98,7 @@ template <class T>
 void launch_cfl_real(DeviceState* st, const T* u, const T* v, const T* c, int nx, int ny, int row_length,
                      int index_start, double cfl_dx, double cfl_dy, hipStream_t s)
 {
-    k_reset_min<<<1, 1, 0, s>>>(st);
+    k_reset_min<<<1, kDtSlots, 0, s>>>(st);
     check_launch("cfl_reset");
     k_cfl_real<T><<<grid_for((int64_t) nx * ny, 256, 2048), 256, 0, s>>>(st, u, v, c, nx, ny, row_length, index_start,
                                                                          cfl_dx, cfl_dy);

@@ -147,6 +147,138 @@ __global__ void __launch_bounds__(256) k_check_sqrt(uint64_t seed, int64_t n, un
     if (fast) atomicAdd(&counts[1], fast);
 }
 
+// Values as the sweeps' stages meet them and as they should not: mostly physical states, one in
+// eight a difference that vanishes or nearly does, one in sixteen anything at all.
+__device__ double draw_value(uint64_t& s, bool positive)
+{
+    const uint64_t r = splitmix64(s);
+    const bool neg = !positive && ((r >> 8) & 1);
+    const int span = (int) ((r >> 16) & 0xFFFF);
+    switch (r & 15) {
+    case 0: return (r >> 40) & 1 ? special(r >> 20) : with_exponent(s, -1075 + span % 2099, (r >> 41) & 1);
+    case 1: return neg ? -0.0 : 0.0;
+    case 2: return with_exponent(s, -1075 + span % 1000, neg);
+    default: return with_exponent(s, -12 + span % 25, neg);
+    }
+}
+
+__device__ bool same(double a, double b) { return to_bits(a) == to_bits(b) || (!(a == a) && !(b == b)); }
+
+// The fused sweeps' form of each stage against the plain one (godunov, gad_correct with every
+// limiter, the two divisions of cell_update, advection_flux_2 for both donors, projection in both
+// ways of dividing by dx, perfect_gas). counts[0]: results that differ; counts[1]: samples whose
+// shared reciprocals all served; first[0]: the index of a differing sample, first[1]: the stages.
+__global__ void __launch_bounds__(256) k_check_stages(uint64_t seed, int64_t n, unsigned long long* counts,
+                                                       double* first, int* first_taken)
+{
+    using namespace armon;
+    unsigned long long bad = 0, fast = 0;
+    for (int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t) gridDim.x * blockDim.x) {
+        uint64_t s = seed ^ ((uint64_t) i * 0xD1B54A32D192ED03ull);
+        const bool pow2 = splitmix64(s) & 1;
+        const double dx = pow2 ? with_exponent(s, -12, false) : 1.0 / (double) (3 + splitmix64(s) % 10000);
+        const double dx2 = pow2 ? 0x1p-12 : dx, inv_dx = 1.0 / dx2;
+        const double dt = (splitmix64(s) & 63) == 0 ? draw_value(s, true) : dx2 * 0x1p-3 * with_exponent(s, 0, false);
+        double rho[4], c[4], u[4], v[4], E[4], us[4];
+        for (int k = 0; k < 4; k++) {
+            rho[k] = draw_value(s, true);
+            c[k] = draw_value(s, true);
+            u[k] = draw_value(s, false);
+            v[k] = draw_value(s, false);
+            E[k] = draw_value(s, true);
+            us[k] = k && (splitmix64(s) & 7) == 0 ? us[k - 1] : draw_value(s, false);
+        }
+        int wrong = 0;
+        bool shared = true;
+        {   // faces: p stands in E's place
+            double a, b, x, y;
+            godunov<double, false>(rho[1], rho[0], c[1], c[0], u[1], u[0], E[1], E[0], a, b);
+            face_godunov<double>(rho[0] * c[0], rho[1] * c[1], u[0], u[1], E[0], E[1], x, y);
+            wrong |= (same(a, x) && same(b, y) ? 0 : 1);
+            auto gad = [&]<int L>() {
+                gad_correct<L, double>(dt, dx2, rho[0], rho[1], c[0], c[1], u[0], u[1], E[0], E[1], us[0], v[0], us[1],
+                                       v[1], us[2], v[2], a, b);
+                const double th = gad_theta<double>(dt, rho[0] * dx2, rho[1] * dx2, rho[0] * c[0], rho[1] * c[1]);
+                x = gad_star<L, double>(th, us[1], us[1] - u[0], us[2] - u[1], u[1] - us[1], u[0] - us[0]);
+                y = gad_star<L, double>(th, v[1], v[1] - E[0], v[2] - E[1], E[1] - v[1], E[0] - v[0]);
+                wrong |= (same(a, x) && same(b, y) ? 0 : 2);
+            };
+            gad.template operator()<0>();
+            gad.template operator()<1>();
+            gad.template operator()<2>();
+        }
+        {   // update: rho and dt / dm
+            const double y = shared_recip<double>(rho[0]), dm = rho[0] * dx2;
+            double q = pow2 ? mass_quotient<DX_POW2>(dt, dm, y, inv_dx) : mass_quotient<DX_RECIP>(dt, dm, y, inv_dx);
+            const int no = unusable(q);
+            if (no) q = dt / dm;
+            wrong |= (same(q, dt / dm) ? 0 : 4);
+            const double L = dx2 + dt * (us[1] - us[0]), yL = shared_recip<double>(L);
+            double r = quot<double>(dm, L, yL);
+            if (no | unusable(yL)) r = dm / L;
+            shared &= !(no | unusable(yL));
+            wrong |= (same(r, dm / L) ? 0 : 8);
+            double p0, c0, g0, p1, c1;
+            perfect_gas<double>(1.4, rho[0], E[0], u[0], v[0], p0, c0, g0);
+            perfect_gas_pc<double>(1.4, rho[0], E[0], u[0], v[0], y, p1, c1);
+            wrong |= (same(p0, p1) && same(c0, c1) ? 0 : 16);
+        }
+        {   // advection from the donor 1 with neighbours 0 and 2; its faces carry us[1] and us[2]
+            double L[3], yS[4], q[3][4];
+            for (int k = 0; k < 3; k++) {
+                L[k] = dx2 + dt * (us[k + 1] - us[k]);
+                q[k][0] = rho[k];
+                q[k][1] = rho[k] * u[k];
+                q[k][2] = rho[k] * v[k];
+                q[k][3] = rho[k] * E[k];
+            }
+            for (int k = 1; k < 3; k++) yS[k] = shared_recip<double>(L[k] + L[k - 1]);
+            for (int up = 0; up < 2; up++) {
+                // up: the face above the donor (u* > 0 there), else the face below it
+                const double disp = dt * us[up ? 2 : 1];
+                if (up ? !(disp > 0) : disp > 0) continue;
+                const double plain = up ? -(dx2 - dt * us[1]) : dx2 + dt * us[2];
+                const double Dx = donor_length<double>(dx2, dt, disp, us[1], us[2]);
+                double a[4], f[4];
+                advection_flux_2<double>(dx2, dt, disp, plain, us[0], us[1], us[2], us[3], rho[0], rho[1], rho[2],
+                                         u[0], u[1], u[2], v[0], v[1], v[2], E[0], E[1], E[2], a[0], a[1], a[2], a[3]);
+                double r_m, r_p, slope[4];
+                slope_ratios<double>(L[1], L[1] + L[0], yS[1], L[2] + L[1], yS[2], r_m, r_p);
+                for (int k = 0; k < 4; k++)
+                    slope[k] = slope_minmod_t<double>(r_p * (q[2][k] - q[1][k]), r_m * (q[1][k] - q[0][k]));
+                donor_flux_2<double>(disp, length_factor<double>(Dx, L[1], shared_recip<double>(L[1])), q[1], slope,
+                                     f);
+                for (int k = 0; k < 4; k++) wrong |= (same(a[k], f[k]) ? 0 : 32);
+            }
+        }
+        {   // projection, from fluxes of any kind
+            const double f[4] = {draw_value(s, false), draw_value(s, false), draw_value(s, false), draw_value(s, false)};
+            const double fp[4] = {draw_value(s, false), (splitmix64(s) & 3) ? f[1] : draw_value(s, false),
+                                  draw_value(s, false), draw_value(s, false)};
+            double a[4] = {rho[0], u[0], v[0], E[0]}, b[4] = {rho[0], u[0], v[0], E[0]};
+            const double L = dx2 + dt * (us[1] - us[0]);
+            if (pow2) {
+                projection<DX_POW2, double, false>(dx2, inv_dx, dt, us[0], us[1], f[0], fp[0], f[1], fp[1], f[2], fp[2],
+                                                   f[3], fp[3], a[0], a[1], a[2], a[3]);
+                project<DX_POW2, double>(dx2, inv_dx, L, f, fp, b[0], b[1], b[2], b[3]);
+            } else {
+                projection<DX_RECIP, double, false>(dx2, inv_dx, dt, us[0], us[1], f[0], fp[0], f[1], fp[1], f[2],
+                                                    fp[2], f[3], fp[3], a[0], a[1], a[2], a[3]);
+                project<DX_RECIP, double>(dx2, inv_dx, L, f, fp, b[0], b[1], b[2], b[3]);
+            }
+            for (int k = 0; k < 4; k++) wrong |= (same(a[k], b[k]) ? 0 : 64);
+        }
+        bad += (unsigned long long) (wrong != 0);
+        fast += (unsigned long long) shared;
+        if (wrong && atomicCAS(first_taken, 0, 1) == 0) {
+            first[0] = (double) i;
+            first[1] = (double) wrong;
+        }
+    }
+    if (bad) atomicAdd(&counts[0], bad);
+    if (fast) atomicAdd(&counts[1], fast);
+}
+
 using CheckKernel = void (*)(uint64_t, int64_t, unsigned long long*, double*, int*);
 
 // Runs one check kernel over n samples and copies its two counts and, when a sample failed,
@@ -201,4 +333,15 @@ extern "C" __attribute__((visibility("default"))) int armon_selftest_sqrt(uint64
                                                                           double* first_bad)
 {
     return run_check(k_check_sqrt, seed, n, mismatches, fast, first_bad, 1);
+}
+
+// Checks n samples of the sweeps' stages drawn from seed. mismatches: samples with a result whose
+// bits differ from the plain form's; shared: samples whose shared reciprocals served; first_bad: the
+// index of one differing sample and the stages that differ (1 Godunov, 2 GAD, 4 dt / dm, 8 dm / L,
+// 16 EOS, 32 advection, 64 projection). Returns 0, or the HIP error code.
+extern "C" __attribute__((visibility("default"))) int armon_selftest_stages(uint64_t seed, int64_t n,
+                                                                            uint64_t* mismatches, uint64_t* shared,
+                                                                            double* first_bad)
+{
+    return run_check(k_check_stages, seed, n, mismatches, shared, first_bad, 2);
 }

@@ -7,12 +7,13 @@
 // projection, reading the state once and writing it once (out of place, ping-pong buffers).
 //
 //  * X sweep (k_sweep_x): one 256-thread block per tile of a stream of padded rows. Each
-//    thread owns one cell of the tile (outputs plus an R-cell halo on each side, R = ghost
-//    layers read; the batched sweeps can also give each thread 2 cells); the stage results are
-//    exchanged through LDS between barriers. Loads and stores are contiguous.
-//  * Y sweep (k_sweep_y): one thread per column, marching down a run of rows. Every
-//    stage's stencil neighbours along y live in the thread's own registers (a sliding
-//    window), so no LDS and no barriers; consecutive lanes touch consecutive columns.
+//    thread owns one cell of the tile (FP32: two; outputs plus an R-cell halo on each side, R =
+//    ghost layers read); the stage results are exchanged through LDS between barriers. Loads and
+//    stores are contiguous.
+//  * Y sweep of large domains (k_sweep_y): one thread per column, marching down a run of rows.
+//    Every stage's stencil neighbours along y live in the thread's own registers and LDS (a sliding
+//    window); consecutive lanes touch consecutive columns.
+//  * Y sweep of the others (k_sweep_y_tile): the X tile's stages on tiles of 16 columns.
 //  * Both number their blocks XCD by XCD (xcd_block) so that each XCD's L2 serves a
 //    contiguous part of the arrays.
 //  * The batched ensemble (k_batch_x, k_batch_x1, k_batch_y, k_batch_y1) runs the same tile and
@@ -44,19 +45,18 @@ namespace sweep {
 constexpr int kTile = 256;    // X sweep: cells per tile (FP64 single-domain sweep, batched default)
 constexpr int kYBlock = 256;  // Y sweep: columns per block
 
-// Y march: rows per unrolled loop body, the minimum waves per SIMD the register allocation
-// must allow (0: the compiler's choice), and whether the FP64 marches load each row's state
-// one row before they use it (1) or within the row (0).
-#ifndef ARMON_Y_UNROLL
-#define ARMON_Y_UNROLL 4
+// Y march: rows per unrolled loop body (FP64: 4 rows spill, 1 row moves its windows, 982 -> 992 us at
+// 8192^2) and the minimum waves per SIMD the register allocation must allow (0: the compiler's choice).
+#ifndef ARMON_Y_UNROLL_FP64
+#define ARMON_Y_UNROLL_FP64 2
+#endif
+#ifndef ARMON_Y_UNROLL_FP32
+#define ARMON_Y_UNROLL_FP32 2
 #endif
 #ifndef ARMON_Y_WAVES_PER_EU
 #define ARMON_Y_WAVES_PER_EU 3   // the FP64 march's occupancy (168 VGPRs); 0: no hint
 #endif
-#ifndef ARMON_Y_PREFETCH
-#define ARMON_Y_PREFETCH 1
-#endif
-constexpr int kYUnroll = ARMON_Y_UNROLL;
+constexpr int kYUnrollFp64 = ARMON_Y_UNROLL_FP64, kYUnrollFp32 = ARMON_Y_UNROLL_FP32;
 #if ARMON_Y_WAVES_PER_EU > 0
 #define ARMON_Y_OCCUPANCY __attribute__((amdgpu_waves_per_eu(ARMON_Y_WAVES_PER_EU)))
 #else
@@ -66,6 +66,7 @@ constexpr int kYUnroll = ARMON_Y_UNROLL;
 template <class T>
 struct Cell {
     T rho, un, ut, E, p, c;   // un: velocity along the sweep axis, ut: across it
+    T y;                      // shared_recip(rho)
 };
 
 __device__ __forceinline__ double bits_to_double(unsigned long long b) { return __longlong_as_double((long long) b); }
@@ -76,15 +77,27 @@ __device__ __forceinline__ bool finite_d(double x)
     return (double_to_bits(x) & 0x7FF0000000000000ull) != 0x7FF0000000000000ull;
 }
 
-// EOS of one cell (fluid_eos.cpp:9-62). The perfect gas is evaluated in the working
-// precision T; the Bizarrium EOS always in FP64, because its `e - eps_k0` and `p - pk0`
-// terms cancel to a few digits near the reference density (p and c rounded to T).
+// Element at `byte` bytes past a base that is the same for the whole wave: the base stays in scalar
+// registers and the lanes' offsets in one 32-bit register for all arrays.
+template <class T>
+__device__ __forceinline__ T load_at(const T* base, unsigned byte)
+{
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + byte);
+}
+template <class T>
+__device__ __forceinline__ void store_at(T* base, unsigned byte, T v)
+{
+    *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + byte) = v;
+}
+
+// EOS of one cell (fluid_eos.cpp:9-62) with y = shared_recip(rho). The perfect gas is evaluated in
+// the working precision T; the Bizarrium EOS always in FP64, because its `e - eps_k0` and
+// `p - pk0` terms cancel to a few digits near the reference density (p and c rounded to T).
 template <class T, int EOS>
-__device__ __forceinline__ void cell_eos(double gamma, T rho, T u, T v, T E, T& p, T& c)
+__device__ __forceinline__ void cell_eos(double gamma, T rho, T u, T v, T E, T y, T& p, T& c)
 {
     if constexpr (EOS == 0) {
-        T g;
-        perfect_gas<T>((T) gamma, rho, E, u, v, p, c, g);
+        perfect_gas_pc<T>((T) gamma, rho, E, u, v, y, p, c);
     } else {
         double pd, cd, gd;
         bizarrium((double) rho, (double) E, (double) u, (double) v, pd, cd, gd);
@@ -93,40 +106,42 @@ __device__ __forceinline__ void cell_eos(double gamma, T rho, T u, T v, T E, T& 
     }
 }
 
-// Cell `k` (along the sweep axis, `n` real cells) of pencil `q` (row for X, column for Y).
-// Real cells are loaded; ghost layers 1..stencil_width mirror real cells: the real cell's
-// rho, E, p and c, its velocities times the side's factors; deeper ghost layers are read as
-// they are, with p and c from stale_p/stale_c.
+// Cell `k` (along the sweep axis, `n` real cells) of the pencil whose cell 0 lies `first` elements
+// past `base` (the same for the whole wave) and whose cells lie `stride` apart. Real cells are
+// loaded; ghost layers 1..stencil_width mirror real cells: the real cell's rho, E, p and c, its
+// velocities times the side's factors; deeper ghost layers are read as they are, with p and c from
+// stale_p/stale_c.
 template <class T, int AXIS, int EOS>
-__device__ __forceinline__ Cell<T> load_cell(const SweepArgs<T>& a, int q, int k, int n)
+__device__ __forceinline__ Cell<T> load_cell(const SweepArgs<T>& a, int64_t base, int first, int k, int stride, int n)
 {
     int kk = k;
     int mirror = 0;   // 0 real, 1 low side, 2 high side
     bool stale = false;
-    if (k < 0) {
-        if (-k <= a.stencil_width) { kk = -k - 1; mirror = 1; }
-        else stale = true;
-    } else if (k >= n) {
-        if (k - n + 1 <= a.stencil_width) { kk = 2 * n - 1 - k; mirror = 2; }
-        else stale = true;
+    if (__builtin_expect((unsigned) k >= (unsigned) n, 0)) {
+        if (k < 0) {
+            if (-k <= a.stencil_width) { kk = -k - 1; mirror = 1; }
+            else stale = true;
+        } else {
+            if (k - n + 1 <= a.stencil_width) { kk = 2 * n - 1 - k; mirror = 2; }
+            else stale = true;
+        }
     }
-    const int idx = AXIS == 0 ? a.index_start + q * a.row_length + kk : a.index_start + kk * a.row_length + q;
-    T rho = a.in_rho[idx], u = a.in_u[idx], v = a.in_v[idx], E = a.in_E[idx];
+    const unsigned o = (unsigned) (first + kk * stride) * (unsigned) sizeof(T);
+    T rho = load_at(a.in_rho + base, o), u = load_at(a.in_u + base, o), v = load_at(a.in_v + base, o),
+      E = load_at(a.in_E + base, o);
     Cell<T> cell;
-    if (stale) {
-        cell.p = a.stale_p[idx];
-        cell.c = a.stale_c[idx];
-    } else {
-        // a mirror ghost takes the p and c of its real cell (halo_exchange.cpp:23-30): the EOS
-        // of the unscaled state
-        cell_eos<T, EOS>(a.gamma, rho, u, v, E, cell.p, cell.c);
-    }
-    if (mirror == 1) {
-        u = u * (T) a.lo_u;
-        v = v * (T) a.lo_v;
-    } else if (mirror == 2) {
-        u = u * (T) a.hi_u;
-        v = v * (T) a.hi_v;
+    cell.y = shared_recip<T>(rho);
+    // a mirror ghost takes the p and c of its real cell (halo_exchange.cpp:23-30): the EOS of the
+    // unscaled state
+    cell_eos<T, EOS>(a.gamma, rho, u, v, E, cell.y, cell.p, cell.c);
+    if (__builtin_expect(stale | (mirror != 0), 0)) {
+        if (stale) {
+            cell.p = load_at(a.stale_p + base, o);
+            cell.c = load_at(a.stale_c + base, o);
+        } else {
+            u = u * (T) (mirror == 1 ? a.lo_u : a.hi_u);
+            v = v * (T) (mirror == 1 ? a.lo_v : a.hi_v);
+        }
     }
     cell.rho = rho;
     cell.E = E;
@@ -135,46 +150,49 @@ __device__ __forceinline__ Cell<T> load_cell(const SweepArgs<T>& a, int q, int k
     return cell;
 }
 
-// load_cell in two parts, for the Y march, which loads a row's state one row before it makes
-// the cell: where cell `k` comes from (cell_source: the index it is read at, the mirror side or
-// staleness), then the cell from the loaded state (make_cell). The row-ahead loads make the
-// FP64 Y sweep 4-9% faster and the FP32-mixed one 2-3% (its 5 waves per SIMD already cover
-// most of the load latency).
-struct CellSource {
-    int idx;
+// load_cell in two parts, for the Y march, which loads a row's state one row before it makes the
+// cell: where row `k` comes from (the same for the whole wave: the row it is read at, the mirror side
+// or staleness), then the cell from the loaded state.
+struct RowSource {
+    int row;
     int mirror;
     bool stale;
 };
 
 // STALE = false: the caller guarantees that the stencil width covers every ghost layer read
 // (|k| beyond the domain is at most the read extent), so no layer is stale.
-template <class T, int AXIS, bool STALE = true>
-__device__ __forceinline__ CellSource cell_source(const SweepArgs<T>& a, int q, int k, int n)
+template <class T, bool STALE = true>
+__device__ __forceinline__ RowSource row_source(const SweepArgs<T>& a, int k)
 {
-    int kk = k;
-    CellSource s{0, 0, false};
+    RowSource s{k, 0, false};
     if (k < 0) {
-        if (!STALE || -k <= a.stencil_width) { kk = -k - 1; s.mirror = 1; }
+        if (!STALE || -k <= a.stencil_width) { s.row = -k - 1; s.mirror = 1; }
         else s.stale = true;
-    } else if (k >= n) {
-        if (!STALE || k - n + 1 <= a.stencil_width) { kk = 2 * n - 1 - k; s.mirror = 2; }
+    } else if (k >= a.ny) {
+        if (!STALE || k - a.ny + 1 <= a.stencil_width) { s.row = 2 * a.ny - 1 - k; s.mirror = 2; }
         else s.stale = true;
     }
-    s.idx = AXIS == 0 ? a.index_start + q * a.row_length + kk : a.index_start + kk * a.row_length + q;
     return s;
 }
 
-// The cell from its loaded state (rho, u, v, E at s.idx): EOS (or the stale p and c), then the
-// mirror factors.
-template <class T, int AXIS, int EOS, bool STALE = true>
-__device__ __forceinline__ Cell<T> make_cell(const SweepArgs<T>& a, const CellSource& s, T rho, T u, T v, T E)
+// The first cell of row `row` within an array (64-bit, in scalar registers).
+template <class T>
+__device__ __forceinline__ int64_t row_start(const SweepArgs<T>& a, int row)
+{
+    return (int64_t) a.index_start + (int64_t) row * a.row_length;
+}
+
+template <class T, int EOS, bool STALE = true>
+__device__ __forceinline__ Cell<T> make_row_cell(const SweepArgs<T>& a, const RowSource& s, unsigned column, T rho, T u,
+                                                 T v, T E)
 {
     Cell<T> cell;
+    cell.y = shared_recip<T>(rho);
     if (STALE && s.stale) {
-        cell.p = a.stale_p[s.idx];
-        cell.c = a.stale_c[s.idx];
+        cell.p = load_at(a.stale_p + row_start(a, s.row), column);
+        cell.c = load_at(a.stale_c + row_start(a, s.row), column);
     } else {
-        cell_eos<T, EOS>(a.gamma, rho, u, v, E, cell.p, cell.c);   // unscaled, as load_cell
+        cell_eos<T, EOS>(a.gamma, rho, u, v, E, cell.y, cell.p, cell.c);   // unscaled, as load_cell
     }
     if (s.mirror == 1) {
         u = u * (T) a.lo_u;
@@ -185,8 +203,8 @@ __device__ __forceinline__ Cell<T> make_cell(const SweepArgs<T>& a, const CellSo
     }
     cell.rho = rho;
     cell.E = E;
-    cell.un = AXIS == 0 ? u : v;
-    cell.ut = AXIS == 0 ? v : u;
+    cell.un = v;
+    cell.ut = u;
     return cell;
 }
 
@@ -194,49 +212,437 @@ template <class T>
 __device__ __forceinline__ Cell<T> benign_cell()
 {
     Cell<T> c;
-    c.rho = T(1); c.un = T(0); c.ut = T(0); c.E = T(1); c.p = T(1); c.c = T(1);
+    c.rho = T(1); c.un = T(0); c.ut = T(0); c.E = T(1); c.p = T(1); c.c = T(1); c.y = T(1);
     return c;
 }
 
-template <class T, int L>
-__device__ __forceinline__ void face_flux_gad(T dt, T dx, const Cell<T>& m, const Cell<T>& c, T gu_im, T gp_im,
-                                              T gu_i, T gp_i, T gu_ip, T gp_ip, T& us, T& ps)
+// `v` of the lane that a DPP control names, this lane's where that reaches no lane.
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v)
 {
-    gad_correct<L, T>(dt, dx, m.rho, c.rho, m.c, c.c, m.un, c.un, m.p, c.p, gu_im, gp_im, gu_i, gp_i, gu_ip, gp_ip,
-                      us, ps);
+    const uint64_t b = double_to_bits(v);
+    const int lo = (int) (uint32_t) b, hi = (int) (b >> 32);
+    const uint32_t l = (uint32_t) __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false);
+    const uint32_t h = (uint32_t) __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false);
+    return bits_to_double((unsigned long long) h << 32 | l);
 }
 
-__device__ __forceinline__ double wave_min(double v)
+// Minimum over the wave, in lane 63 (no NaN among the operands): neighbours, pairs and halves of each
+// row of 16 lanes, then row 0 into 1 and 2 into 3, then rows 0-1 into 2-3.
+__device__ __forceinline__ double wave_min_last(double v)
 {
-    for (int off = 32; off > 0; off >>= 1) v = kmin(v, __shfl_xor(v, off, 64));
-    return v;
+    v = __builtin_fmin(v, dpp<0xB1>(v));    // quad_perm [1,0,3,2]
+    v = __builtin_fmin(v, dpp<0x4E>(v));    // quad_perm [2,3,0,1]
+    v = __builtin_fmin(v, dpp<0x141>(v));   // row_half_mirror
+    v = __builtin_fmin(v, dpp<0x140>(v));   // row_mirror
+    v = __builtin_fmin(v, dpp<0x142>(v));   // row_bcast:15
+    return __builtin_fmin(v, dpp<0x143>(v));   // row_bcast:31
 }
 
-// Merges a per-lane CFL bound into the device accumulator: one atomic per wave.
+// Merges a per-lane CFL bound into one of the state's accumulators, which the blocks share out among
+// themselves. An accumulator only falls, so a wave whose bound is not below what it reads there (some
+// earlier value at most) has nothing to add, and most waves of a large sweep need no atomic.
 __device__ __forceinline__ void reduce_cfl(DeviceState* st, double local)
 {
-    local = wave_min(local);
-    if ((threadIdx.x & 63) == 0) atomicMin(&st->dt_min_bits, double_to_bits(local));
+    const unsigned long long bits = double_to_bits(wave_min_last(local));
+    unsigned long long* slot = &st->dt_min[(blockIdx.x + (threadIdx.x >> 6)) % kDtSlots].bits;
+    if ((threadIdx.x & 63) == 63 && bits < __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMin(slot, bits);
 }
+
+// The least of a state's accumulators, for every lane of the calling wave.
+__device__ __forceinline__ double least_bound(const DeviceState* st)
+{
+    const int lane = threadIdx.x & 63;
+    const double v = lane < kDtSlots ? bits_to_double(st->dt_min[lane].bits) : DBL_MAX;
+    const uint64_t b = double_to_bits(wave_min_last(v));
+    const uint32_t lo = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) b, 63);
+    const uint32_t hi = (uint32_t) __builtin_amdgcn_readlane((int) (b >> 32), 63);
+    return bits_to_double((unsigned long long) hi << 32 | lo);
+}
+
+// ---------------------------------------------------------------------------------------
+// Time step (armon_2D.cpp:212-252 and the loop condition of :347)
+// ---------------------------------------------------------------------------------------
+
+struct NextStep {
+    double current_dt, next_dt, time, error_dt;
+    int cycle, active, error, error_cycle;
+};
+
+// The next cycle's step from the state `st` and the CFL minimum of its current fields; called by a
+// whole wave, whose lanes all compute it.
+__device__ __forceinline__ NextStep next_step(const DeviceState* st, const TimeStepConfig& c)
+{
+    NextStep s{st->current_dt, st->next_dt, st->time, st->error_dt, st->cycle, 0, st->error, st->error_cycle};
+    if (s.error || !(s.time < c.max_time && s.cycle < c.max_cycles)) return s;
+    double current = s.next_dt;
+    double next;
+    if (c.cst_dt) {
+        next = c.Dt;
+    } else if (!c.dt_on_even_cycles || (s.cycle % 2 == 0) || current == 0) {
+        const double dt = least_bound(st);
+        double local;
+        if (!finite_d(dt) || dt <= 0) local = dt;
+        else if (current == 0) local = c.cfl * dt;
+        else local = kmin(c.cfl * dt, 1.05 * current);
+        if (!finite_d(local) || local <= 0) {
+            s.error = 1;
+            s.error_cycle = s.cycle;
+            s.error_dt = local;
+            return s;
+        }
+        next = local;
+    } else {
+        next = current;
+    }
+    if (s.cycle == 0) current = next;
+    s.current_dt = current;
+    s.next_dt = next;
+    s.time += current;
+    s.cycle += 1;
+    s.active = 1;
+    return s;
+}
+
+// Writes it down, by one whole wave, with the bounds of the fields to come cleared.
+__device__ __forceinline__ void write_step(DeviceState* st, const NextStep& s)
+{
+    if ((threadIdx.x & 63) < kDtSlots) st->dt_min[threadIdx.x & 63].bits = kNoBound;
+    if ((threadIdx.x & 63) != 0) return;
+    st->current_dt = s.current_dt;
+    st->next_dt = s.next_dt;
+    st->time = s.time;
+    st->error_dt = s.error_dt;
+    st->cycle = s.cycle;
+    st->active = s.active;
+    st->error = s.error;
+    st->error_cycle = s.error_cycle;
+}
+
+// Whether the cycle runs, and its dt: as its time step left them, or made here, and written down by the
+// first wave of the block that is told to (`writer`: one block of the launch).
+template <class T>
+__device__ __forceinline__ bool begin_sweep(const SweepArgs<T>& a, bool writer, double& dt)
+{
+    if (a.prev == nullptr) {
+        dt = a.st->current_dt;
+        return a.st->active != 0;
+    }
+    const NextStep s = next_step(a.prev, a.step);
+    if (writer && threadIdx.x < 64) write_step(a.st, s);
+    dt = s.current_dt;
+    return s.active != 0;
+}
+
+// The CFL bound of the cells that a thread has seen (cfl_cell), kept as the largest wave speeds: a
+// correctly rounded dx / a never grows with a, so the smallest bound is the one of the largest speed,
+// and the divisions are made once. max(|u + c|, |u - c|) is |u| + |c| with the same rounding. A cell
+// whose x bound is NaN has no bound, one whose y bound is NaN only that of x, as comparisons that a
+// NaN loses leave it: a NaN speed counts as none (its high half cleared).
+struct CflSpeeds {
+    double x = 0, y = 0;
+    __device__ __forceinline__ void add(double u, double v, double c)
+    {
+        const bool nan_x = !(u + c == u + c), nan_y = !(v + c == v + c);
+        x = __builtin_fmax(x, speed(u, c, nan_x));
+        y = __builtin_fmax(y, speed(v, c, (bool) ((int) nan_x | (int) nan_y)));
+    }
+    __device__ __forceinline__ double bound(double dx, double dy) const
+    {
+        return __builtin_fmin(DBL_MAX, __builtin_fmin(dx / x, dy / y));
+    }
+    static __device__ __forceinline__ double speed(double u, double c, bool none)
+    {
+        const uint64_t b = double_to_bits(__builtin_fabs(u) + __builtin_fabs(c));
+        const uint32_t hi = none ? 0u : (uint32_t) (b >> 32);
+        return bits_to_double((unsigned long long) hi << 32 | (uint32_t) b);
+    }
+};
 
 // ---------------------------------------------------------------------------------------
 // X sweep: LDS-staged row tiles
 // ---------------------------------------------------------------------------------------
 
-// LDS of one X tile: the cell state, the final face fluxes, and a 4-array scratch that holds
-// p, c and the Godunov fluxes until the face fluxes are done (stages 0-2), then the advection
-// fluxes (stages 4-5); a barrier separates the last read of the former from the first write
-// of the latter. 10 arrays: 20 KiB in FP64, so that 8 blocks fit in a CU's LDS.
-template <class T, int TILE = kTile>
-struct SmemX {
-    T rho[TILE], un[TILE], ut[TILE], E[TILE], us[TILE], ps[TILE];
-    T x[4][TILE];
-    __device__ T* p() { return x[0]; }
-    __device__ T* c() { return x[1]; }
-    __device__ T* gu() { return x[2]; }
-    __device__ T* gp() { return x[3]; }
-    __device__ T (&f())[4][TILE] { return x; }
+// LDS of one tile of CELLS slots whose neighbours along the axis lie S slots apart. The values that
+// neighbours read together are stored together, 16 bytes (or 8) an access, and each slot's
+// neighbours are reached by constant offsets from its own address: 2S slots of padding before the
+// tile and S after it stand for the neighbours that the tile's end slots do not have (what is read
+// there is never written by anyone and reaches no output, as outputs lie R slots inside).
+//   stages 0-2: a0 = rho dx, un | a1 = p, rho c     b, f = Godunov's A, B     w = the face's u*, p*
+//   stages 3-4: a0 = rho, rho un | a1 = rho ut, rho E   b = L, 1/L | c = 1/S (see tile_sweep)
+//   stages 4-5: the advection fluxes, in FP64 in w and f, in FP32 in a0 and a1 after one more barrier
+// FP64: 88 bytes a slot, 22.8 KB for a tile of 256: 7 blocks fit in a CU's 160 KB. FP32: 40 bytes, 20.6
+// KB for a tile of 512, 7 blocks too. X sweep at 8192^2: FP64 846 us (96 bytes, 6 blocks: 892; the
+// tile of before, which divided everywhere and exchanged single words: 914), FP32 408 us (48 bytes
+// and no barrier more: 433; before: 416).
+template <class T>
+struct alignas(2 * sizeof(T)) Pair {
+    T x, y;
 };
+template <class T>
+struct alignas(16) Quad {
+    T x, y, z, w;
+};
+
+template <class T, int CELLS, int S>
+struct TileLds;
+
+template <int CELLS, int S>
+struct TileLds<double, CELLS, S> {
+    static constexpr int N = CELLS + 3 * S;
+    static constexpr bool kFluxBarrier = false;
+    using P = Pair<double>;
+    P a0_[N], a1_[N], b_[N], w_[N], f_[N];
+    double c_[N];
+    __device__ __forceinline__ P& a0(int t) { return a0_[t + 2 * S]; }
+    __device__ __forceinline__ P& a1(int t) { return a1_[t + 2 * S]; }
+    __device__ __forceinline__ P& w(int t) { return w_[t + 2 * S]; }
+    __device__ __forceinline__ void put_differences(int t, P A, P B)
+    {
+        b_[t + 2 * S] = A;
+        f_[t + 2 * S] = B;
+    }
+    __device__ __forceinline__ P get_A(int t) { return b_[t + 2 * S]; }
+    __device__ __forceinline__ P get_B(int t) { return f_[t + 2 * S]; }
+    __device__ __forceinline__ void put_state(int t, double dm, double un, double p, double rc)
+    {
+        a0(t) = {dm, un};
+        a1(t) = {p, rc};
+    }
+    __device__ __forceinline__ void get_state(int t, double& dm, double& un, double& p, double& rc)
+    {
+        const P l = a0(t), h = a1(t);
+        dm = l.x; un = l.y; p = h.x; rc = h.y;
+    }
+    // what the slopes read: rho and the products rho u, rho v, rho E
+    __device__ __forceinline__ void put_carried(int t, double rho, double un, double ut, double E)
+    {
+        a0(t) = {rho, rho * un};
+        a1(t) = {rho * ut, rho * E};
+    }
+    __device__ __forceinline__ void get_carried(int t, double (&q)[4])
+    {
+        const P l = a0(t), h = a1(t);
+        q[0] = l.x; q[1] = l.y; q[2] = h.x; q[3] = h.y;
+    }
+    __device__ __forceinline__ void put_lengths(int t, double L, double yL, double yS)
+    {
+        b_[t + 2 * S] = {L, yL};
+        c_[t + 2 * S] = yS;
+    }
+    // around the donor cell t: its length and 1/L, the sums of its length and its neighbours'
+    // lengths and their reciprocals
+    __device__ __forceinline__ void get_lengths(int t, double& L, double& yL, double& lo, double& y_lo, double& hi,
+                                                double& y_hi)
+    {
+        const P l = b_[t + 2 * S];
+        L = l.x;
+        yL = l.y;
+        lo = L + b_[t + S].x;
+        hi = b_[t + 3 * S].x + L;
+        y_lo = c_[t + 2 * S];
+        y_hi = c_[t + 3 * S];
+    }
+    __device__ __forceinline__ void put_flux(int t, const double (&f)[4])
+    {
+        w(t) = {f[0], f[1]};
+        f_[t + 2 * S] = {f[2], f[3]};
+    }
+    __device__ __forceinline__ void get_flux(int t, double (&f)[4])
+    {
+        const P l = w(t), h = f_[t + 2 * S];
+        f[0] = l.x; f[1] = l.y; f[2] = h.x; f[3] = h.y;
+    }
+};
+
+template <int CELLS, int S>
+struct TileLds<float, CELLS, S> {
+    static constexpr int N = CELLS + 3 * S;
+    using P = Pair<float>;
+    using Q = Quad<float>;
+    static constexpr bool kFluxBarrier = true;
+    Q a_[N], b_[N];   // a: the state, what the slopes read, then the fluxes; b: Godunov's A and B, then the lengths
+    P w_[N];
+    __device__ __forceinline__ void put_differences(int t, P A, P B) { b_[t + 2 * S] = {A.x, A.y, B.x, B.y}; }
+    __device__ __forceinline__ P get_A(int t)
+    {
+        const Q v = b_[t + 2 * S];
+        return {v.x, v.y};
+    }
+    __device__ __forceinline__ P get_B(int t)
+    {
+        const Q v = b_[t + 2 * S];
+        return {v.z, v.w};
+    }
+    __device__ __forceinline__ P& w(int t) { return w_[t + 2 * S]; }
+    __device__ __forceinline__ void put_state(int t, float dm, float un, float p, float rc)
+    {
+        a_[t + 2 * S] = {dm, un, p, rc};
+    }
+    __device__ __forceinline__ void get_state(int t, float& dm, float& un, float& p, float& rc)
+    {
+        const Q v = a_[t + 2 * S];
+        dm = v.x; un = v.y; p = v.z; rc = v.w;
+    }
+    // the state itself: its products are taken by the reader, as a flux fuses one of them
+    __device__ __forceinline__ void put_carried(int t, float rho, float un, float ut, float E)
+    {
+        a_[t + 2 * S] = {rho, un, ut, E};
+    }
+    __device__ __forceinline__ void get_carried(int t, float (&q)[4])
+    {
+        const Q v = a_[t + 2 * S];
+        q[0] = v.x; q[1] = v.y; q[2] = v.z; q[3] = v.w;
+    }
+    __device__ __forceinline__ void put_lengths(int t, float L, float yL, float yS)
+    {
+        b_[t + 2 * S] = {L, yL, yS, 0.0f};
+    }
+    __device__ __forceinline__ void get_lengths(int t, float& L, float& yL, float& lo, float& y_lo, float& hi,
+                                                float& y_hi)
+    {
+        const Q l = b_[t + 2 * S], h = b_[t + 3 * S];
+        L = l.x;
+        yL = l.y;
+        y_lo = l.z;
+        y_hi = h.z;
+        lo = hi = 0.0f;   // a quotient is the numerator times the reciprocal
+    }
+    __device__ __forceinline__ void put_flux(int t, const float (&f)[4]) { a_[t + 2 * S] = {f[0], f[1], f[2], f[3]}; }
+    __device__ __forceinline__ void get_flux(int t, float (&f)[4])
+    {
+        const Q v = a_[t + 2 * S];
+        f[0] = v.x; f[1] = v.y; f[2] = v.z; f[3] = v.w;
+    }
+};
+
+// The whole per-axis chain of one tile, from the loaded cells (EOS done) to the projected ones:
+// thread t computes the slots slot[0..CPT), and cell[] holds their new rho, un, ut, E afterwards
+// (c stays the input state's). Every thread of the block calls it; outputs are right for the slots
+// whose R neighbours on both sides are in the tile.
+//
+// What neighbours need is computed once and handed over through LDS: besides the states and fluxes
+// these are each cell's Lagrangian length L = dx + dt (u*_right - u*_left), the sum S of its length
+// and the lower neighbour's, and the refined reciprocals of both, over which the update, the slopes
+// and the length factor of the advection divide (2 reciprocals where there were 4 divisions, and no
+// length computed more than twice). The arithmetic of each result is the reference's, so FP64 keeps
+// the bits of dividing everywhere; operands outside shared_recip's ranges take the divisions.
+template <class T, int FLUX, int PROJ, int DXM, int CELLS, int S, int CPT>
+__device__ __forceinline__ void tile_sweep(T dx, T inv_dx, T dt, TileLds<T, CELLS, S>& sm, const int (&slot)[CPT],
+                                           Cell<T> (&cell)[CPT])
+{
+    constexpr bool GAD = FLUX > 0;
+    constexpr bool E2 = PROJ == 2;
+    // Stage 0: what the faces read.
+    T dm[CPT], rc[CPT], dtdm[CPT];
+    int bad[CPT];
+#pragma unroll
+    for (int k = 0; k < CPT; k++) {
+        dm[k] = cell[k].rho * dx;
+        rc[k] = cell[k].rho * cell[k].c;
+        sm.put_state(slot[k], dm[k], cell[k].un, cell[k].p, rc[k]);
+        dtdm[k] = mass_quotient<DXM>(dt, dm[k], cell[k].y, inv_dx);
+        bad[k] = unusable(dtdm[k]);
+        if (__builtin_expect(bad[k], 0)) dtdm[k] = dv<T>(dt, dm[k]);
+    }
+    __syncthreads();
+
+    // Stages 1-2: the flux at face t, between the cells t-S and t.
+    T us[CPT], ps[CPT];
+    {
+        T dm_m[CPT], un_m[CPT], p_m[CPT], rc_m[CPT];
+#pragma unroll
+        for (int k = 0; k < CPT; k++) {
+            sm.get_state(slot[k] - S, dm_m[k], un_m[k], p_m[k], rc_m[k]);
+            face_godunov<T>(rc_m[k], rc[k], un_m[k], cell[k].un, p_m[k], cell[k].p, us[k], ps[k]);
+        }
+        if constexpr (GAD) {
+            Pair<T> A[CPT], B[CPT];
+#pragma unroll
+            for (int k = 0; k < CPT; k++) {
+                A[k] = {us[k] - un_m[k], ps[k] - p_m[k]};
+                B[k] = {cell[k].un - us[k], cell[k].p - ps[k]};
+                sm.put_differences(slot[k], A[k], B[k]);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < CPT; k++) {
+                const Pair<T> above = sm.get_A(slot[k] + S), below = sm.get_B(slot[k] - S);
+                const T theta = gad_theta<T>(dt, dm_m[k], dm[k], rc_m[k], rc[k]);
+                us[k] = gad_star<FLUX - 1, T>(theta, us[k], A[k].x, above.x, B[k].x, below.x);
+                ps[k] = gad_star<FLUX - 1, T>(theta, ps[k], A[k].y, above.y, B[k].y, below.y);
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < CPT; k++) sm.w(slot[k]) = {us[k], ps[k]};
+    __syncthreads();
+
+    // Stage 3: Lagrangian update of cell t from the faces t and t+S.
+    T us_m[CPT], us_p[CPT], L[CPT];
+#pragma unroll
+    for (int k = 0; k < CPT; k++) {
+        const Pair<T> wp = sm.w(slot[k] + S);
+        us_p[k] = wp.x;
+        L[k] = dx + dt * (us_p[k] - us[k]);
+        const T yL = shared_recip<T>(L[k]);
+        cell[k].un += dtdm[k] * (ps[k] - wp.y);
+        cell[k].E += dtdm[k] * (ps[k] * us[k] - wp.y * us_p[k]);
+        cell[k].rho = quot<T>(dm[k], L[k], yL);
+        if (__builtin_expect(bad[k] | unusable(yL), 0)) cell[k].rho = dv<T>(dm[k], L[k]);
+        if constexpr (E2) {
+            us_m[k] = sm.w(slot[k] - S).x;
+            const T L_m = dx + dt * (us[k] - us_m[k]);
+            const T sum = L[k] + L_m;
+            sm.put_lengths(slot[k], L[k], yL, shared_recip<T>(sum));
+        }
+        sm.put_carried(slot[k], cell[k].rho, cell[k].un, cell[k].ut, cell[k].E);
+    }
+    __syncthreads();
+
+    // Stage 4: the advection flux at face t, from the donor cell t or t-S.
+    T f[CPT][4];
+#pragma unroll
+    for (int k = 0; k < CPT; k++) {
+        const T disp = dt * us[k];
+        const int d = disp > 0 ? slot[k] - S : slot[k];
+        T q[4];
+        sm.get_carried(d, q);
+        if constexpr (E2) {
+            T qm[4], qp[4];
+            sm.get_carried(d - S, qm);
+            sm.get_carried(d + S, qp);
+            T Ld, yLd, lo, y_lo, hi, y_hi;
+            sm.get_lengths(d, Ld, yLd, lo, y_lo, hi, y_hi);
+            const T lf = length_factor<T>(donor_length<T>(dx, dt, disp, us_m[k], us_p[k]), Ld, yLd);
+            T r_m, r_p, slope[4];
+            slope_ratios<T>(Ld, lo, y_lo, hi, y_hi, r_m, r_p);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                // FP64 tiles hold the products
+                const T c = sizeof(T) == 8 ? q[i] : carried(q, i), m = sizeof(T) == 8 ? qm[i] : carried(qm, i),
+                        p = sizeof(T) == 8 ? qp[i] : carried(qp, i);
+                slope[i] = slope_minmod_t<T>(r_p * (p - c), r_m * (c - m));
+            }
+            donor_flux_2<T>(disp, lf, q, slope, f[k]);
+        } else {
+            donor_flux_1<T>(disp, q, f[k]);
+        }
+    }
+    if constexpr (TileLds<T, CELLS, S>::kFluxBarrier) __syncthreads();
+#pragma unroll
+    for (int k = 0; k < CPT; k++) sm.put_flux(slot[k], f[k]);
+    __syncthreads();
+
+    // Stage 5: projection of cell t.
+#pragma unroll
+    for (int k = 0; k < CPT; k++) {
+        T fp[4];
+        sm.get_flux(slot[k] + S, fp);
+        project<DXM, T>(dx, inv_dx, L[k], f[k], fp, cell[k].rho, cell[k].un, cell[k].ut, cell[k].E);
+    }
+}
 
 // One X tile of the domain described by `a`, with the cycle's dt. Called by all TILE / CPT
 // threads of a block; each thread computes CPT cells of the tile, at slots t, t + TILE / CPT, ...
@@ -249,15 +655,11 @@ struct SmemX {
 // result depends only on the cells within R of it in its own row, so a tile may span the end
 // of one row and the start of the next; no thread is spent on a tile's share of a row end.
 template <class T, int FLUX, int PROJ, int EOS, int DXM, int TILE = kTile, int CPT = 1>
-__device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, T dt, int j0, int k0, SmemX<T, TILE>& sm)
+__device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, T dt, int j0, int k0, TileLds<T, TILE, 1>& sm)
 {
-    constexpr int GAD = FLUX > 0 ? 1 : 0;
-    constexpr int E2 = PROJ == 2 ? 1 : 0;
-    constexpr int R = 2 + GAD + E2;
-    constexpr int W = TILE - 2 * R;
+    constexpr int R = 2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0);
     constexpr int NT = TILE / CPT;
     static_assert(TILE % CPT == 0, "a tile is a whole number of cells per thread");
-    const T dx = (T) a.dx;
 
     int slot[CPT], jc[CPT], kc[CPT];
     bool in_range[CPT];
@@ -271,7 +673,7 @@ __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, T dt, int j0
         for (int c = 0; c < CPT; c++) {
             const int n = k0 + (int) threadIdx.x + c * NT;
             const int dj = n >= a.x_slots ? 1 : 0;
-            jc[c] = j0 + dj;
+            jc[c] = dj;
             kc[c] = n - (dj ? a.x_slots : 0) - R;
         }
     } else {
@@ -282,146 +684,43 @@ __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, T dt, int j0
             int r = n - dj * a.x_slots;
             if (r < 0) { dj--; r += a.x_slots; }
             else if (r >= a.x_slots) { dj++; r -= a.x_slots; }
-            jc[c] = j0 + dj;
+            jc[c] = dj;
             kc[c] = r - R;
         }
     }
-    // Stage 0: load (or synthesise) the cells, EOS.
+    // Offsets within the arrays count from the tile's first row less its R ghost cells, so that they
+    // are small, unsigned and shared by all arrays, and the bases stay in scalar registers.
+    const int64_t base = (int64_t) a.index_start + (int64_t) j0 * a.row_length - R;
+    const int rows_left = a.ny - j0;
 #pragma unroll
     for (int c = 0; c < CPT; c++) {
-        const int t = threadIdx.x + c * NT;
-        slot[c] = t;
-        in_range[c] = jc[c] < a.ny;       // false for slots past the last row
-        cell[c] = in_range[c] ? load_cell<T, 0, EOS>(a, jc[c], kc[c], a.nx) : benign_cell<T>();
-        sm.rho[t] = cell[c].rho;
-        sm.un[t] = cell[c].un;
-        sm.p()[t] = cell[c].p;
-        sm.c()[t] = cell[c].c;
+        slot[c] = threadIdx.x + c * NT;
+        in_range[c] = jc[c] < rows_left;       // false for slots past the last row
+        cell[c] = in_range[c] ? load_cell<T, 0, EOS>(a, base, jc[c] * a.row_length + R, kc[c], 1, a.nx)
+                              : benign_cell<T>();
     }
-    __syncthreads();
+    tile_sweep<T, FLUX, PROJ, DXM, TILE, 1, CPT>((T) a.dx, (T) a.inv_dx, dt, sm, slot, cell);
 
-    // Stage 1-2: face flux at face k (between cells k-1 and k).
-    T us[CPT], ps[CPT];
-    {
-        T gu[CPT], gp[CPT];
-#pragma unroll
-        for (int c = 0; c < CPT; c++) {
-            const int t = slot[c], tm = t > 0 ? t - 1 : 0;
-            godunov<T>(cell[c].rho, sm.rho[tm], cell[c].c, sm.c()[tm], cell[c].un, sm.un[tm], cell[c].p, sm.p()[tm],
-                       gu[c], gp[c]);
-        }
-        if constexpr (GAD) {
-#pragma unroll
-            for (int c = 0; c < CPT; c++) {
-                sm.gu()[slot[c]] = gu[c];
-                sm.gp()[slot[c]] = gp[c];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int c = 0; c < CPT; c++) {
-                const int t = slot[c], tm = t > 0 ? t - 1 : 0, tp = t < TILE - 1 ? t + 1 : TILE - 1;
-                Cell<T> m;
-                m.rho = sm.rho[tm]; m.un = sm.un[tm]; m.p = sm.p()[tm]; m.c = sm.c()[tm];
-                face_flux_gad<T, FLUX - 1>(dt, dx, m, cell[c], sm.gu()[tm], sm.gp()[tm], gu[c], gp[c], sm.gu()[tp],
-                                           sm.gp()[tp], us[c], ps[c]);
-            }
-        } else {
-#pragma unroll
-            for (int c = 0; c < CPT; c++) {
-                us[c] = gu[c];
-                ps[c] = gp[c];
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < CPT; c++) {
-        sm.us[slot[c]] = us[c];
-        sm.ps[slot[c]] = ps[c];
-    }
-    __syncthreads();
-
-    // Stage 3: Lagrangian update of cell k from faces k and k+1.
-    T rho[CPT], un[CPT], ut[CPT], E[CPT], us_p[CPT];
-#pragma unroll
-    for (int c = 0; c < CPT; c++) {
-        const int t = slot[c], tp = t < TILE - 1 ? t + 1 : TILE - 1;
-        rho[c] = cell[c].rho; un[c] = cell[c].un; ut[c] = cell[c].ut; E[c] = cell[c].E;
-        us_p[c] = sm.us[tp];
-        cell_update<T>(dx, dt, us[c], us_p[c], ps[c], sm.ps[tp], rho[c], un[c], E[c]);
-    }
+    CflSpeeds speeds;
 #pragma unroll
     for (int c = 0; c < CPT; c++) {
         const int t = slot[c];
-        sm.rho[t] = rho[c];
-        sm.un[t] = un[c];
-        sm.ut[t] = ut[c];
-        sm.E[t] = E[c];
-    }
-    __syncthreads();
-
-    // Stage 4: advection flux at face k.
-    T f[CPT][4];
-#pragma unroll
-    for (int c = 0; c < CPT; c++) {
-        const int t = slot[c], tm = t > 0 ? t - 1 : 0, tp = t < TILE - 1 ? t + 1 : TILE - 1;
-        const T disp = dt * us[c];
-        if constexpr (E2) {
-            T Dx;
-            int td;
-            if (disp > 0) {
-                Dx = -(dx - dt * sm.us[tm]);
-                td = tm;
-            } else {
-                Dx = dx + dt * sm.us[tp];
-                td = t;
-            }
-            const int tdm = td > 0 ? td - 1 : 0;
-            const int tdp = td < TILE - 1 ? td + 1 : TILE - 1;
-            const int tdpp = td < TILE - 2 ? td + 2 : TILE - 1;
-            advection_flux_2<T>(dx, dt, disp, Dx, sm.us[tdm], sm.us[td], sm.us[tdp], sm.us[tdpp], sm.rho[tdm],
-                                sm.rho[td], sm.rho[tdp], sm.un[tdm], sm.un[td], sm.un[tdp], sm.ut[tdm], sm.ut[td],
-                                sm.ut[tdp], sm.E[tdm], sm.E[td], sm.E[tdp], f[c][0], f[c][1], f[c][2], f[c][3]);
-        } else {
-            const int td = disp > 0 ? tm : t;
-            advection_flux_1<T>(disp, sm.rho[td], sm.un[td], sm.ut[td], sm.E[td], f[c][0], f[c][1], f[c][2], f[c][3]);
+        if (t >= R && t < TILE - R && in_range[c] && (unsigned) kc[c] < (unsigned) a.nx) {
+            const unsigned o = (unsigned) (jc[c] * a.row_length + R + kc[c]) * (unsigned) sizeof(T);
+            store_at(a.out_rho + base, o, cell[c].rho);
+            store_at(a.out_u + base, o, cell[c].un);
+            store_at(a.out_v + base, o, cell[c].ut);
+            store_at(a.out_E + base, o, cell[c].E);
+            if (a.reduce) speeds.add((double) cell[c].un, (double) cell[c].ut, (double) cell[c].c);
         }
     }
-#pragma unroll
-    for (int c = 0; c < CPT; c++) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) sm.f()[q][slot[c]] = f[c][q];
-    }
-    __syncthreads();
-
-    // Stage 5: projection of cell k, output.
-    double local = DBL_MAX;
-    bool any = false;
-#pragma unroll
-    for (int c = 0; c < CPT; c++) {
-        const int t = slot[c], tp = t < TILE - 1 ? t + 1 : TILE - 1;
-        if (t >= R && t < R + W && in_range[c] && kc[c] >= 0 && kc[c] < a.nx) {
-            projection<DXM, T>(dx, (T) a.inv_dx, dt, us[c], us_p[c], f[c][0], sm.f()[0][tp], f[c][1], sm.f()[1][tp],
-                               f[c][2], sm.f()[2][tp], f[c][3], sm.f()[3][tp], rho[c], un[c], ut[c], E[c]);
-            const int idx = a.index_start + jc[c] * a.row_length + kc[c];
-            a.out_rho[idx] = rho[c];
-            a.out_u[idx] = un[c];
-            a.out_v[idx] = ut[c];
-            a.out_E[idx] = E[c];
-            if (a.reduce) {
-                const double v = cfl_cell<double>(a.cfl_dx, a.cfl_dy, (double) un[c], (double) ut[c],
-                                                  (double) cell[c].c, 1.0);
-                local = any ? kmin(local, v) : v;
-                any = true;
-            }
-        }
-    }
-    if (a.reduce) reduce_cfl(a.st, local);
+    if (a.reduce) reduce_cfl(a.st, speeds.bound(a.cfl_dx, a.cfl_dy));
 }
 
 // Tile of the single-domain X sweep per element type: FP64 tiles of 256 cells at one cell per
-// thread; FP32 tiles of 512 cells at two cells per thread (256 threads, the same 20 KiB of LDS),
-// which measured faster for the FP32-mixed sweep and slower for the FP64 one, whose 3 VALU
-// instructions of 4 are FP64 arithmetic with little latency left to hide.
+// thread; FP32 tiles of 512 cells at two cells per thread (256 threads), which measured faster for
+// the FP32-mixed sweep (408 us at 8192^2, one cell per thread 468) and slower for the FP64 one. The
+// LDS leaves room for 7 waves per SIMD, so the kernels are held to the 72 VGPRs that 7 waves have.
 template <class T>
 struct XTile {
     static constexpr int cells = 256, cpt = 1;
@@ -432,13 +731,15 @@ struct XTile<float> {
 };
 
 template <class T, int FLUX, int PROJ, int EOS, int DXM>
-__global__ void __launch_bounds__(XTile<T>::cells / XTile<T>::cpt) k_sweep_x(SweepArgs<T> a)
+__global__ void __launch_bounds__(XTile<T>::cells / XTile<T>::cpt) __attribute__((amdgpu_waves_per_eu(7)))
+        k_sweep_x(SweepArgs<T> a)
 {
     constexpr int TILE = XTile<T>::cells;
     constexpr int W = TILE - 2 * (2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0));
-    if (!a.st->active) return;
-    const T dt = (T) (a.st->current_dt * a.dt_factor);
-    __shared__ SmemX<T, TILE> sm;
+    double cycle_dt;
+    if (!begin_sweep(a, blockIdx.x == 0, cycle_dt)) return;
+    const T dt = (T) (cycle_dt * a.dt_factor);
+    __shared__ TileLds<T, TILE, 1> sm;
     const int s0 = xcd_block(blockIdx.x, gridDim.x) * W;   // first slot of the tile
     const int j0 = s0 / a.x_slots;
     sweep_x_tile<T, FLUX, PROJ, EOS, DXM, TILE, XTile<T>::cpt>(a, dt, j0, s0 - j0 * a.x_slots, sm);
@@ -456,159 +757,282 @@ __device__ __forceinline__ void push(T (&w)[N], T v)
     w[N - 1] = v;
 }
 
-// The march state of one column of a Y run: sliding windows of the stage results along y.
-// AHEAD: each row's state is loaded one row before it is used (the FP64 sweeps); with
-// STALE = false, when the stencil width covers the read extent so that no ghost layer is stale,
-// the march then loads nothing else.
-// Whether the Y march shares divisors between Godunov's two quotients and the projection's three
-// (with_divisor), as the X tiles do (3 of their 17 FP64 reciprocals per cell removed, 3% of
-// their time). While the march's waves ran independently it gained nothing (4% fewer VALU busy
-// cycles, the same time: the waves waited on their dependency chains); with the block barrier
-// every 4 rows it is 2.3% faster at 8192^2 and still fits 168 VGPRs with no spill.
-constexpr bool kYSharedDivisor = true;
+// What a thread of the march keeps in LDS until a later row, off the arithmetic's dependency chains
+// (a slot is read before the row that wraps round to it writes it): the parts of a cell that the
+// faces do not read and, for the CFL bound, its sound speed.
+template <class T>
+struct MarchLds {
+    Pair<T> ut_E[2][kYBlock];
+    T dtdm[2][kYBlock], c[4][kYBlock];
+};
 
-template <class T, int FLUX, int PROJ, int EOS, int DXM, bool STALE, bool AHEAD>
+// What else waits for the next row or two: the reciprocal of an updated cell's length, its slopes and
+// its state once the next cell is there, and a face's advection fluxes. In FP64 in LDS too (32 VGPRs
+// fewer: with register windows the unrolled march does not fit the 168 of 3 waves per SIMD; 48 KB
+// with the rest, 3 blocks a CU); in FP32 in registers, where the march has them (100 VGPRs) and is
+// 4% faster so (494 -> 472 us at 8192^2).
+template <class T>
+struct MarchWindows;
+
+template <>
+struct MarchWindows<double> {
+    struct Lds {
+        double yL[2][kYBlock];
+        Pair<double> cell[2][kYBlock], slope[2][kYBlock], flux[2][kYBlock];
+    };
+    Lds* lds;
+    static __device__ __forceinline__ void swap(Pair<double> (&at)[2][kYBlock], const double (&put)[4], double (&got)[4])
+    {
+        get(at, got);
+        at[0][threadIdx.x] = {put[0], put[1]};
+        at[1][threadIdx.x] = {put[2], put[3]};
+    }
+    static __device__ __forceinline__ void get(const Pair<double> (&at)[2][kYBlock], double (&v)[4])
+    {
+        const Pair<double> l = at[0][threadIdx.x], h = at[1][threadIdx.x];
+        v[0] = l.x; v[1] = l.y; v[2] = h.x; v[3] = h.y;
+    }
+    __device__ __forceinline__ void init(Lds* at) { lds = at; }
+    __device__ __forceinline__ void cell(const double (&put)[4], double (&got)[4]) { swap(lds->cell, put, got); }
+    __device__ __forceinline__ void flux(const double (&put)[4], double (&got)[4]) { swap(lds->flux, put, got); }
+    __device__ __forceinline__ void slope_below(double (&v)[4]) const { get(lds->slope, v); }
+    __device__ __forceinline__ double yL_below(int U) const { return lds->yL[U & 1][threadIdx.x]; }
+    __device__ __forceinline__ double yL_own(int U) const { return lds->yL[(U - 1) & 1][threadIdx.x]; }
+    __device__ __forceinline__ void put(int U, const double (&slope)[4], double yL)
+    {
+        double old[4];
+        swap(lds->slope, slope, old);
+        lds->yL[U & 1][threadIdx.x] = yL;
+    }
+};
+
+template <>
+struct MarchWindows<float> {
+    struct Lds {};
+    float cell_[4], flux_[4], slope_[4], yL_[2];
+    static __device__ __forceinline__ void swap(float (&at)[4], const float (&put)[4], float (&got)[4])
+    {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            got[k] = at[k];
+            at[k] = put[k];
+        }
+    }
+    __device__ __forceinline__ void init(Lds*)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; k++) cell_[k] = flux_[k] = slope_[k] = 1.0f;
+        yL_[0] = yL_[1] = 1.0f;
+    }
+    __device__ __forceinline__ void cell(const float (&put)[4], float (&got)[4]) { swap(cell_, put, got); }
+    __device__ __forceinline__ void flux(const float (&put)[4], float (&got)[4]) { swap(flux_, put, got); }
+    __device__ __forceinline__ void slope_below(float (&v)[4]) const
+    {
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = slope_[k];
+    }
+    __device__ __forceinline__ float yL_below(int) const { return yL_[0]; }
+    __device__ __forceinline__ float yL_own(int) const { return yL_[1]; }
+    __device__ __forceinline__ void put(int, const float (&slope)[4], float yL)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; k++) slope_[k] = slope[k];
+        yL_[0] = yL_[1];
+        yL_[1] = yL;
+    }
+};
+
+// The march state of one column of a Y run: sliding windows of the stage results along y. Each row's
+// state is loaded one row before it is used (with STALE = false, when the stencil width covers the
+// read extent so that no ghost layer is stale, the march then loads nothing else).
+//
+// Per row it makes the cell n, Godunov's face n, the final face F, the update of the cell U below it,
+// the slopes of the cell below that, the advection flux at a face A and the projection of the cell P
+// below A. What several rows or stages need is made once: the differences A and B of a face, theta,
+// the Lagrangian lengths, their sums and the reciprocals of both, the differences and slopes of the
+// carried quantities (per cell, whichever face takes them).
+template <class T, int FLUX, int PROJ, int EOS, int DXM, bool STALE>
 struct YColumn {
     static constexpr int GAD = FLUX > 0 ? 1 : 0;
     static constexpr int E2 = PROJ == 2 ? 1 : 0;
     static constexpr int R = 2 + GAD + E2;
 
-    // Windows, oldest first (see the index map in each stage of step()).
-    Cell<T> pre[3];                       // cells n-2, n-1, n (pre-update state + EOS)
-    T g_u[3], g_p[3];                     // Godunov at faces n-2, n-1, n
-    T f_u[5], f_p[2];                     // final face flux: u* at faces F-4..F, p* at F-1..F (F = n - GAD)
-    T q_rho[4], q_un[4], q_ut[4], q_E[4]; // post-update cells U-3..U (U = F - 1)
-    T h0[2], h1[2], h2[2], h3[2];         // advection fluxes at faces A-1, A (A = U - E2)
-    T nx_rho, nx_u, nx_v, nx_E;           // the next row's state (AHEAD)
-    int x;
+    // Windows, oldest first.
+    T dm[3], un[3];                       // cells n-2, n-1, n
+    T rc, p;                              // cell n
+    T theta[2], g_u[2], g_p[2];           // faces n-1, n
+    Pair<T> A[2], B[3];                   // faces n-1, n; n-2, n-1, n
+    T us[4], ps[2];                       // final faces F-3..F; F-1, F (F = n - GAD)
+    T L[3], S[2], yS[2];                  // cells U-2, U-1, U; U-1, U (U = F - 1)
+    T q[2][4];                            // updated cells U-1, U: rho, un, ut, E
+    T dq[2][4];                           // carried quantities: U-1 over U-2, U over U-1
+    T nx_rho, nx_u, nx_v, nx_E;           // the next row's state
+    unsigned column;                      // byte offset of the column within a row
     bool lane_ok;                         // false for lanes past the domain
-    double local;                         // CFL bound of the column's outputs
+    CflSpeeds speeds;                     // of the column's outputs
+    MarchWindows<T> windows;
 
-    __device__ __forceinline__ void init(int x_, bool ok)
+    __device__ __forceinline__ void init(int x, bool ok, typename MarchWindows<T>::Lds* lds)
     {
-        x = x_;
+        windows.init(lds);
+        column = (unsigned) x * (unsigned) sizeof(T);
         lane_ok = ok;
 #pragma unroll
-        for (int i = 0; i < 3; i++) { pre[i] = benign_cell<T>(); g_u[i] = T(0); g_p[i] = T(0); }
+        for (int i = 0; i < 3; i++) {
+            dm[i] = L[i] = T(1);
+            un[i] = T(0);
+            B[i] = {T(0), T(0)};
+        }
+        rc = p = T(1);
 #pragma unroll
-        for (int i = 0; i < 5; i++) f_u[i] = T(0);
+        for (int i = 0; i < 2; i++) {
+            theta[i] = g_u[i] = g_p[i] = ps[i] = T(0);
+            A[i] = {T(0), T(0)};
+            S[i] = yS[i] = T(1);
+            q[i][0] = q[i][3] = T(1);
+            q[i][1] = q[i][2] = T(0);
 #pragma unroll
-        for (int i = 0; i < 4; i++) { q_rho[i] = T(1); q_un[i] = T(0); q_ut[i] = T(0); q_E[i] = T(1); }
-        f_p[0] = f_p[1] = T(0);
-        h0[0] = h0[1] = h1[0] = h1[1] = h2[0] = h2[1] = h3[0] = h3[1] = T(0);
+            for (int k = 0; k < 4; k++) dq[i][k] = T(0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) us[i] = T(0);
         nx_rho = T(1); nx_u = T(0); nx_v = T(0); nx_E = T(1);
-        local = DBL_MAX;
     }
 
     __device__ __forceinline__ void fetch(const SweepArgs<T>& a, int k)
     {
         if (lane_ok) {
-            const int idx = cell_source<T, 1, STALE>(a, x, k, a.ny).idx;
-            nx_rho = a.in_rho[idx];
-            nx_u = a.in_u[idx];
-            nx_v = a.in_v[idx];
-            nx_E = a.in_E[idx];
+            const int64_t row = row_start(a, row_source<T, STALE>(a, k).row);
+            nx_rho = load_at(a.in_rho + row, column);
+            nx_u = load_at(a.in_u + row, column);
+            nx_v = load_at(a.in_v + row, column);
+            nx_E = load_at(a.in_E + row, column);
         }
     }
 
-    // Row n of a run that outputs rows [y0, y1). `ring` (LDS, 8 rows x the block's columns) keeps
-    // each row's sound speed until the CFL bound of its output, R rows later: off the arithmetic's
-    // dependency chains, and 8 VGPRs fewer than a register window.
+    // Row n of a run that outputs rows [y0, y1).
     __device__ __forceinline__ void step(const SweepArgs<T>& a, T dt, T dx, T inv_dx, int n, int y0, int y1,
-                                         T (*ring)[kYBlock])
+                                         MarchLds<T>& keep)
     {
-        Cell<T> cn;
-        if constexpr (AHEAD) {
-            // the next load is issued after this row's cell is made: a stale layer's p, c loads
-            // are waited for there
-            cn = lane_ok ? make_cell<T, 1, EOS, STALE>(a, cell_source<T, 1, STALE>(a, x, n, a.ny), nx_rho, nx_u, nx_v,
-                                                       nx_E)
-                         : benign_cell<T>();
-            if (n + 1 < y1 + R) fetch(a, n + 1);
-        } else {
-            cn = lane_ok ? load_cell<T, 1, EOS>(a, x, n, a.ny) : benign_cell<T>();
-        }
-        pre[0] = pre[1];
-        pre[1] = pre[2];
-        pre[2] = cn;
-        ring[n & 7][threadIdx.x] = cn.c;
+        const int t = threadIdx.x;
+        // Keeps the column's offset out of the loop-invariant addresses that the compiler would make
+        // of it and the arrays' bases (16 VGPRs, and a 64-bit sum per access): base and row stay scalar.
+        asm("" : "+v"(column));
+        // the next load is issued after this row's cell is made: a stale layer's p, c loads are
+        // waited for there
+        const Cell<T> cn = lane_ok ? make_row_cell<T, EOS, STALE>(a, row_source<T, STALE>(a, n), column, nx_rho, nx_u,
+                                                                  nx_v, nx_E)
+                                   : benign_cell<T>();
+        if (n + 1 < y1 + R) fetch(a, n + 1);
+        const T rc_m = rc, p_m = p;
+        push(dm, cn.rho * dx);
+        push(un, cn.un);
+        rc = cn.rho * cn.c;
+        p = cn.p;
+        T dtdm = mass_quotient<DXM>(dt, dm[2], cn.y, inv_dx);
+        if (__builtin_expect(unusable(dtdm), 0)) dtdm = dv<T>(dt, dm[2]);
+        // what is left of cell U (the one before n, or two before it) and the sound speed of cell n-4
+        constexpr int W = GAD ? 0 : 1;    // window index of cell U among n-2, n-1, n
+        const Pair<T> rest = keep.ut_E[(n + W) & 1][t];
+        const T dtdm_U = keep.dtdm[(n + W) & 1][t];
+        const T c_P = keep.c[(n - R) & 3][t];
+        keep.ut_E[n & 1][t] = {cn.ut, cn.E};
+        keep.dtdm[n & 1][t] = dtdm;
+        keep.c[n & 3][t] = cn.c;
 
         // Godunov at face n (cells n-1 | n).
         T gu, gp;
-        godunov<T, kYSharedDivisor>(pre[2].rho, pre[1].rho, pre[2].c, pre[1].c, pre[2].un, pre[1].un, pre[2].p,
-                                    pre[1].p, gu, gp);
-        push(g_u, gu);
-        push(g_p, gp);
-
+        face_godunov<T>(rc_m, rc, un[1], un[2], p_m, p, gu, gp);
         // Final flux at face F: GAD at F = n-1 (cells n-2 | n-1, Godunov n-2, n-1, n), else F = n.
-        T us, ps;
         if constexpr (GAD) {
-            face_flux_gad<T, FLUX - 1>(dt, dx, pre[0], pre[1], g_u[0], g_p[0], g_u[1], g_p[1], g_u[2], g_p[2], us,
-                                       ps);
+            push(g_u, gu);
+            push(g_p, gp);
+            push(A, Pair<T>{gu - un[1], gp - p_m});
+            push(B, Pair<T>{un[2] - gu, p - gp});
+            push(us, gad_star<FLUX - 1, T>(theta[1], g_u[0], A[0].x, A[1].x, B[1].x, B[0].x));
+            push(ps, gad_star<FLUX - 1, T>(theta[1], g_p[0], A[0].y, A[1].y, B[1].y, B[0].y));
+            push(theta, gad_theta<T>(dt, dm[1], dm[2], rc_m, rc));
         } else {
-            us = gu;
-            ps = gp;
+            push(us, gu);
+            push(ps, gp);
         }
-        push(f_u, us);
-        push(f_p, ps);
 
-        // Lagrangian update of cell U = F-1 from faces U (f_*[3], f_p[0]) and F (f_*[4], f_p[1]).
-        const Cell<T>& pu = GAD ? pre[0] : pre[1];
-        T rho = pu.rho, un = pu.un, ut = pu.ut, E = pu.E;
-        cell_update<T>(dx, dt, f_u[3], f_u[4], f_p[0], f_p[1], rho, un, E);
-        push(q_rho, rho);
-        push(q_un, un);
-        push(q_ut, ut);
-        push(q_E, E);
+        // Lagrangian update of cell U = F-1 from the faces U and F.
+        const int U = n - 2 + W;
+        const T len = dx + dt * (us[3] - us[2]);
+        push(L, len);
+        const T yL = shared_recip<T>(len);
+        T rho = quot<T>(dm[W], len, yL);
+        // a mass out of quot()'s range came with a density out of shared_recip's
+        if (__builtin_expect(unusable(rho) | too_small(dm[W]), 0)) rho = dv<T>(dm[W], len);
+        T u = un[W], E = rest.y;
+        u += dtdm_U * (ps[0] - ps[1]);
+        E += dtdm_U * (ps[0] * us[2] - ps[1] * us[3]);
+        T older[4];                       // cell U-2
+        windows.cell(q[1], older);
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[0][k] = q[1][k];
+        q[1][0] = rho; q[1][1] = u; q[1][2] = rest.x; q[1][3] = E;
 
         // Advection flux at face A.
-        T fa0, fa1, fa2, fa3;
+        const T disp = dt * us[E2 ? 1 : 2];
+        T f[4];
         if constexpr (E2) {
-            // A = U-1 = F-2: u*[A] = f_u[2]; cells q[k] = U-3+k.
-            const T disp = dt * f_u[2];
-            if (disp > 0) {
-                const T Dx = -(dx - dt * f_u[1]);
-                // donor d = A-1 = q[1]; u* at d-1..d+2 = f_u[0..3]
-                advection_flux_2<T>(dx, dt, disp, Dx, f_u[0], f_u[1], f_u[2], f_u[3], q_rho[0], q_rho[1], q_rho[2],
-                                    q_un[0], q_un[1], q_un[2], q_ut[0], q_ut[1], q_ut[2], q_E[0], q_E[1], q_E[2], fa0,
-                                    fa1, fa2, fa3);
-            } else {
-                const T Dx = dx + dt * f_u[3];
-                // donor d = A = q[2]; u* at d-1..d+2 = f_u[1..4]
-                advection_flux_2<T>(dx, dt, disp, Dx, f_u[1], f_u[2], f_u[3], f_u[4], q_rho[1], q_rho[2], q_rho[3],
-                                    q_un[1], q_un[2], q_un[3], q_ut[1], q_ut[2], q_ut[3], q_E[1], q_E[2], q_E[3], fa0,
-                                    fa1, fa2, fa3);
+            push(S, L[2] + L[1]);
+            push(yS, shared_recip<T>(S[1]));
+            // the slopes of cell U-1
+            T r_m, r_p, slope[4];
+            slope_ratios<T>(L[1], S[0], yS[0], S[1], yS[1], r_m, r_p);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                dq[0][k] = dq[1][k];
+                dq[1][k] = carried(q[1], k) - carried(q[0], k);
+                slope[k] = slope_minmod_t<T>(r_p * dq[1][k], r_m * dq[0][k]);
             }
+            // A = U-1: the cells A-1 = U-2 and A = U-1
+            const T Dx = donor_length<T>(dx, dt, disp, us[0], us[2]);
+            T from[4];
+            if (disp > 0) {
+                windows.slope_below(from);
+                flux_from(disp, length_factor<T>(Dx, L[0], windows.yL_below(U)), older, from, f);
+            } else {
+                flux_from(disp, length_factor<T>(Dx, L[1], windows.yL_own(U)), q[0], slope, f);
+            }
+            windows.put(U, slope, yL);
         } else {
-            // A = U = F-1: u*[A] = f_u[3]; donor A-1 = q[2] or A = q[3].
-            const T disp = dt * f_u[3];
-            if (disp > 0)
-                advection_flux_1<T>(disp, q_rho[2], q_un[2], q_ut[2], q_E[2], fa0, fa1, fa2, fa3);
-            else
-                advection_flux_1<T>(disp, q_rho[3], q_un[3], q_ut[3], q_E[3], fa0, fa1, fa2, fa3);
+            // A = U: the cells A-1 = U-1 and A = U
+            const T none[4] = {T(0), T(0), T(0), T(0)};
+            if (disp > 0) flux_from(disp, T(0), q[0], none, f);
+            else flux_from(disp, T(0), q[1], none, f);
         }
-        push(h0, fa0);
-        push(h1, fa1);
-        push(h2, fa2);
-        push(h3, fa3);
+        T below[4];                       // the fluxes of face P
+        windows.flux(f, below);
 
-        // Projection of cell P = A-1 = n-R from faces P (h*[0]) and A (h*[1]).
+        // Projection of cell P = A-1 = n-R from the faces P and A.
         const int P = n - R;
         if (P >= y0 && P < y1 && lane_ok) {
-            constexpr int QP = E2 ? 1 : 2;    // q index of cell P
-            constexpr int FP = E2 ? 1 : 2;    // f_u index of face P
-            T r = q_rho[QP], u = q_un[QP], v = q_ut[QP], e = q_E[QP];
-            projection<DXM, T, kYSharedDivisor>(dx, inv_dx, dt, f_u[FP], f_u[FP + 1], h0[0], h0[1], h1[0], h1[1],
-                                                h2[0], h2[1], h3[0], h3[1], r, u, v, e);
-            const int idx = a.index_start + P * a.row_length + x;
-            a.out_rho[idx] = r;
-            a.out_u[idx] = v;   // ut is the x velocity in a Y sweep
-            a.out_v[idx] = u;
-            a.out_E[idx] = e;
-            if (a.reduce)
-                local = kmin(local, cfl_cell<double>(a.cfl_dx, a.cfl_dy, (double) v, (double) u,
-                                                     (double) ring[P & 7][threadIdx.x], 1.0));
+            const T(&c)[4] = E2 ? older : q[0];
+            T r = c[0], un_P = c[1], ut_P = c[2], e = c[3];
+            project<DXM, T>(dx, inv_dx, L[E2 ? 0 : 1], below, f, r, un_P, ut_P, e);
+            const int64_t row = row_start(a, P);
+            store_at(a.out_rho + row, column, r);
+            store_at(a.out_u + row, column, ut_P);   // ut is the x velocity in a Y sweep
+            store_at(a.out_v + row, column, un_P);
+            store_at(a.out_E + row, column, e);
+            if (a.reduce) speeds.add((double) ut_P, (double) un_P, (double) c_P);
         }
+    }
+
+    // The flux from the donor cell `c`.
+    static __device__ __forceinline__ void flux_from(T disp, T lf, const T (&c)[4], const T (&slope)[4], T (&f)[4])
+    {
+        T d[4] = {c[0], c[1], c[2], c[3]};
+        if constexpr (sizeof(T) == 8) {
+#pragma unroll
+            for (int k = 1; k < 4; k++) d[k] = c[0] * c[k];
+        }
+        if constexpr (E2) donor_flux_2<T>(disp, lf, d, slope, f);
+        else donor_flux_1<T>(disp, d, f);
     }
 };
 
@@ -627,10 +1051,10 @@ struct YColumn {
 // barriers only. SYNC needs the same number of rows for the whole block: the loop-free batched
 // kernel takes it for a block whose 4 waves hold live runs of equal length (most blocks, as
 // the runs are listed longest first) and the independent march otherwise.
-template <class T, int FLUX, int PROJ, int EOS, int DXM, bool STALE, bool AHEAD, bool SYNC = false>
+template <class T, int FLUX, int PROJ, int EOS, int DXM, bool STALE, bool SYNC = false>
 __device__ __forceinline__ void sweep_y_run(const SweepArgs<T>& a, T dt, int x, int y0, int y1, bool idle = false)
 {
-    using Col = YColumn<T, FLUX, PROJ, EOS, DXM, STALE, AHEAD>;
+    using Col = YColumn<T, FLUX, PROJ, EOS, DXM, STALE>;
     constexpr int R = Col::R;
     // a row counter from 0 keeps the loop and the row index in scalar registers (counting
     // from y0 - R, the compiler carried the row index in a vector register)
@@ -647,20 +1071,21 @@ __device__ __forceinline__ void sweep_y_run(const SweepArgs<T>& a, T dt, int x, 
         }
     }
     Col col;
-    __shared__ T ring[8][kYBlock];
-    col.init(x, x < a.nx);
-    if constexpr (AHEAD) col.fetch(a, y0 - R);
+    __shared__ MarchLds<T> keep;
+    __shared__ typename MarchWindows<T>::Lds windows;
+    col.init(x, x < a.nx, &windows);
+    col.fetch(a, y0 - R);
     if constexpr (SYNC) {
         for (int g = 0; g < groups; ++g) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) col.step(a, dt, (T) a.dx, (T) a.inv_dx, y0 - R + 4 * g + k, y0, y1, ring);
+#pragma unroll(sizeof(T) == 8 ? kYUnrollFp64 : kYUnrollFp32)
+            for (int k = 0; k < 4; ++k) col.step(a, dt, (T) a.dx, (T) a.inv_dx, y0 - R + 4 * g + k, y0, y1, keep);
             __syncthreads();
         }
     } else {
-#pragma unroll kYUnroll
-        for (int i = 0; i < rows; ++i) col.step(a, dt, (T) a.dx, (T) a.inv_dx, y0 - R + i, y0, y1, ring);
+#pragma unroll(sizeof(T) == 8 ? kYUnrollFp64 : kYUnrollFp32)
+        for (int i = 0; i < rows; ++i) col.step(a, dt, (T) a.dx, (T) a.inv_dx, y0 - R + i, y0, y1, keep);
     }
-    if (a.reduce) reduce_cfl(a.st, col.local);
+    if (a.reduce) reduce_cfl(a.st, col.speeds.bound(a.cfl_dx, a.cfl_dy));
 }
 
 template <class T, int FLUX, int PROJ, int EOS, int DXM, bool STALE>
@@ -673,10 +1098,87 @@ __global__ void __launch_bounds__(kYBlock) ARMON_Y_OCCUPANCY k_sweep_y(SweepArgs
     const int x = (bid - seg * ncolblk) * kYBlock + threadIdx.x;
     const bool idle = x - (int) (threadIdx.x & 63) >= a.nx;   // a wave past the last column
     const int y0 = seg * a.seg_len;
-    constexpr bool ahead = ARMON_Y_PREFETCH;
     constexpr bool sync = !STALE;   // see sweep_y_run
     if (idle && !sync) return;   // no barriers follow
-    sweep_y_run<T, FLUX, PROJ, EOS, DXM, STALE, ahead, sync>(a, dt, x, y0, min(y0 + a.seg_len, a.ny), idle);
+    sweep_y_run<T, FLUX, PROJ, EOS, DXM, STALE, sync>(a, dt, x, y0, min(y0 + a.seg_len, a.ny), idle);
+}
+
+// ---------------------------------------------------------------------------------------
+// Y sweep of domains too small to fill the chip with marches: LDS tiles
+// ---------------------------------------------------------------------------------------
+
+// One Y tile: the columns [x0, x0 + COLS) and the output rows [y0, y0 + ROWS - 2R) of the domain
+// described by `a`, through the stages of tile_sweep with neighbours a tile row apart. Called by NT
+// threads, each with COLS ROWS / NT cells of one column.
+template <class T, int FLUX, int PROJ, int EOS, int DXM, int COLS, int ROWS, int NT>
+__device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, T dt, int x0, int y0,
+                                             TileLds<T, COLS * ROWS, COLS>& sm)
+{
+    constexpr int R = 2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0);
+    constexpr int CPT = COLS * ROWS / NT;
+    static_assert(NT % COLS == 0 && COLS * ROWS % NT == 0, "a thread's cells are in one column");
+    const int col = threadIdx.x % COLS, x = x0 + col;
+    // offsets count from the tile's first row (a mirror's real cell never lies above it)
+    const int64_t base = (int64_t) a.index_start + (int64_t) (y0 - R) * a.row_length + x0;
+    int slot[CPT], row[CPT];
+    bool in_range[CPT];
+    Cell<T> cell[CPT];
+#pragma unroll
+    for (int c = 0; c < CPT; c++) {
+        slot[c] = threadIdx.x + c * NT;
+        row[c] = threadIdx.x / COLS + c * (NT / COLS);
+        const int k = y0 - R + row[c];
+        in_range[c] = x < a.nx && k < a.ny + R;
+        cell[c] = in_range[c] ? load_cell<T, 1, EOS>(a, base, col + (R - y0) * a.row_length, k, a.row_length, a.ny)
+                              : benign_cell<T>();
+    }
+    tile_sweep<T, FLUX, PROJ, DXM, COLS * ROWS, COLS, CPT>((T) a.dx, (T) a.inv_dx, dt, sm, slot, cell);
+    CflSpeeds speeds;
+#pragma unroll
+    for (int c = 0; c < CPT; c++) {
+        if (row[c] >= R && row[c] < ROWS - R && x < a.nx && y0 - R + row[c] < a.ny) {
+            const unsigned o = (unsigned) (col + row[c] * a.row_length) * (unsigned) sizeof(T);
+            store_at(a.out_rho + base, o, cell[c].rho);
+            store_at(a.out_u + base, o, cell[c].ut);   // ut is the x velocity in a Y sweep
+            store_at(a.out_v + base, o, cell[c].un);
+            store_at(a.out_E + base, o, cell[c].E);
+            if (a.reduce) speeds.add((double) cell[c].ut, (double) cell[c].un, (double) cell[c].c);
+        }
+    }
+    if (a.reduce) reduce_cfl(a.st, speeds.bound(a.cfl_dx, a.cfl_dy));
+}
+
+// Tiles of 16 columns x 32 rows: 128 bytes of a row in FP64, and 24 of the 32 rows are outputs. FP64:
+// one cell a thread, 49 KB of LDS, 3 blocks a CU; FP32: two cells a thread. Of the shapes measured
+// (4 to 32 columns, 24 to 96 rows, 1 to 4 cells a thread; Y sweep at 512^2 / 1024^2, us): FP64 16x32
+// 12.1 / 27.8, 8x64 12.9 / 27.1, 16x64 19 / 37, 32x32 18 / 39; FP32 16x32 10.5 / 16.9, 16x64 at two cells
+// 10.4 / 17.2, at one cell 11.5 / 20.4.
+//
+// A march has a wave per 64 columns and run, which works through its rows one after the other, some
+// 1.5 us each; a tile has a thread per cell or two. The march is the cheaper per cell (its runs are
+// longer than 24 rows, and nothing passes through LDS) once its waves fill the chip: us per Y sweep,
+// march / tile, FP64 512^2 24.7 / 12.1, 1024^2 35.9 / 27.8, 2048^2 86 / 92; FP32 512^2 16.9 / 10.5,
+// 1024^2 23 / 16.9, 2048^2 40 / 41. `max_cells`: the domains that take tiles.
+template <class T>
+struct YTile {
+    static constexpr int cols = 16, rows = 32, threads = sizeof(T) == 8 ? 512 : 256;
+    static constexpr int64_t max_cells = sizeof(T) == 8 ? 5 << 19 : 7 << 19;   // 2.6 M, 3.7 M
+    static_assert(kFoldedCells <= max_cells, "the march makes no time step");
+};
+
+template <class T, int FLUX, int PROJ, int EOS, int DXM>
+__global__ void __launch_bounds__(YTile<T>::threads) k_sweep_y_tile(SweepArgs<T> a, int ncolblk)
+{
+    double cycle_dt;
+    if (!begin_sweep(a, blockIdx.x == 0, cycle_dt)) return;
+    using Y = YTile<T>;
+    constexpr int W = Y::rows - 2 * (2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0));
+    const T dt = (T) (cycle_dt * a.dt_factor);
+    __shared__ TileLds<T, Y::cols * Y::rows, Y::cols> sm;
+    const int bid = xcd_block(blockIdx.x, gridDim.x);
+    const int band = bid / ncolblk;
+    sweep_y_tile<T, FLUX, PROJ, EOS, DXM, Y::cols, Y::rows, Y::threads>(a, dt, (bid - band * ncolblk) * Y::cols,
+                                                                        band * W, sm);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -705,6 +1207,7 @@ __device__ __forceinline__ SweepArgs<T> batch_domain_args(const BatchArgs<T>& b,
     a.stale_p = b.stale_p + D.offset;
     a.stale_c = b.stale_c + D.offset;
     a.st = b.states + d;
+    a.prev = nullptr;
     a.nx = D.nx;
     a.ny = D.ny;
     a.row_length = D.row_length;
@@ -731,7 +1234,7 @@ __device__ __forceinline__ SweepArgs<T> batch_domain_args(const BatchArgs<T>& b,
 template <class T, int FLUX, int PROJ, int EOS, int TILE>
 __global__ void __launch_bounds__(TILE) k_batch_x(BatchArgs<T> b, const BatchItemX* __restrict__ items, int nitems)
 {
-    __shared__ SmemX<T, TILE> sm;
+    __shared__ TileLds<T, TILE, 1> sm;
     for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
         const BatchItemX item = items[it];
         const DeviceState* st = b.states + item.domain;
@@ -749,7 +1252,7 @@ __global__ void __launch_bounds__(TILE) k_batch_x(BatchArgs<T> b, const BatchIte
 template <class T, int FLUX, int PROJ, int EOS, int TILE, int CPT = 1>
 __global__ void __launch_bounds__(TILE / CPT) k_batch_x1(BatchArgs<T> b, const BatchItemX* __restrict__ items)
 {
-    __shared__ SmemX<T, TILE> sm;
+    __shared__ TileLds<T, TILE, 1> sm;
     const BatchItemX item = items[xcd_block(blockIdx.x, gridDim.x)];
     const DeviceState* st = b.states + item.domain;
     if (!st->active) return;
@@ -776,8 +1279,7 @@ __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)
         if (!st->active) continue;   // the same for the whole wave
         const SweepArgs<T> a = batch_domain_args(b, item.domain, 1);
         const int x = item.x0 + lane;
-        constexpr bool ahead = ARMON_Y_PREFETCH;
-        sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE, ahead>(a, (T) (st->current_dt * b.dt_factor), x,
+            sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE>(a, (T) (st->current_dt * b.dt_factor), x,
                                                                        item.y0, item.y1);
     }
 }
@@ -813,15 +1315,14 @@ __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)
     const DeviceState* st = b.states + item.domain;
     const SweepArgs<T> a = batch_domain_args(b, item.domain, 1);
     const int x = item.x0 + lane;
-    constexpr bool ahead = ARMON_Y_PREFETCH;
     const T dt = (T) (st->current_dt * b.dt_factor);
     if constexpr (!STALE) {
         if (sync) {
-            sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE, ahead, true>(a, dt, x, item.y0, item.y1);
+            sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE, true>(a, dt, x, item.y0, item.y1);
             return;
         }
     }
-    sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE, ahead>(a, dt, x, item.y0, item.y1);
+    sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE>(a, dt, x, item.y0, item.y1);
 }
 
 // X tiles covering a stream of `slots` slots (tiles of W outputs overlapping by 2R): the last
@@ -910,6 +1411,15 @@ void launch_variant(int axis, const SweepArgs<T>& a, hipStream_t s)
         k_sweep_x<T, F, P, E, DXM><<<dim3((unsigned) tiles), dim3(XTile<T>::cells / XTile<T>::cpt), 0, s>>>(b);
         check_launch("sweep_x");
     } else {
+        using Y = YTile<T>;
+        // a run length that the caller gives is a march's
+        if (a.seg_len <= 0 && (int64_t) a.nx * a.ny <= Y::max_cells) {
+            constexpr int W = Y::rows - 2 * R;
+            const int nc = (a.nx + Y::cols - 1) / Y::cols, nb = (a.ny + W - 1) / W;
+            k_sweep_y_tile<T, F, P, E, DXM><<<dim3((unsigned) (nc * nb)), dim3(Y::threads), 0, s>>>(a, nc);
+            check_launch("sweep_y_tile");
+            return;
+        }
         // Each block marches down a run of rows of its 256 columns (the warm-up is paid once
         // per run); blocks are numbered row band by row band (segment-major).
         const int ncolblk = (a.nx + kYBlock - 1) / kYBlock;
