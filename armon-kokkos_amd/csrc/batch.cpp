@@ -62,13 +62,14 @@ struct ArmonBatch {
     ArmonParams common{};
     std::vector<ArmonParams> p;          // per domain, through armon_params_init
     std::vector<ArmonTestState> states;
+    std::vector<BatchDomain> domains;    // as on the device
     std::vector<int64_t> offset;         // first element of each domain in the packed arrays
     int64_t total = 0;                   // packed elements
     int64_t real_cells = 0;
     double* arr[ARMON_FIELD_COUNT] = {};
     float* f32[10] = {};                 // FP32-mixed: A rho,u,v,E | B rho,u,v,E | stale p, c
     BatchDomain* d_domains = nullptr;
-    DeviceState* d_states = nullptr;
+    DeviceState* d_states = nullptr;     // two per domain: the cycles step from one set to the other
     DeviceState* d_tune = nullptr;       // scratch states used while timing candidates
     TimeStepConfig* d_cfgs = nullptr;
     std::vector<BatchItemX> items_x;
@@ -76,6 +77,7 @@ struct ArmonBatch {
     BatchItemX* d_items_x = nullptr;
     BatchItemY* d_items_y = nullptr;
     ArmonBatchTuning tuning{};
+    bool y_tiles = false;                // the Y items are LDS tiles, not the tuning's marching runs
     SweepVariant var{};
     int sweeps_per_cycle = 2;
     int64_t cycles_enqueued = 0;
@@ -91,6 +93,16 @@ struct ArmonBatch {
         return view{arr[field] + offset[d], (int64_t) p[d].nb_cells, nullptr};
     }
     bool fp64() const { return common.precision == ARMON_PREC_FP64; }
+    // the states as of `cycles` enqueued cycles
+    DeviceState* states_at(int64_t cycles) const { return d_states + (cycles & 1) * (int64_t) p.size(); }
+    FieldArrays fields() const
+    {
+        FieldArrays f{arr[ARMON_FIELD_RHO],  arr[ARMON_FIELD_UMAT], arr[ARMON_FIELD_VMAT], arr[ARMON_FIELD_EMAT],
+                      arr[ARMON_FIELD_PMAT], arr[ARMON_FIELD_CMAT], arr[ARMON_FIELD_GMAT], {}, {}};
+        for (int k = 0; k < 4; k++) f.other[k] = arr[ARMON_FIELD_WORK1 + k];
+        for (int k = 0; k < 10; k++) f.f32[k] = f32[k];
+        return f;
+    }
 };
 
 ArmonBatch::~ArmonBatch()
@@ -122,7 +134,7 @@ void fail(const char* where, const std::exception& e)
 // at most `run` rows) of every domain, band by band, so that the waves of a block march
 // neighbouring column groups of one band (measured 2% faster in FP64 and 12% in FP32-mixed
 // than column group by column group); then longest runs first (a stable sort) so that a
-// grid-stride walk over them balances well.
+// grid-stride walk over them balances well. Y tiles: band by band too.
 // Destroys the captured graphs: they hold the work lists' addresses and the launch grids.
 void drop_graphs(ArmonBatch* b)
 {
@@ -149,6 +161,12 @@ void build_items(ArmonBatch* b, int run)
         for (int64_t t = 0; t < tiles; t++) {
             const int64_t s0 = t * W;
             b->items_x.push_back(BatchItemX{d, (int) (s0 / slots), (int) (s0 % slots), 0});
+        }
+        if (b->y_tiles) {
+            const int rows = y_tile_outputs(b->var);
+            for (int y0 = 0; y0 < q.ny; y0 += rows)
+                for (int x0 = 0; x0 < q.nx; x0 += y_tile_cols()) b->items_y.push_back(BatchItemY{d, x0, y0, 0});
+            continue;
         }
         for (int y0 = 0; y0 < q.ny; y0 += run)
             for (int x0 = 0; x0 < q.nx; x0 += kWave) b->items_y.push_back(BatchItemY{d, x0, y0, std::min(y0 + run, q.ny)});
@@ -184,7 +202,8 @@ int blocks_y(const ArmonBatch* b, int grid)
 }
 
 template <class T>
-BatchArgs<T> batch_args(ArmonBatch* b, int parity, double factor, bool reduce, DeviceState* states)
+BatchArgs<T> batch_args(ArmonBatch* b, int parity, double factor, bool reduce, DeviceState* states,
+                        const DeviceState* prev)
 {
     BatchArgs<T> a{};
     T* A[4];
@@ -211,6 +230,8 @@ BatchArgs<T> batch_args(ArmonBatch* b, int parity, double factor, bool reduce, D
     a.stale_c = sc;
     a.domains = b->d_domains;
     a.states = states;
+    a.prev = prev;
+    a.steps = b->d_cfgs;
     a.stencil_width = b->common.stencil_width;
     a.reduce = reduce ? 1 : 0;
     a.gamma = 1.4;
@@ -218,18 +239,21 @@ BatchArgs<T> batch_args(ArmonBatch* b, int parity, double factor, bool reduce, D
     return a;
 }
 
-void launch_one_sweep(ArmonBatch* b, int axis, int parity, double factor, bool reduce, DeviceState* states)
+// With `prev`, the sweep makes the domains' time step from there into `states`.
+void launch_one_sweep(ArmonBatch* b, int axis, int parity, double factor, bool reduce, DeviceState* states,
+                      const DeviceState* prev = nullptr)
 {
     const bool x = axis == ARMON_AXIS_X;
     const void* items = x ? (const void*) b->d_items_x : (const void*) b->d_items_y;
     const int nitems = x ? (int) b->items_x.size() : (int) b->items_y.size();
     const int grid = x ? blocks_x(b, b->tuning.grid_x) : blocks_y(b, b->tuning.grid_y);
+    const int tile = x ? b->tuning.tile_x : b->y_tiles ? 1 : 0;
     if (b->fp64())
-        launch_batch_sweep<double>(axis, b->var, batch_args<double>(b, parity, factor, reduce, states), items, nitems,
-                                   grid, b->tuning.tile_x, b->tuning.x_cells_per_thread, b->stream);
+        launch_batch_sweep<double>(axis, b->var, batch_args<double>(b, parity, factor, reduce, states, prev), items,
+                                   nitems, grid, tile, b->tuning.x_cells_per_thread, b->stream);
     else
-        launch_batch_sweep<float>(axis, b->var, batch_args<float>(b, parity, factor, reduce, states), items, nitems,
-                                  grid, b->tuning.tile_x, b->tuning.x_cells_per_thread, b->stream);
+        launch_batch_sweep<float>(axis, b->var, batch_args<float>(b, parity, factor, reduce, states, prev), items, nitems,
+                                  grid, tile, b->tuning.x_cells_per_thread, b->stream);
 }
 
 struct Timer {
@@ -261,18 +285,23 @@ struct Timer {
 // Cycle `cycle` of every domain: the per-domain time step, then the sweeps of the splitting.
 void enqueue_cycle(ArmonBatch* b, int64_t cycle, Timer* t)
 {
-    if (t) t->begin();
-    launch_batch_time_step(b->d_states, b->d_states, b->d_cfgs, (int) b->p.size(), b->stream);
-    if (t) t->end(2);
+    const DeviceState* prev = b->states_at(cycle);
+    DeviceState* states = b->states_at(cycle + 1);
     ArmonParams pc = b->common;
     pc.cycle = (int) cycle;
     int axes[3];
     double factors[3];
     const int n = armon_split_axes(&pc, axes, factors);
+    // the first sweep makes the time step where each of its blocks has one item
+    const bool single = axes[0] == ARMON_AXIS_X ? b->tuning.grid_x == 0 : b->y_tiles;
+    const bool folded = n > 1 && single && b->real_cells <= kFoldedCells;
+    if (t) t->begin();
+    if (!folded) launch_batch_time_step(prev, states, b->d_cfgs, (int) b->p.size(), b->stream);
+    if (t) t->end(2);
     int parity = (int) ((cycle * b->sweeps_per_cycle) & 1);
     for (int k = 0; k < n; k++) {
         if (t) t->begin();
-        launch_one_sweep(b, axes[k], parity, factors[k], k == n - 1, b->d_states);
+        launch_one_sweep(b, axes[k], parity, factors[k], k == n - 1, states, folded && k == 0 ? prev : nullptr);
         if (t) t->end(axes[k] == ARMON_AXIS_X ? 0 : 1);
         parity ^= 1;
     }
@@ -320,32 +349,26 @@ void advance(ArmonBatch* b, int64_t n)
 std::vector<DeviceState> read_states(ArmonBatch* b)
 {
     std::vector<DeviceState> h(b->p.size());
-    hip_check(hipMemcpyAsync(h.data(), b->d_states, sizeof(DeviceState) * h.size(), hipMemcpyDeviceToHost, b->stream),
+    hip_check(hipMemcpyAsync(h.data(), b->states_at(b->cycles_enqueued), sizeof(DeviceState) * h.size(), hipMemcpyDeviceToHost, b->stream),
               "read device states");
     hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
     return h;
 }
 
-// Working buffers from the reference arrays: FP64 copies A into B (ghost layers the sweeps
-// never write must hold the initial values in both); FP32-mixed rounds A into both FP32
-// buffers and pmat/cmat into the stale-ghost buffers.
-void prepare_buffers(ArmonBatch* b)
+// The states before the first cycle, then the EOS and CFL minima of the initial fields and the working
+// buffers (launch_begin).
+void begin_fields(ArmonBatch* b, DeviceState* states)
 {
-    const size_t n = (size_t) b->total;
-    const int src[4] = {ARMON_FIELD_RHO, ARMON_FIELD_UMAT, ARMON_FIELD_VMAT, ARMON_FIELD_EMAT};
-    if (b->fp64()) {
-        for (int f = 0; f < 4; f++)
-            hip_check(hipMemcpyAsync(b->arr[ARMON_FIELD_WORK1 + f], b->arr[src[f]], sizeof(double) * n,
-                                     hipMemcpyDeviceToDevice, b->stream),
-                      "copy state");
-    } else {
-        for (int f = 0; f < 4; f++) {
-            launch_convert_d2f(b->arr[src[f]], b->f32[f], (int64_t) n, b->stream);
-            launch_convert_d2f(b->arr[src[f]], b->f32[4 + f], (int64_t) n, b->stream);
-        }
-        launch_convert_d2f(b->arr[ARMON_FIELD_PMAT], b->f32[8], (int64_t) n, b->stream);
-        launch_convert_d2f(b->arr[ARMON_FIELD_CMAT], b->f32[9], (int64_t) n, b->stream);
+    const int n = (int) b->p.size();
+    std::vector<DeviceState> zero(n);
+    for (auto& s : zero) {
+        memset(&s, 0, sizeof s);
+        for (auto& slot : s.dt_min) slot.bits = kNoBound;
     }
+    hip_check(hipMemcpyAsync(states, zero.data(), sizeof(DeviceState) * n, hipMemcpyHostToDevice, b->stream),
+              "init device states");
+    launch_begin(b->fields(), b->d_domains, n, b->domains[0], b->total, states, b->var.eos, 1.4, b->stream);
+    hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
 }
 
 // Average time of `reps` launches of one sweep under the current tuning (after one warm-up).
@@ -507,14 +530,16 @@ ARMON_EXPORT ArmonBatch* armon_batch_create(const ArmonParams* common, int n, co
             D.x_inv_slots = 1.0f / (float) D.x_slots;
             cfg[d] = TimeStepConfig{q.cfl, q.Dt, q.max_time, q.max_cycles, q.cst_dt, q.dt_on_even_cycles};
         }
+        b->domains = dom;
         b->d_domains = device_alloc<BatchDomain>(n, "hipMalloc(domains)");
         b->d_cfgs = device_alloc<TimeStepConfig>(n, "hipMalloc(configs)");
-        b->d_states = device_alloc<DeviceState>(n, "hipMalloc(states)");
+        b->d_states = device_alloc<DeviceState>(2 * (size_t) n, "hipMalloc(states)");
         b->d_tune = device_alloc<DeviceState>(n, "hipMalloc(tune states)");
         hip_check(hipMemcpy(b->d_domains, dom.data(), sizeof(BatchDomain) * n, hipMemcpyHostToDevice), "upload domains");
         hip_check(hipMemcpy(b->d_cfgs, cfg.data(), sizeof(TimeStepConfig) * n, hipMemcpyHostToDevice), "upload configs");
-        // default configuration: 256-cell X tiles of one cell per thread, 256-row Y runs, one
-        // block per work item
+        // default configuration: 256-cell X tiles of one cell per thread, Y tiles or 256-row Y runs by
+        // the number of cells, one block per work item
+        b->y_tiles = b->real_cells <= y_tile_max_cells(b->fp64() ? 8 : 4);
         b->tuning.tile_x = 256;
         b->tuning.x_cells_per_thread = 1;
         b->tuning.grid_x = 0;
@@ -597,6 +622,7 @@ ARMON_EXPORT int armon_batch_set_tuning(ArmonBatch* b, const ArmonBatchTuning* t
         b->tuning.x_cells_per_thread = cpt;
         b->tuning.grid_x = std::max(0, t->grid_x);
         b->tuning.grid_y = std::max(0, t->grid_y);
+        b->y_tiles = false;
         build_items(b, t->y_run_rows);
         return 0;
     } catch (const std::exception& e) {
@@ -609,7 +635,7 @@ ARMON_EXPORT int armon_batch_autotune(ArmonBatch* b, ArmonBatchTuning* out)
 {
     try {
         check_ready(b, true, true);
-        prepare_buffers(b);
+        begin_fields(b, b->d_tune);
         // every domain active with a small positive dt: the work of a real cycle
         std::vector<DeviceState> tune(b->p.size());
         for (auto& s : tune) {
@@ -629,6 +655,7 @@ ARMON_EXPORT int armon_batch_autotune(ArmonBatch* b, ArmonBatchTuning* out)
         // X: tile width (128, 256, 512 cells, one per thread) x (persistent grids of 1, 2, 4
         // resident rounds | one block per tile), then tiles of 256 and 512 cells at two cells
         // per thread (one block per tile)
+        b->y_tiles = false;
         double best_x = 1e300;
         int grid_x = 0, tile_x = 256, cpt_x = 1;
         const int run0 = b->tuning.y_run_rows;
@@ -668,8 +695,17 @@ ARMON_EXPORT int armon_batch_autotune(ArmonBatch* b, ArmonBatchTuning* out)
                 if (ms < best_y) { best_y = ms; grid_y = g; run_y = run; }
             }
         }
-        b->tuning.grid_y = grid_y;
+        // Y tiles beside the marches: the fastest march stays in the tuning, for a batch that takes it
+        b->y_tiles = true;
         build_items(b, run_y);
+        const double ms_tiles = time_sweep(b, ARMON_AXIS_Y, reps);
+        b->tuning.grid_y = grid_y;
+        if (ms_tiles < best_y) {
+            best_y = ms_tiles;
+        } else {
+            b->y_tiles = false;
+            build_items(b, run_y);
+        }
         b->tuning.ms_x = best_x;
         b->tuning.ms_y = best_y;
         if (out) *out = b->tuning;
@@ -686,35 +722,7 @@ ARMON_EXPORT int armon_batch_begin(ArmonBatch* b)
 {
     try {
         check_ready(b, true, true);
-        StreamScope scope(b->stream);
-        const uint64_t e0 = report_count();
-        const int n = (int) b->p.size();
-        for (int d = 0; d < n; d++) {
-            const ArmonParams& q = b->p[d];
-            DomainRange dr = armon_real_domain(&q);
-            Range range;
-            InnerRange2D inner;
-            armon_domain_iter2D(&dr, &range, &inner);
-            view rho = b->slice(ARMON_FIELD_RHO, d), u = b->slice(ARMON_FIELD_UMAT, d), v = b->slice(ARMON_FIELD_VMAT, d),
-                 E = b->slice(ARMON_FIELD_EMAT, d), pm = b->slice(ARMON_FIELD_PMAT, d), cm = b->slice(ARMON_FIELD_CMAT, d),
-                 gm = b->slice(ARMON_FIELD_GMAT, d);
-            if (q.test == 3) bizarrium_EOS(range, inner, rho, u, v, E, pm, cm, gm);
-            else perfect_gas_EOS(range, inner, 1.4, rho, E, u, v, pm, cm, gm);
-        }
-        if (report_count() != e0) return 1;
-        prepare_buffers(b);
-        std::vector<DeviceState> zero(n);
-        memset(zero.data(), 0, sizeof(DeviceState) * n);
-        hip_check(hipMemcpyAsync(b->d_states, zero.data(), sizeof(DeviceState) * n, hipMemcpyHostToDevice, b->stream),
-                  "init device states");
-        for (int d = 0; d < n; d++) {
-            const ArmonParams& q = b->p[d];
-            const int64_t o = b->offset[d];
-            launch_cfl_real<double>(b->d_states + d, b->arr[ARMON_FIELD_UMAT] + o, b->arr[ARMON_FIELD_VMAT] + o,
-                                    b->arr[ARMON_FIELD_CMAT] + o, q.nx, q.ny, q.row_length, q.index_start,
-                                    q.domain_size[0] / (double) q.nx, q.domain_size[1] / (double) q.ny, b->stream);
-        }
-        hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
+        begin_fields(b, b->d_states);
         b->cycles_enqueued = 0;
         // both graphs now, so that no later advance pays for a capture
         if (b->common.graph_chunk > 0)
@@ -780,7 +788,6 @@ ARMON_EXPORT int armon_batch_finish(ArmonBatch* b)
         if (b->finished) return 0;
         b->final_states = read_states(b);
         int status = 0;
-        const int eos = b->var.eos;
         for (int d = 0; d < (int) b->p.size(); d++) {
             const DeviceState& h = b->final_states[d];
             ArmonParams& q = b->p[d];
@@ -789,32 +796,9 @@ ARMON_EXPORT int armon_batch_finish(ArmonBatch* b)
             q.current_cycle_dt = h.current_dt;
             q.next_cycle_dt = h.next_dt;
             if (h.error) status = 1;
-            const int64_t sweeps = (int64_t) h.cycle * b->sweeps_per_cycle;
-            if (sweeps == 0) continue;
-            const int cur = (int) (sweeps & 1);
-            const int64_t o = b->offset[d];
-            double* P = b->arr[ARMON_FIELD_PMAT] + o;
-            double* C = b->arr[ARMON_FIELD_CMAT] + o;
-            double* G = b->arr[ARMON_FIELD_GMAT] + o;
-            const int fa[4] = {ARMON_FIELD_RHO, ARMON_FIELD_UMAT, ARMON_FIELD_VMAT, ARMON_FIELD_EMAT};
-            const int fb[4] = {ARMON_FIELD_WORK1, ARMON_FIELD_WORK2, ARMON_FIELD_WORK3, ARMON_FIELD_WORK4};
-            if (b->fp64()) {
-                const int* in = cur ? fa : fb;   // input of the last sweep
-                launch_eos_real<double>(b->arr[in[0]] + o, b->arr[in[1]] + o, b->arr[in[2]] + o, b->arr[in[3]] + o, P,
-                                        C, G, eos, 1.4, q.nx, q.ny, q.row_length, q.index_start, b->stream);
-                if (cur)
-                    for (int f = 0; f < 4; f++)
-                        hip_check(hipMemcpyAsync(b->arr[fa[f]] + o, b->arr[fb[f]] + o, sizeof(double) * q.nb_cells,
-                                                 hipMemcpyDeviceToDevice, b->stream),
-                                  "copy final state");
-            } else {
-                float* const* in = cur ? &b->f32[0] : &b->f32[4];
-                launch_eos_real<float>(in[0] + o, in[1] + o, in[2] + o, in[3] + o, P, C, G, eos, 1.4, q.nx, q.ny,
-                                       q.row_length, q.index_start, b->stream);
-                for (int f = 0; f < 4; f++)
-                    launch_convert_f2d(b->f32[(cur ? 4 : 0) + f] + o, b->arr[fa[f]] + o, q.nb_cells, b->stream);
-            }
         }
+        launch_finish(b->fields(), b->d_domains, (int) b->p.size(), b->domains[0], b->total,
+                      b->states_at(b->cycles_enqueued), b->sweeps_per_cycle, b->var.eos, 1.4, b->stream);
         hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
         b->finished = true;
         b->initialized = false;   // a new run starts from armon_batch_init

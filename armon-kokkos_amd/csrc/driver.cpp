@@ -547,30 +547,36 @@ DeviceState read_state(ArmonSolver* s)
     return h;
 }
 
+FieldArrays field_arrays(ArmonSolver* s)
+{
+    FieldArrays f{s->arr[ARMON_FIELD_RHO],  s->arr[ARMON_FIELD_UMAT], s->arr[ARMON_FIELD_VMAT], s->arr[ARMON_FIELD_EMAT],
+                  s->arr[ARMON_FIELD_PMAT], s->arr[ARMON_FIELD_CMAT], s->arr[ARMON_FIELD_GMAT], {}, {}};
+    for (int k = 0; k < 4; k++) f.other[k] = s->arr[ARMON_FIELD_WORK1 + k];
+    for (int k = 0; k < 10; k++) f.f32[k] = s->f32[k];
+    return f;
+}
+
+// The solver's domain as launch_begin and launch_finish take it.
+BatchDomain own_domain(const ArmonSolver* s)
+{
+    const ArmonParams& p = s->p;
+    BatchDomain d{};
+    d.nx = p.nx;
+    d.ny = p.ny;
+    d.row_length = p.row_length;
+    d.index_start = p.index_start;
+    d.cfl_dx = p.domain_size[0] / (double) p.nx;
+    d.cfl_dy = p.domain_size[1] / (double) p.ny;
+    return d;
+}
+
 void fused_begin(ArmonSolver* s)
 {
     ArmonParams& p = s->p;
-    const int64_t n = s->n;
-    const size_t bytes = sizeof(double) * (size_t) n;
-    if (p.precision == ARMON_PREC_FP64) {
-        for (int f = 0; f < 4; f++)
-            hip_check(hipMemcpyAsync(s->arr[ARMON_FIELD_WORK1 + f], s->arr[ARMON_FIELD_RHO + (f == 3 ? 3 : f)], bytes,
-                                     hipMemcpyDeviceToDevice, s->stream),
-                      "copy state");
-    } else {
-        const int src[4] = {ARMON_FIELD_RHO, ARMON_FIELD_UMAT, ARMON_FIELD_VMAT, ARMON_FIELD_EMAT};
-        for (int f = 0; f < 4; f++) {
-            launch_convert_d2f(s->arr[src[f]], s->f32[f], n, s->stream);
-            launch_convert_d2f(s->arr[src[f]], s->f32[4 + f], n, s->stream);
-        }
-        launch_convert_d2f(s->arr[ARMON_FIELD_PMAT], s->f32[8], n, s->stream);
-        launch_convert_d2f(s->arr[ARMON_FIELD_CMAT], s->f32[9], n, s->stream);
-    }
     DeviceState h{};
+    for (auto& slot : h.dt_min) slot.bits = kNoBound;
     hip_check(hipMemcpyAsync(s->st, &h, sizeof h, hipMemcpyHostToDevice, s->stream), "init device state");
-    launch_cfl_real<double>(s->st, s->arr[ARMON_FIELD_UMAT], s->arr[ARMON_FIELD_VMAT], s->arr[ARMON_FIELD_CMAT], p.nx,
-                            p.ny, p.row_length, p.index_start, p.domain_size[0] / (double) p.nx,
-                            p.domain_size[1] / (double) p.ny, s->stream);
+    launch_begin(field_arrays(s), nullptr, 1, own_domain(s), s->n, s->st, p.test == 3 ? 1 : 0, 1.4, s->stream);
     hip_check(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
     s->cycles_enqueued = 0;
     // both graphs now, so that no later advance pays for a capture
@@ -581,37 +587,11 @@ void fused_begin(ArmonSolver* s)
 
 // After the loop: put the final state in rho/umat/vmat/Emat and the EOS of the last sweep's
 // input state in pmat/cmat/gmat, as the reference leaves them.
-void fused_finish(ArmonSolver* s, const DeviceState& h)
+void fused_finish(ArmonSolver* s)
 {
     const ArmonParams& p = s->p;
-    const int64_t sweeps = (int64_t) h.cycle * s->sweeps_per_cycle;
-    if (sweeps == 0) return;
-    const int cur = (int) (sweeps & 1);    // buffer holding the final state (0: A, 1: B)
-    const int eos = p.test == 3 ? 1 : 0;
-    double* P = s->arr[ARMON_FIELD_PMAT];
-    double* C = s->arr[ARMON_FIELD_CMAT];
-    double* G = s->arr[ARMON_FIELD_GMAT];
-    if (p.precision == ARMON_PREC_FP64) {
-        double* A[4] = {s->arr[ARMON_FIELD_RHO], s->arr[ARMON_FIELD_UMAT], s->arr[ARMON_FIELD_VMAT],
-                        s->arr[ARMON_FIELD_EMAT]};
-        double* B[4] = {s->arr[ARMON_FIELD_WORK1], s->arr[ARMON_FIELD_WORK2], s->arr[ARMON_FIELD_WORK3],
-                        s->arr[ARMON_FIELD_WORK4]};
-        double** in = cur ? A : B;   // input of the last sweep
-        launch_eos_real<double>(in[0], in[1], in[2], in[3], P, C, G, eos, 1.4, p.nx, p.ny, p.row_length,
-                                p.index_start, s->stream);
-        if (cur)
-            for (int f = 0; f < 4; f++)
-                hip_check(hipMemcpyAsync(A[f], B[f], sizeof(double) * (size_t) s->n, hipMemcpyDeviceToDevice,
-                                         s->stream),
-                          "copy final state");
-    } else {
-        float* in = cur ? s->f32[0] : s->f32[4];
-        launch_eos_real<float>(in, in == s->f32[0] ? s->f32[1] : s->f32[5], in == s->f32[0] ? s->f32[2] : s->f32[6],
-                               in == s->f32[0] ? s->f32[3] : s->f32[7], P, C, G, eos, 1.4, p.nx, p.ny, p.row_length,
-                               p.index_start, s->stream);
-        const int dst[4] = {ARMON_FIELD_RHO, ARMON_FIELD_UMAT, ARMON_FIELD_VMAT, ARMON_FIELD_EMAT};
-        for (int f = 0; f < 4; f++) launch_convert_f2d(s->f32[(cur ? 4 : 0) + f], s->arr[dst[f]], s->n, s->stream);
-    }
+    launch_finish(field_arrays(s), nullptr, 1, own_domain(s), s->n, s->st + (s->cycles_enqueued & 1),
+                  s->sweeps_per_cycle, p.test == 3 ? 1 : 0, 1.4, s->stream);
     hip_check(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
 }
 
@@ -1074,10 +1054,14 @@ ARMON_EXPORT int armon_solver_begin(ArmonSolver* s)
         s->t_begin = std::chrono::steady_clock::now();
         s->compare_stop = false;
         armon_update_axis(&p, ARMON_AXIS_X);
-        { Stage st(s->clock, "EOS_init", nullptr); staged_update_EOS(s); }
-        step_checkpoint(s, "EOS_init");
+        if (p.engine == ARMON_ENGINE_FUSED) {
+            Stage st(s->clock, "EOS_init", nullptr);
+            fused_begin(s);
+        } else {
+            { Stage st(s->clock, "EOS_init", nullptr); staged_update_EOS(s); }
+            step_checkpoint(s, "EOS_init");
+        }
         if (p.verbose <= 1) conservation(s, &s->initial_mass, &s->initial_energy);
-        if (p.engine == ARMON_ENGINE_FUSED) fused_begin(s);
         s->begun = true;
         return g_error_count != s->error_count_at_begin ? 1 : 0;
     } catch (const std::exception& e) {
@@ -1139,7 +1123,7 @@ ARMON_EXPORT int armon_solver_finish(ArmonSolver* s, ArmonResult* out)
                 armon_update_axis(&p, axes[n - 1]);
                 p.cycle_dt = p.current_cycle_dt * factors[n - 1];
             }
-            fused_finish(s, h);
+            fused_finish(s);
             if (h.error) {
                 char buf[128];
                 snprintf(buf, sizeof buf, "Invalid dt at cycle %d: %f", h.error_cycle, h.error_dt);

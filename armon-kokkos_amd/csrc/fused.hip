@@ -1,6 +1,5 @@
-// Fused engine, FP64 instantiation of the sweep kernels (sweep_kernels.hpp), plus the
-// device time step, the CFL reduction of a whole state, the EOS of a whole state and the
-// FP32 <-> FP64 conversions used by the FP32-mixed form.
+// Fused engine, FP64 instantiation of the sweep kernels (sweep_kernels.hpp), plus the kernels of
+// the time step and of what comes before the first cycle and after the last one.
 #include "sweep_kernels.hpp"
 
 #include <cfloat>
@@ -26,49 +25,130 @@ __global__ void __launch_bounds__(256) k_batch_time_step(const DeviceState* prev
     if (d < n) write_step(states + d, next_step(prev + d, cfgs[d]));
 }
 
-__global__ void k_reset_min(DeviceState* st) { st->dt_min[threadIdx.x].bits = kNoBound; }
-
-template <class T>
-__global__ void __launch_bounds__(256) k_cfl_real(DeviceState* st, const T* u, const T* v, const T* c, int nx, int ny,
-                                                  int row_length, int index_start, double cfl_dx, double cfl_dy)
-{
-    double local = DBL_MAX;
-    const int64_t total = (int64_t) nx * ny;
-    for (int64_t k = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; k < total; k += (int64_t) gridDim.x * blockDim.x) {
-        const int j = (int) (k / nx), i = (int) (k - (int64_t) j * nx);
-        const int idx = index_start + j * row_length + i;
-        local = kmin(local, cfl_cell<double>(cfl_dx, cfl_dy, (double) u[idx], (double) v[idx], (double) c[idx], 1.0));
-    }
-    reduce_cfl(st, local);
-}
-
-__global__ void k_d2f(const double* in, float* out, int64_t n)
-{
-    for (int64_t k = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t) gridDim.x * blockDim.x)
-        out[k] = (float) in[k];
-}
-
 __global__ void k_f2d(const float* in, double* out, int64_t n)
 {
     for (int64_t k = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t) gridDim.x * blockDim.x)
         out[k] = (double) in[k];
 }
 
-template <class T>
-__global__ void __launch_bounds__(256) k_eos_real(const T* rho, const T* u, const T* v, const T* E, double* p,
-                                                  double* c, double* g, int eos, double gamma, int nx, int ny,
-                                                  int row_length, int index_start)
+// Domains start on multiples of a wave's 64 elements, so a wave's elements belong to one domain: the
+// last whose offset is not past them.
+__device__ __forceinline__ int domain_of(const BatchDomain* domains, int n, int64_t element)
 {
-    const int64_t total = (int64_t) nx * ny;
-    for (int64_t k = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; k < total; k += (int64_t) gridDim.x * blockDim.x) {
-        const int j = (int) (k / nx), i = (int) (k - (int64_t) j * nx);
-        const int idx = index_start + j * row_length + i;
-        double pd, cd, gd;
-        if (eos == 0) perfect_gas<double>(gamma, (double) rho[idx], (double) E[idx], (double) u[idx], (double) v[idx], pd, cd, gd);
-        else bizarrium((double) rho[idx], (double) E[idx], (double) u[idx], (double) v[idx], pd, cd, gd);
-        p[idx] = pd;
-        c[idx] = cd;
-        g[idx] = gd;
+    int lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (domains[mid].offset <= element) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Whether element `i` of a domain is one of its real cells.
+__device__ __forceinline__ bool real_cell(const BatchDomain& d, int64_t i)
+{
+    const int g = d.index_start % d.row_length;   // ghost layers: index_start = (row_length + 1) g
+    const unsigned row = (unsigned) i / (unsigned) d.row_length, col = (unsigned) i - row * (unsigned) d.row_length;
+    return row - (unsigned) g < (unsigned) d.ny && col - (unsigned) g < (unsigned) d.nx;
+}
+
+__device__ __forceinline__ void full_eos(int eos, double gamma, double rho, double u, double v, double E, double& p,
+                                         double& c, double& g)
+{
+    if (eos == 0) perfect_gas<double>(gamma, rho, E, u, v, p, c, g);
+    else bizarrium(rho, E, u, v, p, c, g);
+}
+
+// Both kernels: one element a thread. They are bound by memory (FP64: 12 words an element in begin).
+__global__ void __launch_bounds__(256) k_begin(FieldArrays f, const BatchDomain* domains, int n, BatchDomain one,
+                                               int64_t elements, DeviceState* states, int eos, double gamma)
+{
+    const int64_t e = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t wave = (int64_t) blockIdx.x * blockDim.x + __builtin_amdgcn_readfirstlane((int) threadIdx.x);
+    if (wave >= elements) return;
+    const int which = n == 1 ? 0 : domain_of(domains, n, wave);
+    const BatchDomain d = n == 1 ? one : domains[which];
+    CflSpeeds speeds;
+    if (e < elements) {
+        const double rho = f.rho[e], u = f.u[e], v = f.v[e], E = f.E[e];
+        double p, c, g;
+        if (real_cell(d, e - d.offset)) {
+            full_eos(eos, gamma, rho, u, v, E, p, c, g);
+            f.p[e] = p;
+            f.c[e] = c;
+            f.g[e] = g;
+            speeds.add(u, v, c);
+        } else if (f.f32[0]) {
+            p = f.p[e];
+            c = f.c[e];
+        }
+        if (f.f32[0]) {
+            f.f32[0][e] = f.f32[4][e] = (float) rho;
+            f.f32[1][e] = f.f32[5][e] = (float) u;
+            f.f32[2][e] = f.f32[6][e] = (float) v;
+            f.f32[3][e] = f.f32[7][e] = (float) E;
+            f.f32[8][e] = (float) p;
+            f.f32[9][e] = (float) c;
+        } else {
+            f.other[0][e] = rho;
+            f.other[1][e] = u;
+            f.other[2][e] = v;
+            f.other[3][e] = E;
+        }
+    }
+    reduce_cfl(states + which, speeds.bound(d.cfl_dx, d.cfl_dy));
+}
+
+__global__ void __launch_bounds__(256) k_finish(FieldArrays f, const BatchDomain* domains, int n, BatchDomain one,
+                                                int64_t elements, const DeviceState* states, int sweeps_per_cycle,
+                                                int eos, double gamma)
+{
+    const int64_t e = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t wave = (int64_t) blockIdx.x * blockDim.x + __builtin_amdgcn_readfirstlane((int) threadIdx.x);
+    if (wave >= elements) return;
+    const int which = n == 1 ? 0 : domain_of(domains, n, wave);
+    const BatchDomain d = n == 1 ? one : domains[which];
+    const int64_t sweeps = (int64_t) states[which].cycle * sweeps_per_cycle;
+    if (sweeps == 0 || e >= elements) return;
+    const bool second = sweeps & 1;   // the final state is in the second buffer, the last input in the first
+    const bool real = real_cell(d, e - d.offset);
+    double rho, u, v, E;              // the last sweep's input
+    if (f.f32[0]) {
+        float* const* in = second ? f.f32 : f.f32 + 4;
+        float* const* out = second ? f.f32 + 4 : f.f32;
+        if (real) {
+            rho = (double) in[0][e];
+            u = (double) in[1][e];
+            v = (double) in[2][e];
+            E = (double) in[3][e];
+        }
+        f.rho[e] = (double) out[0][e];
+        f.u[e] = (double) out[1][e];
+        f.v[e] = (double) out[2][e];
+        f.E[e] = (double) out[3][e];
+    } else if (second) {
+        if (real) {
+            rho = f.rho[e];
+            u = f.u[e];
+            v = f.v[e];
+            E = f.E[e];
+        }
+        f.rho[e] = f.other[0][e];
+        f.u[e] = f.other[1][e];
+        f.v[e] = f.other[2][e];
+        f.E[e] = f.other[3][e];
+    } else if (real) {
+        rho = f.other[0][e];
+        u = f.other[1][e];
+        v = f.other[2][e];
+        E = f.other[3][e];
+    }
+    if (real) {
+        double p, c, g;
+        full_eos(eos, gamma, rho, u, v, E, p, c, g);
+        f.p[e] = p;
+        f.c[e] = c;
+        f.g[e] = g;
     }
 }
 
@@ -94,26 +174,26 @@ void launch_batch_time_step(const DeviceState* prev, DeviceState* states, const 
     check_launch("batch_time_step");
 }
 
-template <class T>
-void launch_cfl_real(DeviceState* st, const T* u, const T* v, const T* c, int nx, int ny, int row_length,
-                     int index_start, double cfl_dx, double cfl_dy, hipStream_t s)
+static unsigned element_blocks(int64_t elements)
 {
-    k_reset_min<<<1, kDtSlots, 0, s>>>(st);
-    check_launch("cfl_reset");
-    k_cfl_real<T><<<grid_for((int64_t) nx * ny, 256, 2048), 256, 0, s>>>(st, u, v, c, nx, ny, row_length, index_start,
-                                                                         cfl_dx, cfl_dy);
-    check_launch("cfl_real");
+    const int64_t g = (elements + 255) / 256;
+    if (g > INT32_MAX) throw std::runtime_error("too many elements for one launch");
+    return (unsigned) g;
 }
 
-template void launch_cfl_real<double>(DeviceState*, const double*, const double*, const double*, int, int, int, int,
-                                      double, double, hipStream_t);
-template void launch_cfl_real<float>(DeviceState*, const float*, const float*, const float*, int, int, int, int,
-                                     double, double, hipStream_t);
-
-void launch_convert_d2f(const double* in, float* out, int64_t n, hipStream_t s)
+void launch_begin(const FieldArrays& f, const BatchDomain* domains, int n, const BatchDomain& one, int64_t elements,
+                  DeviceState* states, int eos, double gamma, hipStream_t s)
 {
-    k_d2f<<<grid_for(n, 256, 8192), 256, 0, s>>>(in, out, n);
-    check_launch("convert_d2f");
+    k_begin<<<element_blocks(elements), 256, 0, s>>>(f, domains, n, one, elements, states, eos, gamma);
+    check_launch("begin");
+}
+
+void launch_finish(const FieldArrays& f, const BatchDomain* domains, int n, const BatchDomain& one, int64_t elements,
+                   const DeviceState* states, int sweeps_per_cycle, int eos, double gamma, hipStream_t s)
+{
+    k_finish<<<element_blocks(elements), 256, 0, s>>>(f, domains, n, one, elements, states, sweeps_per_cycle, eos,
+                                                      gamma);
+    check_launch("finish");
 }
 
 void launch_convert_f2d(const float* in, double* out, int64_t n, hipStream_t s)
@@ -121,19 +201,5 @@ void launch_convert_f2d(const float* in, double* out, int64_t n, hipStream_t s)
     k_f2d<<<grid_for(n, 256, 8192), 256, 0, s>>>(in, out, n);
     check_launch("convert_f2d");
 }
-
-template <class T>
-void launch_eos_real(const T* rho, const T* u, const T* v, const T* E, double* p, double* c, double* g, int eos,
-                     double gamma, int nx, int ny, int row_length, int index_start, hipStream_t s)
-{
-    k_eos_real<T><<<grid_for((int64_t) nx * ny, 256, 8192), 256, 0, s>>>(rho, u, v, E, p, c, g, eos, gamma, nx, ny,
-                                                                          row_length, index_start);
-    check_launch("eos_real");
-}
-
-template void launch_eos_real<double>(const double*, const double*, const double*, const double*, double*, double*,
-                                      double*, int, double, int, int, int, int, hipStream_t);
-template void launch_eos_real<float>(const float*, const float*, const float*, const float*, double*, double*,
-                                     double*, int, double, int, int, int, int, hipStream_t);
 
 }  // namespace armon

@@ -115,7 +115,8 @@ struct BatchArgs {
 // One launch sweeps every domain of the batch along `axis`: `grid` persistent blocks walk
 // the work items (BatchItemX for X, BatchItemY for Y); X tiles are `tile` cells wide (128,
 // 256 or 512, the width the X items were cut for), `cpt` cells per thread (1, or 2 for tiles of
-// 256 or 512 cells, one block per tile whatever `grid`).
+// 256 or 512 cells, one block per tile whatever `grid`). Y items are marching runs (`tile` 0) or LDS
+// tiles (`tile` 1: y_tile_cols() x y_tile_outputs() cells, one block per tile).
 template <class T>
 void launch_batch_sweep(int axis, const SweepVariant& v, const BatchArgs<T>& b, const void* items, int nitems,
                         int grid, int tile, int cpt, hipStream_t s);
@@ -125,22 +126,40 @@ void launch_batch_sweep(int axis, const SweepVariant& v, const BatchArgs<T>& b, 
 template <class T>
 int batch_resident_blocks(int axis, const SweepVariant& v, int tile);
 
+// Columns and output rows of a Y tile, and the number of cells up to which a sweep along y takes tiles.
+constexpr int y_tile_cols() { return 16; }
+constexpr int y_tile_rows() { return 32; }
+inline int y_tile_outputs(const SweepVariant& v) { return y_tile_rows() - 2 * read_extent(v.flux, v.proj); }
+constexpr int64_t y_tile_max_cells(size_t element) { return element == 8 ? 5 << 19 : 7 << 19; }   // 2.6 M, 3.7 M
+
 // The time step of every domain (one wave each), per-domain configuration.
 void launch_batch_time_step(const DeviceState* prev, DeviceState* states, const TimeStepConfig* cfgs, int n,
                             hipStream_t s);
 
-// CFL minimum of the real cells into st->dt_min (after resetting it).
-template <class T>
-void launch_cfl_real(DeviceState* st, const T* u, const T* v, const T* c, int nx, int ny, int row_length,
-                     int index_start, double cfl_dx, double cfl_dy, hipStream_t s);
+// ---- before and after the cycles -----------------------------------------------------------
 
-// Element-wise conversions between the reference FP64 arrays and FP32 working buffers.
-void launch_convert_d2f(const double* in, float* out, int64_t n, hipStream_t s);
+// The arrays of one domain, or of every domain of a batch packed one after the other: the FP64 fields
+// and, where the cycles run in them, the FP32 buffers.
+struct FieldArrays {
+    double *rho, *u, *v, *E, *p, *c, *g;
+    double* other[4];     // FP64: the second state buffer (rho, u, v, E)
+    float* f32[10];       // FP32-mixed: both state buffers, then p and c of stale ghost layers; or null
+};
+
+// What the first cycle finds: the EOS of the real cells into p, c and g, the CFL minimum of each
+// domain's real cells into its state's accumulators (which must be clear), and a copy of every cell
+// (ghosts included) in the cycles' buffers. One pass over memory and one launch for all domains;
+// `n` domains from `domains`, or the one of `one` when n is 1. `elements`: length of the arrays.
+void launch_begin(const FieldArrays& f, const BatchDomain* domains, int n, const BatchDomain& one, int64_t elements,
+                  DeviceState* states, int eos, double gamma, hipStream_t s);
+
+// What the last cycle leaves, per domain after the cycles its state counts: the final state in rho, u, v
+// and E, and in p, c and g the EOS of the last sweep's input over the real cells. Domains that ran no
+// cycle are left alone.
+void launch_finish(const FieldArrays& f, const BatchDomain* domains, int n, const BatchDomain& one, int64_t elements,
+                   const DeviceState* states, int sweeps_per_cycle, int eos, double gamma, hipStream_t s);
+
+// Element-wise conversion of an FP32 working buffer to a reference FP64 array.
 void launch_convert_f2d(const float* in, double* out, int64_t n, hipStream_t s);
-
-// EOS of a (possibly FP32) state over the real cells into FP64 pmat/cmat/gmat.
-template <class T>
-void launch_eos_real(const T* rho, const T* u, const T* v, const T* E, double* p, double* c, double* g, int eos,
-                     double gamma, int nx, int ny, int row_length, int index_start, hipStream_t s);
 
 }  // namespace armon

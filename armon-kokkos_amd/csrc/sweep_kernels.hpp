@@ -1158,11 +1158,11 @@ __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, T dt, int x0
 // 1.5 us each; a tile has a thread per cell or two. The march is the cheaper per cell (its runs are
 // longer than 24 rows, and nothing passes through LDS) once its waves fill the chip: us per Y sweep,
 // march / tile, FP64 512^2 24.7 / 12.1, 1024^2 35.9 / 27.8, 2048^2 86 / 92; FP32 512^2 16.9 / 10.5,
-// 1024^2 23 / 16.9, 2048^2 40 / 41. `max_cells`: the domains that take tiles.
+// 1024^2 23 / 16.9, 2048^2 40 / 41. `max_cells` (2.6 M, 3.7 M): the domains that take tiles.
 template <class T>
 struct YTile {
-    static constexpr int cols = 16, rows = 32, threads = sizeof(T) == 8 ? 512 : 256;
-    static constexpr int64_t max_cells = sizeof(T) == 8 ? 5 << 19 : 7 << 19;   // 2.6 M, 3.7 M
+    static constexpr int cols = y_tile_cols(), rows = y_tile_rows(), threads = sizeof(T) == 8 ? 512 : 256;
+    static constexpr int64_t max_cells = y_tile_max_cells(sizeof(T));
     static_assert(kFoldedCells <= max_cells, "the march makes no time step");
 };
 
@@ -1207,7 +1207,8 @@ __device__ __forceinline__ SweepArgs<T> batch_domain_args(const BatchArgs<T>& b,
     a.stale_p = b.stale_p + D.offset;
     a.stale_c = b.stale_c + D.offset;
     a.st = b.states + d;
-    a.prev = nullptr;
+    a.prev = b.prev ? b.prev + d : nullptr;
+    if (b.prev) a.step = b.steps[d];
     a.nx = D.nx;
     a.ny = D.ny;
     a.row_length = D.row_length;
@@ -1254,11 +1255,24 @@ __global__ void __launch_bounds__(TILE / CPT) k_batch_x1(BatchArgs<T> b, const B
 {
     __shared__ TileLds<T, TILE, 1> sm;
     const BatchItemX item = items[xcd_block(blockIdx.x, gridDim.x)];
-    const DeviceState* st = b.states + item.domain;
-    if (!st->active) return;
     const SweepArgs<T> a = batch_domain_args(b, item.domain, 0);
-    sweep_x_tile<T, FLUX, PROJ, EOS, kBatchDxMode<T>, TILE, CPT>(a, (T) (st->current_dt * b.dt_factor), item.row,
-                                                                item.slot, sm);
+    double dt;
+    if (!begin_sweep(a, item.row == 0 && item.slot == 0, dt)) return;   // a domain's first tile writes its step
+    sweep_x_tile<T, FLUX, PROJ, EOS, kBatchDxMode<T>, TILE, CPT>(a, (T) (dt * b.dt_factor), item.row, item.slot, sm);
+}
+
+// One block per Y tile.
+template <class T, int FLUX, int PROJ, int EOS>
+__global__ void __launch_bounds__(YTile<T>::threads) k_batch_y_tile(BatchArgs<T> b, const BatchItemY* __restrict__ items)
+{
+    using Y = YTile<T>;
+    __shared__ TileLds<T, Y::cols * Y::rows, Y::cols> sm;
+    const BatchItemY item = items[xcd_block(blockIdx.x, gridDim.x)];
+    const SweepArgs<T> a = batch_domain_args(b, item.domain, 1);
+    double dt;
+    if (!begin_sweep(a, item.x0 == 0 && item.y0 == 0, dt)) return;
+    sweep_y_tile<T, FLUX, PROJ, EOS, kBatchDxMode<T>, Y::cols, Y::rows, Y::threads>(a, (T) (dt * b.dt_factor), item.x0,
+                                                                                    item.y0, sm);
 }
 
 // The row-ahead loads of the FP64 march need 179 VGPRs here (the per-item domain arguments
@@ -1476,7 +1490,8 @@ void launch_batch_x2(const BatchArgs<T>& b, const BatchItemX* items, int nitems,
 }
 
 // X: `tile` cells per tile (128, 256 or 512), `cpt` cells per thread (1; or 2 for tiles of 256
-// or 512 cells, one block per tile); `grid` blocks, or one per tile when grid >= nitems.
+// or 512 cells, one block per tile); `grid` blocks, or one per tile when grid >= nitems. Y: marching
+// runs, or LDS tiles (`tile` 1).
 template <class T, int F, int P, int E>
 void launch_batch_variant(int axis, const BatchArgs<T>& b, const void* items, int nitems, int grid, int tile, int cpt,
                           hipStream_t s)
@@ -1499,6 +1514,11 @@ void launch_batch_variant(int axis, const BatchArgs<T>& b, const void* items, in
         constexpr int R = 2 + (F > 0 ? 1 : 0) + (P == 2 ? 1 : 0);
         const auto* y_items = static_cast<const BatchItemY*>(items);
         const int waves_per_block = kYBlock / 64;
+        if (tile == 1) {
+            k_batch_y_tile<T, F, P, E><<<dim3((unsigned) nitems), dim3(YTile<T>::threads), 0, s>>>(b, y_items);
+            check_launch("batch_y_tile");
+            return;
+        }
         if ((int64_t) grid * waves_per_block >= nitems) {
             const unsigned g1 = (unsigned) ((nitems + waves_per_block - 1) / waves_per_block);
             if (b.stencil_width >= R)
