@@ -54,8 +54,8 @@ inline void boundary_factors(const ArmonParams& p, int side, double* uf, double*
 // allocated on first use and kept until the process ends.
 struct Scratch {
     double* partials = nullptr;       // reduction partials, kPartials entries
-    unsigned long long* min_bits = nullptr;  // min-reduction accumulator (bit pattern of a non-negative double)
-    double* result = nullptr;         // final reduction results (up to 8 doubles)
+    double* result = nullptr;         // final results (up to 8 doubles), in pinned host memory that the
+                                      // device writes: no copy after the reduction
     static constexpr int kPartials = 4 * 1024;
 };
 Scratch& scratch();

@@ -71,12 +71,13 @@ Scratch& scratch()
     Scratch& s = per_device[dev];
     if (!s.partials) {
         void* p = nullptr;
-        size_t bytes = sizeof(double) * Scratch::kPartials + 256 + sizeof(double) * 8;
-        hip_check(hipMalloc(&p, bytes), "hipMalloc(scratch)");
-        char* base = static_cast<char*>(p);
-        s.partials = reinterpret_cast<double*>(base);
-        s.min_bits = reinterpret_cast<unsigned long long*>(base + sizeof(double) * Scratch::kPartials);
-        s.result = reinterpret_cast<double*>(base + sizeof(double) * Scratch::kPartials + 256);
+        void* h = nullptr;
+        hip_check(hipMalloc(&p, sizeof(double) * Scratch::kPartials), "hipMalloc(scratch)");
+        hipError_t e = hipHostMalloc(&h, sizeof(double) * 8, hipHostMallocMapped);
+        if (e != hipSuccess) (void) hipFree(p);
+        hip_check(e, "hipHostMalloc(scratch)");
+        s.partials = static_cast<double*>(p);
+        s.result = static_cast<double*>(h);
     }
     return s;
 }
@@ -195,13 +196,6 @@ __device__ __forceinline__ void for_each_1d(const Iter1D& it, F&& f)
     for (int64_t k = it.start + (int64_t) blockIdx.x * blockDim.x + threadIdx.x; k < it.end;
          k += (int64_t) gridDim.x * blockDim.x)
         f(k, k * it.step + it.base);
-}
-
-dim3 grid_2d(const Iter2D& it)
-{
-    const int64_t rows = it.last_row - it.first_row + 1;
-    const int64_t gx = (it.len + kBlock - 1) / kBlock;
-    return dim3((unsigned) gx, (unsigned) (rows < 65535 ? rows : 65535), 1);
 }
 
 // The grid of for_each_2d: kAlignSlack columns more than the row.
@@ -633,18 +627,28 @@ __global__ void __launch_bounds__(kBlock) k_boundary_conditions(Iter1D it, int64
     });
 }
 
+// Element k of a border's range, for each k once. A border is a few columns of many rows: its
+// elements are dealt to the threads one after the other, whatever the rows' length (a row a block, as
+// the other kernels' grids have it, left 4 threads of 256 with work: 5.5 us for the border of 4099
+// rows, now 2.5).
+template <class F>
+__device__ __forceinline__ void for_each_border(const Iter2D& it, F&& f)
+{
+    const int64_t k = it.start + (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= it.end) return;
+    const int64_t row = k / it.len;
+    f(k, it.base + row * it.step + (k - row * it.len));
+}
+
+dim3 grid_border(const Iter2D& it) { return dim3((unsigned) ((it.end - it.start + kBlock - 1) / kBlock), 1, 1); }
+
 __global__ void __launch_bounds__(kBlock) k_read_border(Iter2D it, int64_t side_length, int64_t nghost,
                                                         const flt_t* __restrict__ rho, const flt_t* __restrict__ umat,
                                                         const flt_t* __restrict__ vmat, const flt_t* __restrict__ pmat,
                                                         const flt_t* __restrict__ cmat, const flt_t* __restrict__ gmat,
                                                         const flt_t* __restrict__ Emat, flt_t* __restrict__ values)
 {
-    const int64_t col = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= it.len) return;
-    for (int64_t row = it.first_row + blockIdx.y; row <= it.last_row; row += gridDim.y) {
-        const int64_t k = row * it.len + col;
-        if (k < it.start || k >= it.end) continue;
-        const int64_t idx = it.base + row * it.step + col;
+    for_each_border(it, [&](int64_t k, int64_t idx) {
         const int64_t a = ((k % nghost) * side_length + k / nghost) * 7;
         values[a + 0] = rho[idx];
         values[a + 1] = umat[idx];
@@ -653,7 +657,7 @@ __global__ void __launch_bounds__(kBlock) k_read_border(Iter2D it, int64_t side_
         values[a + 4] = cmat[idx];
         values[a + 5] = gmat[idx];
         values[a + 6] = Emat[idx];
-    }
+    });
 }
 
 __global__ void __launch_bounds__(kBlock) k_write_border(Iter2D it, int64_t side_length, int64_t nghost,
@@ -662,12 +666,7 @@ __global__ void __launch_bounds__(kBlock) k_write_border(Iter2D it, int64_t side
                                                          flt_t* __restrict__ cmat, flt_t* __restrict__ gmat,
                                                          flt_t* __restrict__ Emat, const flt_t* __restrict__ values)
 {
-    const int64_t col = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= it.len) return;
-    for (int64_t row = it.first_row + blockIdx.y; row <= it.last_row; row += gridDim.y) {
-        const int64_t k = row * it.len + col;
-        if (k < it.start || k >= it.end) continue;
-        const int64_t idx = it.base + row * it.step + col;
+    for_each_border(it, [&](int64_t k, int64_t idx) {
         const int64_t a = ((k % nghost) * side_length + k / nghost) * 7;
         rho[idx] = values[a + 0];
         umat[idx] = values[a + 1];
@@ -676,7 +675,7 @@ __global__ void __launch_bounds__(kBlock) k_write_border(Iter2D it, int64_t side
         cmat[idx] = values[a + 4];
         gmat[idx] = values[a + 5];
         Emat[idx] = values[a + 6];
-    }
+    });
 }
 
 // init_test.cpp:12-48 (states) and test_cases.h:50-116 (regions)
@@ -775,14 +774,15 @@ __device__ __forceinline__ double wave_min(double v)
     return v;
 }
 
-// Min of the CFL bound over the range. The per-thread fold starts from the largest finite
-// value, Kokkos' identity for a Min reduction (so a range where every cell gives +inf
-// returns DBL_MAX, like the reference). The block minima are merged with an integer
-// atomicMin on the bit pattern, which orders non-negative doubles (NaN bounds rank above
-// +inf and never win, as with the reference's comparison-based min).
+// Min of the CFL bound over the range, in two launches: each block's minimum, then (k_dt_final, one
+// block) the least of them, straight to where the caller wants it. The per-thread fold starts from
+// the largest finite value, Kokkos' identity for a Min reduction (so a range where every cell gives
+// +inf returns DBL_MAX, like the reference). The block minima are merged by their bit patterns, which
+// order non-negative doubles (NaN bounds rank above +inf and never win, as with the reference's
+// comparison-based min).
 __global__ void __launch_bounds__(kBlock) k_dt_CFL(Iter1D it, flt_t dx, flt_t dy, const flt_t* __restrict__ umat,
                                                    const flt_t* __restrict__ vmat, const flt_t* __restrict__ cmat,
-                                                   const flt_t* __restrict__ mask, unsigned long long* min_bits)
+                                                   const flt_t* __restrict__ mask, unsigned long long* minima)
 {
     flt_t local = (sizeof(flt_t) == 8) ? flt_t(DBL_MAX) : flt_t(FLT_MAX);
     for_each_1d(it, [&](int64_t, int64_t i) {
@@ -797,69 +797,131 @@ __global__ void __launch_bounds__(kBlock) k_dt_CFL(Iter1D it, flt_t dx, flt_t dy
     if (threadIdx.x == 0) {
         double m = smem[0];
         for (int w = 1; w < kBlock / 64; w++) m = kmin(m, smem[w]);
-        atomicMin(min_bits, (unsigned long long) __double_as_longlong(m));
+        minima[blockIdx.x] = (unsigned long long) __double_as_longlong(m);
     }
 }
 
-__global__ void k_fill_bits(unsigned long long* p, unsigned long long v) { *p = v; }
-
-__global__ void k_bits_to_double(const unsigned long long* bits, double* out)
+__global__ void __launch_bounds__(kBlock) k_dt_final(const unsigned long long* minima, int n, double init, double* out)
 {
-    *out = __longlong_as_double((long long) *bits);
+    __shared__ unsigned long long smem[kBlock];
+    unsigned long long m = (unsigned long long) __double_as_longlong(init);
+    for (int k = threadIdx.x; k < n; k += kBlock) m = minima[k] < m ? minima[k] : m;
+    smem[threadIdx.x] = m;
+    __syncthreads();
+    for (int half = kBlock / 2; half > 0; half /= 2) {
+        if ((int) threadIdx.x < half && smem[threadIdx.x + half] < smem[threadIdx.x])
+            smem[threadIdx.x] = smem[threadIdx.x + half];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *out = __longlong_as_double((long long) smem[0]);
 }
 
-// Compensated (Neumaier) sums of mass and energy; per-block partial (sum, compensation)
-// pairs, combined in a fixed order by k_conservation_final: run-to-run deterministic.
-struct Neumaier {
+// Compensated sums of mass and energy: every addition's rounding error, which two_sum gives exactly, is
+// added up beside the sum. Each thread sums its elements, then wave, block and (k_conservation_final,
+// one block) all blocks merge pairs in a fixed order: run-to-run deterministic.
+struct Compensated {
     double s = 0, c = 0;
     __device__ __forceinline__ void add(double v)
     {
-        double t = s + v;
-        if (abs_t<double>(s) >= abs_t<double>(v)) c += (s - t) + v;
-        else c += (v - t) + s;
+        const double t = s + v;
+        const double b = t - s;
+        c += (s - (t - b)) + (v - b);
         s = t;
+    }
+    __device__ __forceinline__ void merge(double s2, double c2)
+    {
+        add(s2);
+        c += c2;
     }
 };
 
+struct MassEnergy {
+    Compensated m, e;
+    __device__ __forceinline__ void merge(const MassEnergy& o)
+    {
+        m.merge(o.m.s, o.m.c);
+        e.merge(o.e.s, o.e.c);
+    }
+};
+
+// The block's sums, in thread 0.
+__device__ __forceinline__ MassEnergy block_sum(MassEnergy v)
+{
+    for (int off = 32; off > 0; off >>= 1) {
+        MassEnergy o;
+        o.m.s = __shfl_down(v.m.s, off, 64);
+        o.m.c = __shfl_down(v.m.c, off, 64);
+        o.e.s = __shfl_down(v.e.s, off, 64);
+        o.e.c = __shfl_down(v.e.c, off, 64);
+        v.merge(o);
+    }
+    __shared__ double smem[kBlock / 64][4];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if (lane == 0) {
+        smem[wid][0] = v.m.s;
+        smem[wid][1] = v.m.c;
+        smem[wid][2] = v.e.s;
+        smem[wid][3] = v.e.c;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / 64; w++) {
+            v.m.merge(smem[w][0], smem[w][1]);
+            v.e.merge(smem[w][2], smem[w][3]);
+        }
+    }
+    return v;
+}
+
+// Bound by memory (3 words a cell), with 4 elements' loads in flight a thread. At 2049 x 4099: 35-48 us; with
+// one element at a time and thread 0 adding up the block's 1024 numbers, 128 us, and 222 more for
+// one thread to add up those of 1024 blocks.
 __global__ void __launch_bounds__(kBlock) k_conservation_partial(Iter1D it, double ds, const flt_t* __restrict__ rho,
                                                                  const flt_t* __restrict__ Emat,
                                                                  const flt_t* __restrict__ mask, double* partials)
 {
-    Neumaier m, e;
-    for_each_1d(it, [&](int64_t, int64_t i) {
-        double cell_mass = (double) rho[i] * (double) mask[i] * ds;
-        double cell_energy = cell_mass * (double) Emat[i];
-        m.add(cell_mass);
-        e.add(cell_energy);
-    });
-    __shared__ double sm[4][kBlock];
-    sm[0][threadIdx.x] = m.s;
-    sm[1][threadIdx.x] = m.c;
-    sm[2][threadIdx.x] = e.s;
-    sm[3][threadIdx.x] = e.c;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        Neumaier bm, be;
-        for (int t = 0; t < kBlock; t++) {
-            bm.add(sm[0][t]); bm.add(sm[1][t]);
-            be.add(sm[2][t]); be.add(sm[3][t]);
+    constexpr int kAhead = 4;
+    MassEnergy sum;
+    const int64_t stride = (int64_t) gridDim.x * blockDim.x;
+    for (int64_t k = it.start + (int64_t) blockIdx.x * blockDim.x + threadIdx.x; k < it.end; k += kAhead * stride) {
+        double r[kAhead], e[kAhead], w[kAhead];
+#pragma unroll
+        for (int j = 0; j < kAhead; j++) {
+            const bool in = k + j * stride < it.end;
+            const int64_t i = (in ? k + j * stride : k) * it.step + it.base;
+            r[j] = (double) rho[i];
+            e[j] = (double) Emat[i];
+            w[j] = (double) mask[i];
         }
-        partials[4 * blockIdx.x + 0] = bm.s;
-        partials[4 * blockIdx.x + 1] = bm.c;
-        partials[4 * blockIdx.x + 2] = be.s;
-        partials[4 * blockIdx.x + 3] = be.c;
+#pragma unroll
+        for (int j = 0; j < kAhead; j++) {
+            if (k + j * stride >= it.end) break;
+            const double cell_mass = r[j] * w[j] * ds;
+            sum.m.add(cell_mass);
+            sum.e.add(cell_mass * e[j]);
+        }
+    }
+    sum = block_sum(sum);
+    if (threadIdx.x == 0) {
+        partials[4 * blockIdx.x + 0] = sum.m.s;
+        partials[4 * blockIdx.x + 1] = sum.m.c;
+        partials[4 * blockIdx.x + 2] = sum.e.s;
+        partials[4 * blockIdx.x + 3] = sum.e.c;
     }
 }
 
-__global__ void k_conservation_final(int nblocks, const double* partials, double* out)
+__global__ void __launch_bounds__(kBlock) k_conservation_final(int nblocks, const double* partials, double* out)
 {
-    Neumaier m, e;
-    for (int b = 0; b < nblocks; b++) {
-        m.add(partials[4 * b + 0]); m.add(partials[4 * b + 1]);
-        e.add(partials[4 * b + 2]); e.add(partials[4 * b + 3]);
+    MassEnergy sum;
+    for (int b = threadIdx.x; b < nblocks; b += kBlock) {
+        sum.m.merge(partials[4 * b + 0], partials[4 * b + 1]);
+        sum.e.merge(partials[4 * b + 2], partials[4 * b + 3]);
     }
-    out[0] = m.s + m.c;
-    out[1] = e.s + e.c;
+    sum = block_sum(sum);
+    if (threadIdx.x == 0) {
+        out[0] = sum.m.s + sum.m.c;
+        out[1] = sum.e.s + sum.e.c;
+    }
 }
 
 // ---- allocation-free conservation sums ----------------------------------------------------
@@ -1223,7 +1285,7 @@ ARMON_KERNEL_TRY
     check_view(Emat, "Emat", sp);
     check_view(value_array, "value_array", border_values_span(it, side_length, nghost), false);
     if (empty_2d(it)) return;
-    k_read_border<<<grid_2d(it), kBlock, 0, stream()>>>(it, side_length, nghost, rho.data, umat.data, vmat.data,
+    k_read_border<<<grid_border(it), kBlock, 0, stream()>>>(it, side_length, nghost, rho.data, umat.data, vmat.data,
                                                          pmat.data, cmat.data, gmat.data, Emat.data,
                                                          value_array.data);
     after_launch("read_border_array");
@@ -1246,7 +1308,7 @@ ARMON_KERNEL_TRY
     check_view(Emat, "Emat", sp);
     check_view(value_array, "value_array", border_values_span(it, side_length, nghost), false);
     if (empty_2d(it)) return;
-    k_write_border<<<grid_2d(it), kBlock, 0, stream()>>>(it, side_length, nghost, rho.data, umat.data, vmat.data,
+    k_write_border<<<grid_border(it), kBlock, 0, stream()>>>(it, side_length, nghost, rho.data, umat.data, vmat.data,
                                                           pmat.data, cmat.data, gmat.data, Emat.data,
                                                           value_array.data);
     after_launch("write_border_array");
@@ -1359,17 +1421,16 @@ static void launch_dt_CFL(const Range& range, const InnerRange1D& inner_range, f
     check_view(domain_mask, "domain_mask", sp);
     Scratch& sc = armon::scratch();
     const double init = (sizeof(flt_t) == 8) ? DBL_MAX : (double) FLT_MAX;
-    k_fill_bits<<<1, 1, 0, stream()>>>(sc.min_bits, (unsigned long long) __builtin_bit_cast(long long, init));
-    after_launch("dt_CFL(init)");
+    auto* minima = reinterpret_cast<unsigned long long*>(sc.partials);
+    int64_t g = 0;
     if (!empty_1d(it)) {
-        int64_t n = it.end - it.start;
-        int64_t g = (n + kBlock - 1) / kBlock;
+        g = (it.end - it.start + kBlock - 1) / kBlock;
         if (g > kRedBlocks) g = kRedBlocks;
         k_dt_CFL<<<(unsigned) g, kBlock, 0, stream()>>>(it, dx, dy, umat.data, vmat.data, cmat.data, domain_mask.data,
-                                                         sc.min_bits);
+                                                         minima);
         after_launch("dt_CFL");
     }
-    k_bits_to_double<<<1, 1, 0, stream()>>>(sc.min_bits, dt_device);
+    k_dt_final<<<1, kBlock, 0, stream()>>>(minima, (int) g, init, dt_device);
     after_launch("dt_CFL(result)");
 }
 
@@ -1379,10 +1440,8 @@ ARMON_EXPORT flt_t dt_CFL(const Range& range, const InnerRange1D& inner_range, f
     try {
         Scratch& sc = armon::scratch();
         launch_dt_CFL(range, inner_range, dx, dy, umat, vmat, cmat, domain_mask, sc.result);
-        double out = 0;
-        hip_check(hipMemcpyAsync(&out, sc.result, sizeof(double), hipMemcpyDeviceToHost, stream()), "dt_CFL copy");
         hip_check(hipStreamSynchronize(stream()), "dt_CFL sync");
-        return (flt_t) out;
+        return (flt_t) *sc.result;
     }
     catch (const armon::Error& err) { armon::report("dt_CFL", err); }
     catch (const std::exception& err) { armon::report_std("dt_CFL", err); }
@@ -1400,10 +1459,12 @@ ARMON_KERNEL_TRY
 ARMON_KERNEL_CATCH("dt_CFL_device")
 
 // The compensated sums over `range` with `max_blocks` blocks of partials at `partials` and the
-// two results at `result` (device memory), returned to the host.
+// two results at `result` (memory that the device writes, and the host reads if `host_result`),
+// returned to the host.
 static void run_conservation(const char* name, const Range& range, const InnerRange1D& inner_range, flt_t dx,
                              const view& rho, const view& Emat, const mask_view& domain_mask, double* partials,
-                             int max_blocks, double* result, flt_t& total_mass, flt_t& total_energy)
+                             int max_blocks, double* result, bool host_result, flt_t& total_mass,
+                             flt_t& total_energy)
 {
     const Iter1D it = make_iter1d(range, inner_range);
     const Span sp = span_of(it);
@@ -1421,11 +1482,16 @@ static void run_conservation(const char* name, const Range& range, const InnerRa
     k_conservation_partial<<<(unsigned) g, kBlock, 0, stream()>>>(it, ds, rho.data, Emat.data, domain_mask.data,
                                                                    partials);
     after_launch(name);
-    k_conservation_final<<<1, 1, 0, stream()>>>((int) g, partials, result);
+    k_conservation_final<<<1, kBlock, 0, stream()>>>((int) g, partials, result);
     after_launch(name);
     double out[2];
-    hip_check(hipMemcpyAsync(out, result, sizeof out, hipMemcpyDeviceToHost, stream()), "conservation copy");
+    if (!host_result)
+        hip_check(hipMemcpyAsync(out, result, sizeof out, hipMemcpyDeviceToHost, stream()), "conservation copy");
     hip_check(hipStreamSynchronize(stream()), "conservation sync");
+    if (host_result) {
+        out[0] = result[0];
+        out[1] = result[1];
+    }
     total_mass = (flt_t) out[0];
     total_energy = (flt_t) out[1];
 }
@@ -1437,7 +1503,7 @@ ARMON_KERNEL_TRY
 {
     Scratch& sc = armon::scratch();
     run_conservation("conservation_vars", range, inner_range, dx, rho, Emat, domain_mask, sc.partials,
-                     Scratch::kPartials / 4, sc.result, total_mass, total_energy);
+                     Scratch::kPartials / 4, sc.result, true, total_mass, total_energy);
 }
 ARMON_KERNEL_CATCH("conservation_vars")
 
@@ -1452,7 +1518,7 @@ ARMON_KERNEL_TRY
 {
     double* base = noalloc_scratch();
     run_conservation("conservation_vars_noalloc", range, inner_range, dx, rho, Emat, domain_mask, base,
-                     kNoAllocBlocks, base + 4 * kNoAllocBlocks, total_mass, total_energy);
+                     kNoAllocBlocks, base + 4 * kNoAllocBlocks, false, total_mass, total_energy);
 }
 ARMON_KERNEL_CATCH("conservation_vars_noalloc")
 
