@@ -113,7 +113,7 @@ struct BatchArgs {
 };
 
 // One launch sweeps every domain of the batch along `axis`: `grid` persistent blocks walk
-// the work items (BatchItemX for X, BatchItemY for Y); X tiles are `tile` cells wide (128,
+// the work items (BatchItemX for X, BatchItemY for Y; with `b.prev` one block each, whatever `grid`); X tiles are `tile` cells wide (128,
 // 256 or 512, the width the X items were cut for), `cpt` cells per thread (1, or 2 for tiles of
 // 256 or 512 cells, one block per tile whatever `grid`). Y items are marching runs (`tile` 0) or LDS
 // tiles (`tile` 1: y_tile_cols() x y_tile_outputs() cells, one block per tile).
