@@ -213,7 +213,18 @@ template <> ARMON_HD double sqrt_t<double>(double x)
 #endif
     return __builtin_sqrt(x);
 }
-template <> ARMON_HD float sqrt_t<float>(float x) { return __builtin_sqrtf(x); }
+template <> ARMON_HD float sqrt_t<float>(float x)
+{
+#if defined(ARMON_FAST_FP32) && defined(__HIP_DEVICE_COMPILE__)
+    // The FP32-mixed form's square root, written out: the compiler makes the native one (1 ulp, with a
+    // subnormal operand scaled) of __builtin_sqrtf in some kernels and the correctly rounded one in
+    // others, and a cell's result must not depend on the kernel it is computed in.
+    const bool small = x < 0x1p-126f;
+    return __builtin_ldexpf(__builtin_amdgcn_sqrtf(__builtin_ldexpf(x, small ? 32 : 0)), small ? -16 : 0);
+#else
+    return __builtin_sqrtf(x);
+#endif
+}
 
 template <class T> ARMON_HD T copysign_t(T a, T b);
 template <> ARMON_HD double copysign_t<double>(double a, double b) { return __builtin_copysign(a, b); }
@@ -497,6 +508,42 @@ template <class T> __device__ __forceinline__ void perfect_gas_pc(T gamma, T rho
     } else {
         (void) y;
         c = sqrt_t<T>(dv<T>(gamma * p, rho));
+    }
+}
+
+// bizarrium without g, with y = shared_recip(rho): the quotients by rho and by 1 - s x go through two
+// shared reciprocals, the one by the constant rho0 through its own (div_by_recip); 5 divisions fewer.
+// Each f is part of the next, so a NaN from any of them reaches f3.
+__device__ __forceinline__ void bizarrium_pc(double rho, double E, double u, double v, double y, double& p, double& c)
+{
+    const double rho0 = 1e4, K0 = 1e11, Cv0 = 1e3, T0 = 300, eps0 = 0;
+    const double G0 = 1.5, s = 1.5, q = -42080895. / 14941154., r = 727668333. / 149411540.;
+
+    double x = div_by_recip(rho, rho0, 1.0 / rho0) - 1;
+    double g = G0 * (1 - refined_quot(rho0, rho, y));
+
+    const double d = 1 - s * x, yd = shared_recip<double>(d);
+    const double n0 = 1 + (s / 3 - 2) * x + q * (x * x) + r * (x * x * x);
+    const double f0 = refined_quot(n0, d, yd);
+    const double n1 = s / 3 - 2 + 2 * q * x + 3 * r * (x * x) + s * f0;
+    const double f1 = refined_quot(n1, d, yd);
+    const double n2 = 2 * q + 6 * r * x + 2 * s * f1;
+    const double f2 = refined_quot(n2, d, yd);
+
+    double eps_k0 = eps0 - Cv0 * T0 * (1 + g) + 0.5 * (K0 / rho0) * (x * x) * f0;
+    double pk0 = -Cv0 * T0 * G0 * rho0 + (0.5 * K0 * x * (1 + x) * (1 + x) * (2 * f0 + x * f1));
+    double pk0prime = -0.5 * K0 * cr_pow3(1 + x)
+            * rho0 * (2 * (1 + 3 * x) * f0 + 2 * x * (2 + 3 * x) * f1 + (x * x) * (1 + x) * f2);
+
+    double e = E - 0.5 * (u * u + v * v);
+    p = pk0 + G0 * rho0 * (e - eps_k0);
+    const double square = G0 * rho0 * (p - pk0) - pk0prime;
+    c = refined_quot(sqrt_core(square), rho, y);
+    const int bad = unusable(y) | unusable(f2) | too_small(n0) | too_small(n1) | too_small(n2) |
+                    (int) !((int) (square >= 0x1p-700) & (int) (square < __builtin_huge_val()));
+    if (__builtin_expect(bad, 0)) {
+        double g_out;
+        bizarrium(rho, E, u, v, p, c, g_out);
     }
 }
 

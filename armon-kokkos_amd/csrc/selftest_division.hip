@@ -166,7 +166,7 @@ __device__ bool same(double a, double b) { return to_bits(a) == to_bits(b) || (!
 
 // The fused sweeps' form of each stage against the plain one (godunov, gad_correct with every
 // limiter, the two divisions of cell_update, advection_flux_2 for both donors, projection in both
-// ways of dividing by dx, perfect_gas). counts[0]: results that differ; counts[1]: samples whose
+// ways of dividing by dx, both equations of state). counts[0]: results that differ; counts[1]: samples whose
 // shared reciprocals all served; first[0]: the index of a differing sample, first[1]: the stages.
 __global__ void __launch_bounds__(256) k_check_stages(uint64_t seed, int64_t n, unsigned long long* counts,
                                                        double* first, int* first_taken)
@@ -222,6 +222,12 @@ __global__ void __launch_bounds__(256) k_check_stages(uint64_t seed, int64_t n, 
             perfect_gas<double>(1.4, rho[0], E[0], u[0], v[0], p0, c0, g0);
             perfect_gas_pc<double>(1.4, rho[0], E[0], u[0], v[0], y, p1, c1);
             wrong |= (same(p0, p1) && same(c0, c1) ? 0 : 16);
+            // Bizarrium's densities lie about 1e4
+            const double heavy = (splitmix64(s) & 7) ? 1e4 * with_exponent(s, 0, false) : rho[1];
+            const double eh = (splitmix64(s) & 3) ? 1e6 * with_exponent(s, 0, false) : E[1];
+            bizarrium(heavy, eh, u[1], v[1], p0, c0, g0);
+            bizarrium_pc(heavy, eh, u[1], v[1], shared_recip<double>(heavy), p1, c1);
+            wrong |= (same(p0, p1) && same(c0, c1) ? 0 : 128);
         }
         {   // advection from the donor 1 with neighbours 0 and 2; its faces carry us[1] and us[2]
             double L[3], yS[4], q[3][4];
@@ -338,7 +344,7 @@ extern "C" __attribute__((visibility("default"))) int armon_selftest_sqrt(uint64
 // Checks n samples of the sweeps' stages drawn from seed. mismatches: samples with a result whose
 // bits differ from the plain form's; shared: samples whose shared reciprocals served; first_bad: the
 // index of one differing sample and the stages that differ (1 Godunov, 2 GAD, 4 dt / dm, 8 dm / L,
-// 16 EOS, 32 advection, 64 projection). Returns 0, or the HIP error code.
+// 16 EOS, 32 advection, 64 projection, 128 Bizarrium's EOS). Returns 0, or the HIP error code.
 extern "C" __attribute__((visibility("default"))) int armon_selftest_stages(uint64_t seed, int64_t n,
                                                                             uint64_t* mismatches, uint64_t* shared,
                                                                             double* first_bad)

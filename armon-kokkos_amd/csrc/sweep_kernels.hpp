@@ -99,59 +99,81 @@ __device__ __forceinline__ void cell_eos(double gamma, T rho, T u, T v, T E, T y
     if constexpr (EOS == 0) {
         perfect_gas_pc<T>((T) gamma, rho, E, u, v, y, p, c);
     } else {
-        double pd, cd, gd;
-        bizarrium((double) rho, (double) E, (double) u, (double) v, pd, cd, gd);
+        double pd, cd;
+        const double yd = sizeof(T) == 8 ? (double) y : shared_recip<double>((double) rho);
+        bizarrium_pc((double) rho, (double) E, (double) u, (double) v, yd, pd, cd);
         p = (T) pd;
         c = (T) cd;
     }
 }
 
+// A tile's cell in two parts: its loads (fetch_cell), which depend on nothing but the launch, and the
+// cell from them (make_cell). The tiles' kernels issue the loads before they wait for the cycle's
+// time step, so that the two latencies overlap: a block of a small sweep spends as long on them as
+// on its arithmetic.
+template <class T>
+struct LoadedCell {
+    T rho, u, v, E;
+    unsigned offset;   // bytes past the base
+    int mirror;        // 0 real, 1 low side, 2 high side
+    bool stale;
+};
+
 // Cell `k` (along the sweep axis, `n` real cells) of the pencil whose cell 0 lies `first` elements
 // past `base` (the same for the whole wave) and whose cells lie `stride` apart. Real cells are
-// loaded; ghost layers 1..stencil_width mirror real cells: the real cell's rho, E, p and c, its
-// velocities times the side's factors; deeper ghost layers are read as they are, with p and c from
-// stale_p/stale_c.
-template <class T, int AXIS, int EOS>
-__device__ __forceinline__ Cell<T> load_cell(const SweepArgs<T>& a, int64_t base, int first, int k, int stride, int n)
+// loaded; ghost layers 1..stencil_width mirror real cells; deeper ghost layers are read as they are.
+template <class T>
+__device__ __forceinline__ LoadedCell<T> fetch_cell(const SweepArgs<T>& a, int64_t base, int first, int k, int stride,
+                                                    int n)
 {
+    LoadedCell<T> l;
     int kk = k;
-    int mirror = 0;   // 0 real, 1 low side, 2 high side
-    bool stale = false;
+    l.mirror = 0;
+    l.stale = false;
     if (__builtin_expect((unsigned) k >= (unsigned) n, 0)) {
         if (k < 0) {
-            if (-k <= a.stencil_width) { kk = -k - 1; mirror = 1; }
-            else stale = true;
+            if (-k <= a.stencil_width) { kk = -k - 1; l.mirror = 1; }
+            else l.stale = true;
         } else {
-            if (k - n + 1 <= a.stencil_width) { kk = 2 * n - 1 - k; mirror = 2; }
-            else stale = true;
+            if (k - n + 1 <= a.stencil_width) { kk = 2 * n - 1 - k; l.mirror = 2; }
+            else l.stale = true;
         }
     }
-    const unsigned o = (unsigned) (first + kk * stride) * (unsigned) sizeof(T);
-    T rho = load_at(a.in_rho + base, o), u = load_at(a.in_u + base, o), v = load_at(a.in_v + base, o),
-      E = load_at(a.in_E + base, o);
+    l.offset = (unsigned) (first + kk * stride) * (unsigned) sizeof(T);
+    l.rho = load_at(a.in_rho + base, l.offset);
+    l.u = load_at(a.in_u + base, l.offset);
+    l.v = load_at(a.in_v + base, l.offset);
+    l.E = load_at(a.in_E + base, l.offset);
+    return l;
+}
+
+// A mirror ghost has the real cell's rho and E, its p and c too (halo_exchange.cpp:23-30: the EOS of the
+// unscaled state) and its velocities times the side's factors; a stale one p and c from
+// stale_p/stale_c.
+template <class T, int AXIS, int EOS>
+__device__ __forceinline__ Cell<T> make_cell(const SweepArgs<T>& a, int64_t base, const LoadedCell<T>& l)
+{
     Cell<T> cell;
-    cell.y = shared_recip<T>(rho);
-    // a mirror ghost takes the p and c of its real cell (halo_exchange.cpp:23-30): the EOS of the
-    // unscaled state
-    cell_eos<T, EOS>(a.gamma, rho, u, v, E, cell.y, cell.p, cell.c);
-    if (__builtin_expect(stale | (mirror != 0), 0)) {
-        if (stale) {
-            cell.p = load_at(a.stale_p + base, o);
-            cell.c = load_at(a.stale_c + base, o);
+    T u = l.u, v = l.v;
+    cell.y = shared_recip<T>(l.rho);
+    cell_eos<T, EOS>(a.gamma, l.rho, u, v, l.E, cell.y, cell.p, cell.c);
+    if (__builtin_expect(l.stale | (l.mirror != 0), 0)) {
+        if (l.stale) {
+            cell.p = load_at(a.stale_p + base, l.offset);
+            cell.c = load_at(a.stale_c + base, l.offset);
         } else {
-            u = u * (T) (mirror == 1 ? a.lo_u : a.hi_u);
-            v = v * (T) (mirror == 1 ? a.lo_v : a.hi_v);
+            u = u * (T) (l.mirror == 1 ? a.lo_u : a.hi_u);
+            v = v * (T) (l.mirror == 1 ? a.lo_v : a.hi_v);
         }
     }
-    cell.rho = rho;
-    cell.E = E;
+    cell.rho = l.rho;
+    cell.E = l.E;
     cell.un = AXIS == 0 ? u : v;
     cell.ut = AXIS == 0 ? v : u;
     return cell;
 }
 
-// load_cell in two parts, for the Y march, which loads a row's state one row before it makes the
-// cell: where row `k` comes from (the same for the whole wave: the row it is read at, the mirror side
+// The Y march loads a row's state one row before it makes the cell: where row `k` comes from (the same for the whole wave: the row it is read at, the mirror side
 // or staleness), then the cell from the loaded state.
 struct RowSource {
     int row;
@@ -192,7 +214,7 @@ __device__ __forceinline__ Cell<T> make_row_cell(const SweepArgs<T>& a, const Ro
         cell.p = load_at(a.stale_p + row_start(a, s.row), column);
         cell.c = load_at(a.stale_c + row_start(a, s.row), column);
     } else {
-        cell_eos<T, EOS>(a.gamma, rho, u, v, E, cell.y, cell.p, cell.c);   // unscaled, as load_cell
+        cell_eos<T, EOS>(a.gamma, rho, u, v, E, cell.y, cell.p, cell.c);   // unscaled, as make_cell
     }
     if (s.mirror == 1) {
         u = u * (T) a.lo_u;
@@ -647,8 +669,8 @@ __device__ __forceinline__ void tile_sweep(T dx, T inv_dx, T dt, TileLds<T, CELL
     }
 }
 
-// One X tile of the domain described by `a`, with the cycle's dt. Called by all TILE / CPT
-// threads of a block; each thread computes CPT cells of the tile, at slots t, t + TILE / CPT, ...
+// One X tile of the domain described by `a`; `begin(dt)` gives the cycle's dt, or false where the cycle
+// does not run (the same for the whole block). Called by all TILE / CPT threads of a block; each thread computes CPT cells of the tile, at slots t, t + TILE / CPT, ...
 // (consecutive lanes on consecutive slots for every load and store).
 //
 // The rows of the domain are laid end to end as a stream of slots, each row taking
@@ -657,8 +679,9 @@ __device__ __forceinline__ void tile_sweep(T dx, T inv_dx, T dt, TileLds<T, CELL
 // slots, and the slots [R, TILE - R) of a tile that hold real cells are its outputs. A cell's
 // result depends only on the cells within R of it in its own row, so a tile may span the end
 // of one row and the start of the next; no thread is spent on a tile's share of a row end.
-template <class T, int FLUX, int PROJ, int EOS, int DXM, int TILE = kTile, int CPT = 1>
-__device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, T dt, int j0, int k0, TileLds<T, TILE, 1>& sm)
+template <class T, int FLUX, int PROJ, int EOS, int DXM, int TILE = kTile, int CPT = 1, class Begin>
+__device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, Begin&& begin, int j0, int k0,
+                                             TileLds<T, TILE, 1>& sm)
 {
     constexpr int R = 2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0);
     constexpr int NT = TILE / CPT;
@@ -666,6 +689,7 @@ __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, T dt, int j0
 
     int slot[CPT], jc[CPT], kc[CPT];
     bool in_range[CPT];
+    LoadedCell<T> loaded[CPT];
     Cell<T> cell[CPT];
     // Row jc and cell kc (-R <= kc < nx + R) of each slot: n = k0 + t < x_slots + TILE. Rows of
     // at least TILE slots: n < 2 x_slots. Shorter rows: the float quotient is within one of the
@@ -699,9 +723,14 @@ __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, T dt, int j0
     for (int c = 0; c < CPT; c++) {
         slot[c] = threadIdx.x + c * NT;
         in_range[c] = jc[c] < rows_left;       // false for slots past the last row
-        cell[c] = in_range[c] ? load_cell<T, 0, EOS>(a, base, jc[c] * a.row_length + R, kc[c], 1, a.nx)
-                              : benign_cell<T>();
+        if (in_range[c]) loaded[c] = fetch_cell<T>(a, base, jc[c] * a.row_length + R, kc[c], 1, a.nx);
     }
+    double cycle_dt;
+    if (!begin(cycle_dt)) return;
+    const T dt = (T) (cycle_dt * a.dt_factor);
+#pragma unroll
+    for (int c = 0; c < CPT; c++)
+        cell[c] = in_range[c] ? make_cell<T, 0, EOS>(a, base, loaded[c]) : benign_cell<T>();
     tile_sweep<T, FLUX, PROJ, DXM, TILE, 1, CPT>((T) a.dx, (T) a.inv_dx, dt, sm, slot, cell);
 
     CflSpeeds speeds;
@@ -739,13 +768,11 @@ __global__ void __launch_bounds__(XTile<T>::cells / XTile<T>::cpt) __attribute__
 {
     constexpr int TILE = XTile<T>::cells;
     constexpr int W = TILE - 2 * (2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0));
-    double cycle_dt;
-    if (!begin_sweep<FOLD>(a, blockIdx.x == 0, cycle_dt)) return;
-    const T dt = (T) (cycle_dt * a.dt_factor);
     __shared__ TileLds<T, TILE, 1> sm;
     const int s0 = xcd_block(blockIdx.x, gridDim.x) * W;   // first slot of the tile
     const int j0 = s0 / a.x_slots;
-    sweep_x_tile<T, FLUX, PROJ, EOS, DXM, TILE, XTile<T>::cpt>(a, dt, j0, s0 - j0 * a.x_slots, sm);
+    sweep_x_tile<T, FLUX, PROJ, EOS, DXM, TILE, XTile<T>::cpt>(
+            a, [&](double& dt) { return begin_sweep<FOLD>(a, blockIdx.x == 0, dt); }, j0, s0 - j0 * a.x_slots, sm);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1111,10 +1138,10 @@ __global__ void __launch_bounds__(kYBlock) ARMON_Y_OCCUPANCY k_sweep_y(SweepArgs
 // ---------------------------------------------------------------------------------------
 
 // One Y tile: the columns [x0, x0 + COLS) and the output rows [y0, y0 + ROWS - 2R) of the domain
-// described by `a`, through the stages of tile_sweep with neighbours a tile row apart. Called by NT
-// threads, each with COLS ROWS / NT cells of one column.
-template <class T, int FLUX, int PROJ, int EOS, int DXM, int COLS, int ROWS, int NT>
-__device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, T dt, int x0, int y0,
+// described by `a` (`begin` as for sweep_x_tile), through the stages of tile_sweep with neighbours a tile
+// row apart. Called by NT threads, each with COLS ROWS / NT cells of one column.
+template <class T, int FLUX, int PROJ, int EOS, int DXM, int COLS, int ROWS, int NT, class Begin>
+__device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, Begin&& begin, int x0, int y0,
                                              TileLds<T, COLS * ROWS, COLS>& sm)
 {
     constexpr int R = 2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0);
@@ -1125,6 +1152,7 @@ __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, T dt, int x0
     const int64_t base = (int64_t) a.index_start + (int64_t) (y0 - R) * a.row_length + x0;
     int slot[CPT], row[CPT];
     bool in_range[CPT];
+    LoadedCell<T> loaded[CPT];
     Cell<T> cell[CPT];
 #pragma unroll
     for (int c = 0; c < CPT; c++) {
@@ -1132,9 +1160,15 @@ __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, T dt, int x0
         row[c] = threadIdx.x / COLS + c * (NT / COLS);
         const int k = y0 - R + row[c];
         in_range[c] = x < a.nx && k < a.ny + R;
-        cell[c] = in_range[c] ? load_cell<T, 1, EOS>(a, base, col + (R - y0) * a.row_length, k, a.row_length, a.ny)
-                              : benign_cell<T>();
+        if (in_range[c])
+            loaded[c] = fetch_cell<T>(a, base, col + (R - y0) * a.row_length, k, a.row_length, a.ny);
     }
+    double cycle_dt;
+    if (!begin(cycle_dt)) return;
+    const T dt = (T) (cycle_dt * a.dt_factor);
+#pragma unroll
+    for (int c = 0; c < CPT; c++)
+        cell[c] = in_range[c] ? make_cell<T, 1, EOS>(a, base, loaded[c]) : benign_cell<T>();
     tile_sweep<T, FLUX, PROJ, DXM, COLS * ROWS, COLS, CPT>((T) a.dx, (T) a.inv_dx, dt, sm, slot, cell);
     CflSpeeds speeds;
 #pragma unroll
@@ -1172,16 +1206,14 @@ struct YTile {
 template <class T, int FLUX, int PROJ, int EOS, int DXM, bool FOLD>
 __global__ void __launch_bounds__(YTile<T>::threads) k_sweep_y_tile(SweepArgs<T> a, int ncolblk)
 {
-    double cycle_dt;
-    if (!begin_sweep<FOLD>(a, blockIdx.x == 0, cycle_dt)) return;
     using Y = YTile<T>;
     constexpr int W = Y::rows - 2 * (2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0));
-    const T dt = (T) (cycle_dt * a.dt_factor);
     __shared__ TileLds<T, Y::cols * Y::rows, Y::cols> sm;
     const int bid = xcd_block(blockIdx.x, gridDim.x);
     const int band = bid / ncolblk;
-    sweep_y_tile<T, FLUX, PROJ, EOS, DXM, Y::cols, Y::rows, Y::threads>(a, dt, (bid - band * ncolblk) * Y::cols,
-                                                                        band * W, sm);
+    sweep_y_tile<T, FLUX, PROJ, EOS, DXM, Y::cols, Y::rows, Y::threads>(
+            a, [&](double& dt) { return begin_sweep<FOLD>(a, blockIdx.x == 0, dt); }, (bid - band * ncolblk) * Y::cols,
+            band * W, sm);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1246,8 +1278,8 @@ __global__ void __launch_bounds__(TILE) k_batch_x(BatchArgs<T> b, const BatchIte
         const DeviceState* st = b.states + item.domain;
         if (!st->active) continue;   // the same for the whole block
         const SweepArgs<T> a = batch_domain_args(b, item.domain, 0);
-        sweep_x_tile<T, FLUX, PROJ, EOS, kBatchDxMode<T>, TILE>(a, (T) (st->current_dt * b.dt_factor), item.row,
-                                                               item.slot, sm);
+        sweep_x_tile<T, FLUX, PROJ, EOS, kBatchDxMode<T>, TILE>(
+                a, [&](double& dt) { dt = st->current_dt; return true; }, item.row, item.slot, sm);
         __syncthreads();             // the next item reuses the LDS
     }
 }
@@ -1261,9 +1293,10 @@ __global__ void __launch_bounds__(TILE / CPT) k_batch_x1(BatchArgs<T> b, const B
     __shared__ TileLds<T, TILE, 1> sm;
     const BatchItemX item = items[xcd_block(blockIdx.x, gridDim.x)];
     const SweepArgs<T> a = batch_domain_args<FOLD>(b, item.domain, 0);
-    double dt;
-    if (!begin_sweep<FOLD>(a, item.row == 0 && item.slot == 0, dt)) return;   // a domain's first tile writes its step
-    sweep_x_tile<T, FLUX, PROJ, EOS, kBatchDxMode<T>, TILE, CPT>(a, (T) (dt * b.dt_factor), item.row, item.slot, sm);
+    // a domain's first tile writes its step
+    sweep_x_tile<T, FLUX, PROJ, EOS, kBatchDxMode<T>, TILE, CPT>(
+            a, [&](double& dt) { return begin_sweep<FOLD>(a, item.row == 0 && item.slot == 0, dt); }, item.row,
+            item.slot, sm);
 }
 
 // One block per Y tile.
@@ -1274,10 +1307,8 @@ __global__ void __launch_bounds__(YTile<T>::threads) k_batch_y_tile(BatchArgs<T>
     __shared__ TileLds<T, Y::cols * Y::rows, Y::cols> sm;
     const BatchItemY item = items[xcd_block(blockIdx.x, gridDim.x)];
     const SweepArgs<T> a = batch_domain_args<FOLD>(b, item.domain, 1);
-    double dt;
-    if (!begin_sweep<FOLD>(a, item.x0 == 0 && item.y0 == 0, dt)) return;
-    sweep_y_tile<T, FLUX, PROJ, EOS, kBatchDxMode<T>, Y::cols, Y::rows, Y::threads>(a, (T) (dt * b.dt_factor), item.x0,
-                                                                                    item.y0, sm);
+    sweep_y_tile<T, FLUX, PROJ, EOS, kBatchDxMode<T>, Y::cols, Y::rows, Y::threads>(
+            a, [&](double& dt) { return begin_sweep<FOLD>(a, item.x0 == 0 && item.y0 == 0, dt); }, item.x0, item.y0, sm);
 }
 
 // The row-ahead loads of the FP64 march need 179 VGPRs here (the per-item domain arguments

@@ -81,3 +81,24 @@ def test_batch_tiles_are_its_marches(armon, precision, splitting, rows):
         assert (ca, da) == (cb, db)
         for x, y in zip(fa, fb):
             assert np.array_equal(x, y)
+
+
+# one domain through the batch's X tiles of every shape and through the single-domain sweeps: FP32's
+# arithmetic is the same in every kernel
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,cells_per_thread", [(128, 1), (256, 1), (512, 1), (256, 2), (512, 2)])
+@pytest.mark.parametrize("test,nx,ny", [("Sod", 152, 98), ("Sod_circ", 256, 256)])
+def test_fp32_batch_is_the_single_domain(armon, test, nx, ny, tile, cells_per_thread):
+    kw = dict(max_cycles=6, precision=armon.PREC_FP32_MIXED, cfl=0.7, **GAD2)
+    a, ca, da = _run(armon, test, nx=nx, ny=ny, **kw)
+    spec = armon.ArmonDomainSpec(test=armon.TESTS[test], nx=nx, ny=ny, state=armon.reference_state(test))
+    b = armon.Batch(armon.batch_params(verbose=5, **kw), [spec])
+    b.set_tuning(16, tile_x=tile, x_cells_per_thread=cells_per_thread)
+    b.init()
+    b.begin()
+    b.run()
+    assert b.finish() == 0, armon.errors()
+    assert (b.result(0).cycles, b.result(0).final_dt) == (ca, da)
+    for f in FIELDS:
+        assert np.array_equal(b.read(0, f), a[f]), f
+    b.close()
