@@ -410,16 +410,17 @@ struct alignas(16) Quad {
     T x, y, z, w;
 };
 
-template <class T, int CELLS, int S>
+// GAD, E2: whether the scheme has those stages (without either, b and c are not there: 64 bytes, 8 blocks).
+template <class T, int CELLS, int S, bool GAD, bool E2>
 struct TileLds;
 
-template <int CELLS, int S>
-struct TileLds<double, CELLS, S> {
+template <int CELLS, int S, bool GAD, bool E2>
+struct TileLds<double, CELLS, S, GAD, E2> {
     static constexpr int N = CELLS + 3 * S;
     static constexpr bool kFluxBarrier = false;
     using P = Pair<double>;
-    P a0_[N], a1_[N], b_[N], w_[N], f_[N];
-    double c_[N];
+    P a0_[N], a1_[N], b_[GAD || E2 ? N : 1], w_[N], f_[N];
+    double c_[E2 ? N : 1];
     __device__ __forceinline__ P& a0(int t) { return a0_[t + 2 * S]; }
     __device__ __forceinline__ P& a1(int t) { return a1_[t + 2 * S]; }
     __device__ __forceinline__ P& w(int t) { return w_[t + 2 * S]; }
@@ -481,13 +482,13 @@ struct TileLds<double, CELLS, S> {
     }
 };
 
-template <int CELLS, int S>
-struct TileLds<float, CELLS, S> {
+template <int CELLS, int S, bool GAD, bool E2>
+struct TileLds<float, CELLS, S, GAD, E2> {
     static constexpr int N = CELLS + 3 * S;
     using P = Pair<float>;
     using Q = Quad<float>;
     static constexpr bool kFluxBarrier = true;
-    Q a_[N], b_[N];   // a: the state, what the slopes read, then the fluxes; b: Godunov's A and B, then the lengths
+    Q a_[N], b_[GAD || E2 ? N : 1];   // a: the state, what the slopes read, then the fluxes; b: Godunov's A and B, then the lengths
     P w_[N];
     __device__ __forceinline__ void put_differences(int t, P A, P B) { b_[t + 2 * S] = {A.x, A.y, B.x, B.y}; }
     __device__ __forceinline__ P get_A(int t)
@@ -542,6 +543,9 @@ struct TileLds<float, CELLS, S> {
     }
 };
 
+template <class T, int FLUX, int PROJ, int CELLS, int S>
+using SchemeLds = TileLds<T, CELLS, S, (FLUX > 0), PROJ == 2>;
+
 // The whole per-axis chain of one tile, from the loaded cells (EOS done) to the projected ones:
 // thread t computes the slots slot[0..CPT), and cell[] holds their new rho, un, ut, E afterwards
 // (c stays the input state's). Every thread of the block calls it; outputs are right for the slots
@@ -554,7 +558,7 @@ struct TileLds<float, CELLS, S> {
 // length computed more than twice). The arithmetic of each result is the reference's, so FP64 keeps
 // the bits of dividing everywhere; operands outside shared_recip's ranges take the divisions.
 template <class T, int FLUX, int PROJ, int DXM, int CELLS, int S, int CPT>
-__device__ __forceinline__ void tile_sweep(T dx, T inv_dx, T dt, TileLds<T, CELLS, S>& sm, const int (&slot)[CPT],
+__device__ __forceinline__ void tile_sweep(T dx, T inv_dx, T dt, SchemeLds<T, FLUX, PROJ, CELLS, S>& sm, const int (&slot)[CPT],
                                            Cell<T> (&cell)[CPT])
 {
     constexpr bool GAD = FLUX > 0;
@@ -655,7 +659,7 @@ __device__ __forceinline__ void tile_sweep(T dx, T inv_dx, T dt, TileLds<T, CELL
             donor_flux_1<T>(disp, q, f[k]);
         }
     }
-    if constexpr (TileLds<T, CELLS, S>::kFluxBarrier) __syncthreads();
+    if constexpr (SchemeLds<T, FLUX, PROJ, CELLS, S>::kFluxBarrier) __syncthreads();
 #pragma unroll
     for (int k = 0; k < CPT; k++) sm.put_flux(slot[k], f[k]);
     __syncthreads();
@@ -681,7 +685,7 @@ __device__ __forceinline__ void tile_sweep(T dx, T inv_dx, T dt, TileLds<T, CELL
 // of one row and the start of the next; no thread is spent on a tile's share of a row end.
 template <class T, int FLUX, int PROJ, int EOS, int DXM, int TILE = kTile, int CPT = 1, class Begin>
 __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, Begin&& begin, int j0, int k0,
-                                             TileLds<T, TILE, 1>& sm)
+                                             SchemeLds<T, FLUX, PROJ, TILE, 1>& sm)
 {
     constexpr int R = 2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0);
     constexpr int NT = TILE / CPT;
@@ -752,7 +756,8 @@ __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, Begin&& begi
 // Tile of the single-domain X sweep per element type: FP64 tiles of 256 cells at one cell per
 // thread; FP32 tiles of 512 cells at two cells per thread (256 threads), which measured faster for
 // the FP32-mixed sweep (408 us at 8192^2, one cell per thread 468) and slower for the FP64 one. The
-// LDS leaves room for 7 waves per SIMD, so the kernels are held to the 72 VGPRs that 7 waves have.
+// LDS leaves room for 7 waves per SIMD (8 without GAD and second order), so the kernels are held to the
+// 72 (64) VGPRs that so many have.
 template <class T>
 struct XTile {
     static constexpr int cells = 256, cpt = 1;
@@ -763,12 +768,12 @@ struct XTile<float> {
 };
 
 template <class T, int FLUX, int PROJ, int EOS, int DXM, bool FOLD>
-__global__ void __launch_bounds__(XTile<T>::cells / XTile<T>::cpt) __attribute__((amdgpu_waves_per_eu(7)))
+__global__ void __launch_bounds__(XTile<T>::cells / XTile<T>::cpt) __attribute__((amdgpu_waves_per_eu(FLUX > 0 || PROJ == 2 ? 7 : 8)))
         k_sweep_x(SweepArgs<T> a)
 {
     constexpr int TILE = XTile<T>::cells;
     constexpr int W = TILE - 2 * (2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0));
-    __shared__ TileLds<T, TILE, 1> sm;
+    __shared__ SchemeLds<T, FLUX, PROJ, TILE, 1> sm;
     const int s0 = xcd_block(blockIdx.x, gridDim.x) * W;   // first slot of the tile
     const int j0 = s0 / a.x_slots;
     sweep_x_tile<T, FLUX, PROJ, EOS, DXM, TILE, XTile<T>::cpt>(
@@ -870,6 +875,13 @@ struct MarchWindows<float> {
         yL_[0] = yL_[1];
         yL_[1] = yL;
     }
+};
+
+// A block's LDS: one in a kernel, also where that holds two copies of the march.
+template <class T>
+struct MarchBlockLds {
+    MarchLds<T> keep;
+    typename MarchWindows<T>::Lds windows;
 };
 
 // The march state of one column of a Y run: sliding windows of the stage results along y. Each row's
@@ -1075,14 +1087,15 @@ struct YColumn {
 // each wave reads and writes per array and row (512 bytes in FP64) then fall in different DRAM
 // pages: a copy with the FP64 march's access pattern and no arithmetic (ymarch_copy.hip) moves
 // 4.2 TB/s that way and 4.6 TB/s with a barrier every 1-8 rows. With the barrier the FP32-mixed
-// march (98 VGPRs) is 9% faster and the FP64 march 3.6%; the FP64 march fits 3 waves per SIMD
-// with it only with the sound-speed window in LDS and the 3-wave occupancy hint (168 VGPRs,
-// against 178 with a register window). `idle` waves (past the last column) take part in the
-// barriers only. SYNC needs the same number of rows for the whole block: the loop-free batched
-// kernel takes it for a block whose 4 waves hold live runs of equal length (most blocks, as
-// the runs are listed longest first) and the independent march otherwise.
+// march is 9% faster and the FP64 march 3.6% (and with stale layers, Godunov and first-order
+// projection, us per sweep at 8192^2 without -> with: FP64 968 -> 909, FP32 568 -> 489).
+// `idle` waves (past the last column) take part in the barriers only. SYNC needs the same number
+// of rows for the whole block: the loop-free batched kernel takes it for a block whose 4 waves
+// hold live runs of equal length (most blocks, as the runs are listed longest first) and the
+// independent march otherwise.
 template <class T, int FLUX, int PROJ, int EOS, int DXM, bool STALE, bool SYNC = false>
-__device__ __forceinline__ void sweep_y_run(const SweepArgs<T>& a, T dt, int x, int y0, int y1, bool idle = false)
+__device__ __forceinline__ void sweep_y_run(const SweepArgs<T>& a, T dt, int x, int y0, int y1, MarchBlockLds<T>& lds,
+                                            bool idle = false)
 {
     using Col = YColumn<T, FLUX, PROJ, EOS, DXM, STALE>;
     constexpr int R = Col::R;
@@ -1091,8 +1104,8 @@ __device__ __forceinline__ void sweep_y_run(const SweepArgs<T>& a, T dt, int x, 
     const int rows = y1 - y0 + 2 * R;
     // SYNC marches whole groups of 4 rows: up to 3 steps past the run, which load nothing (the
     // row-ahead load stops at the run's last row; without stale layers a cell is made from the
-    // loaded state alone) and store nothing (outputs are rows [y0, y1) only)
-    static_assert(!(SYNC && STALE), "the block-synchronised march has no stale ghost layers");
+    // loaded state alone) and store nothing (outputs are rows [y0, y1) only). With stale layers,
+    // whose p and c a step loads, those steps are left out.
     const int groups = (rows + 3) / 4;
     if constexpr (SYNC) {
         if (idle) {
@@ -1101,18 +1114,20 @@ __device__ __forceinline__ void sweep_y_run(const SweepArgs<T>& a, T dt, int x, 
         }
     }
     Col col;
-    __shared__ MarchLds<T> keep;
-    __shared__ typename MarchWindows<T>::Lds windows;
-    col.init(x, x < a.nx, &windows);
+    auto& keep = lds.keep;
+    col.init(x, x < a.nx, &lds.windows);
     col.fetch(a, y0 - R);
     if constexpr (SYNC) {
         for (int g = 0; g < groups; ++g) {
 #pragma unroll(sizeof(T) == 8 ? kYUnrollFp64 : kYUnrollFp32)
-            for (int k = 0; k < 4; ++k) col.step(a, dt, (T) a.dx, (T) a.inv_dx, y0 - R + 4 * g + k, y0, y1, keep);
+            for (int k = 0; k < 4; ++k)
+                if (!STALE || 4 * g + k < rows)
+                    col.step(a, dt, (T) a.dx, (T) a.inv_dx, y0 - R + 4 * g + k, y0, y1, keep);
             __syncthreads();
         }
     } else {
-#pragma unroll(sizeof(T) == 8 ? kYUnrollFp64 : kYUnrollFp32)
+        // not unrolled: step()'s empty asm keeps the compiler from it, and two rows a turn by hand (with the
+        // rest of the rows after it) measured no faster
         for (int i = 0; i < rows; ++i) col.step(a, dt, (T) a.dx, (T) a.inv_dx, y0 - R + i, y0, y1, keep);
     }
     if (a.reduce) reduce_cfl(a.st, col.speeds.bound(a.cfl_dx, a.cfl_dy));
@@ -1128,9 +1143,8 @@ __global__ void __launch_bounds__(kYBlock) ARMON_Y_OCCUPANCY k_sweep_y(SweepArgs
     const int x = (bid - seg * ncolblk) * kYBlock + threadIdx.x;
     const bool idle = x - (int) (threadIdx.x & 63) >= a.nx;   // a wave past the last column
     const int y0 = seg * a.seg_len;
-    constexpr bool sync = !STALE;   // see sweep_y_run
-    if (idle && !sync) return;   // no barriers follow
-    sweep_y_run<T, FLUX, PROJ, EOS, DXM, STALE, sync>(a, dt, x, y0, min(y0 + a.seg_len, a.ny), idle);
+    __shared__ MarchBlockLds<T> lds;
+    sweep_y_run<T, FLUX, PROJ, EOS, DXM, STALE, true>(a, dt, x, y0, min(y0 + a.seg_len, a.ny), lds, idle);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1142,7 +1156,7 @@ __global__ void __launch_bounds__(kYBlock) ARMON_Y_OCCUPANCY k_sweep_y(SweepArgs
 // row apart. Called by NT threads, each with COLS ROWS / NT cells of one column.
 template <class T, int FLUX, int PROJ, int EOS, int DXM, int COLS, int ROWS, int NT, class Begin>
 __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, Begin&& begin, int x0, int y0,
-                                             TileLds<T, COLS * ROWS, COLS>& sm)
+                                             SchemeLds<T, FLUX, PROJ, COLS * ROWS, COLS>& sm)
 {
     constexpr int R = 2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0);
     constexpr int CPT = COLS * ROWS / NT;
@@ -1208,7 +1222,7 @@ __global__ void __launch_bounds__(YTile<T>::threads) k_sweep_y_tile(SweepArgs<T>
 {
     using Y = YTile<T>;
     constexpr int W = Y::rows - 2 * (2 + (FLUX > 0 ? 1 : 0) + (PROJ == 2 ? 1 : 0));
-    __shared__ TileLds<T, Y::cols * Y::rows, Y::cols> sm;
+    __shared__ SchemeLds<T, FLUX, PROJ, Y::cols * Y::rows, Y::cols> sm;
     const int bid = xcd_block(blockIdx.x, gridDim.x);
     const int band = bid / ncolblk;
     sweep_y_tile<T, FLUX, PROJ, EOS, DXM, Y::cols, Y::rows, Y::threads>(
@@ -1272,7 +1286,7 @@ __device__ __forceinline__ SweepArgs<T> batch_domain_args(const BatchArgs<T>& b,
 template <class T, int FLUX, int PROJ, int EOS, int TILE>
 __global__ void __launch_bounds__(TILE) k_batch_x(BatchArgs<T> b, const BatchItemX* __restrict__ items, int nitems)
 {
-    __shared__ TileLds<T, TILE, 1> sm;
+    __shared__ SchemeLds<T, FLUX, PROJ, TILE, 1> sm;
     for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
         const BatchItemX item = items[it];
         const DeviceState* st = b.states + item.domain;
@@ -1290,7 +1304,7 @@ __global__ void __launch_bounds__(TILE) k_batch_x(BatchArgs<T> b, const BatchIte
 template <class T, int FLUX, int PROJ, int EOS, bool FOLD, int TILE, int CPT = 1>
 __global__ void __launch_bounds__(TILE / CPT) k_batch_x1(BatchArgs<T> b, const BatchItemX* __restrict__ items)
 {
-    __shared__ TileLds<T, TILE, 1> sm;
+    __shared__ SchemeLds<T, FLUX, PROJ, TILE, 1> sm;
     const BatchItemX item = items[xcd_block(blockIdx.x, gridDim.x)];
     const SweepArgs<T> a = batch_domain_args<FOLD>(b, item.domain, 0);
     // a domain's first tile writes its step
@@ -1304,21 +1318,18 @@ template <class T, int FLUX, int PROJ, int EOS, bool FOLD>
 __global__ void __launch_bounds__(YTile<T>::threads) k_batch_y_tile(BatchArgs<T> b, const BatchItemY* __restrict__ items)
 {
     using Y = YTile<T>;
-    __shared__ TileLds<T, Y::cols * Y::rows, Y::cols> sm;
+    __shared__ SchemeLds<T, FLUX, PROJ, Y::cols * Y::rows, Y::cols> sm;
     const BatchItemY item = items[xcd_block(blockIdx.x, gridDim.x)];
     const SweepArgs<T> a = batch_domain_args<FOLD>(b, item.domain, 1);
     sweep_y_tile<T, FLUX, PROJ, EOS, kBatchDxMode<T>, Y::cols, Y::rows, Y::threads>(
             a, [&](double& dt) { return begin_sweep<FOLD>(a, item.x0 == 0 && item.y0 == 0, dt); }, item.x0, item.y0, sm);
 }
 
-// The row-ahead loads of the FP64 march need 179 VGPRs here (the per-item domain arguments
-// add to the single-domain sweep's 164), which would leave 2 waves per SIMD; capped at 3 waves,
-// the compiler keeps 7 dwords of item-invariant values in scratch instead (one 16-byte reload
-// per row), and the FP64 sweep is 4% faster than without the row-ahead loads.
 template <class T, int FLUX, int PROJ, int EOS, bool STALE>
 __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)))
         k_batch_y(BatchArgs<T> b, const BatchItemY* __restrict__ items, int nitems)
 {
+    __shared__ MarchBlockLds<T> lds;
     const int lane = threadIdx.x & 63;
     const int nwaves = (gridDim.x * blockDim.x) >> 6;
     // the item index is uniform across the wave: keep it (and what is loaded through it) scalar
@@ -1329,8 +1340,8 @@ __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)
         if (!st->active) continue;   // the same for the whole wave
         const SweepArgs<T> a = batch_domain_args(b, item.domain, 1);
         const int x = item.x0 + lane;
-            sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE>(a, (T) (st->current_dt * b.dt_factor), x,
-                                                                       item.y0, item.y1);
+        sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE>(a, (T) (st->current_dt * b.dt_factor), x,
+                                                                item.y0, item.y1, lds);
     }
 }
 
@@ -1344,6 +1355,7 @@ template <class T, int FLUX, int PROJ, int EOS, bool STALE>
 __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)))
         k_batch_y1(BatchArgs<T> b, const BatchItemY* __restrict__ items, int nitems)
 {
+    __shared__ MarchBlockLds<T> lds;
     const int lane = threadIdx.x & 63;
     const int it = __builtin_amdgcn_readfirstlane((int) ((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
     BatchItemY item{0, 0, 0, 0};
@@ -1352,27 +1364,22 @@ __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)
         item = items[it];
         live = b.states[item.domain].active != 0;
     }
-    bool sync = false;
-    if constexpr (!STALE) {
-        __shared__ int rows_of_wave[kYBlock / 64];
-        if (lane == 0) rows_of_wave[threadIdx.x >> 6] = live ? item.y1 - item.y0 : -1;
-        __syncthreads();
-        sync = true;
+    __shared__ int rows_of_wave[kYBlock / 64];
+    if (lane == 0) rows_of_wave[threadIdx.x >> 6] = live ? item.y1 - item.y0 : -1;
+    __syncthreads();
+    bool sync = true;
 #pragma unroll
-        for (int w = 0; w < kYBlock / 64; w++) sync = sync && rows_of_wave[w] == rows_of_wave[0] && rows_of_wave[w] >= 0;
-    }
+    for (int w = 0; w < kYBlock / 64; w++) sync = sync && rows_of_wave[w] == rows_of_wave[0] && rows_of_wave[w] >= 0;
     if (!live) return;   // the whole wave; never in a synchronised block
     const DeviceState* st = b.states + item.domain;
     const SweepArgs<T> a = batch_domain_args(b, item.domain, 1);
     const int x = item.x0 + lane;
     const T dt = (T) (st->current_dt * b.dt_factor);
-    if constexpr (!STALE) {
-        if (sync) {
-            sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE, true>(a, dt, x, item.y0, item.y1);
-            return;
-        }
+    if (sync) {
+        sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE, true>(a, dt, x, item.y0, item.y1, lds);
+        return;
     }
-    sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE>(a, dt, x, item.y0, item.y1);
+    sweep_y_run<T, FLUX, PROJ, EOS, kBatchDxMode<T>, STALE>(a, dt, x, item.y0, item.y1, lds);
 }
 
 // X tiles covering a stream of `slots` slots (tiles of W outputs overlapping by 2R): the last
