@@ -85,7 +85,8 @@ struct ArmonBatch {
     hipGraphExec_t graph[2] = {};        // graph_chunk cycles from an even (0) or odd (1) cycle
     hipGraph_t graph_def[2] = {};
     bool initialized = false, begun = false, finished = false;
-    std::vector<DeviceState> final_states;
+    StateReports reports;                // of the domains' states, for the host
+    std::vector<StepState> final_states;
 
     ~ArmonBatch();
     view slice(int field, int d)
@@ -346,27 +347,14 @@ void advance(ArmonBatch* b, int64_t n)
     }
 }
 
-std::vector<DeviceState> read_states(ArmonBatch* b)
-{
-    std::vector<DeviceState> h(b->p.size());
-    hip_check(hipMemcpyAsync(h.data(), b->states_at(b->cycles_enqueued), sizeof(DeviceState) * h.size(), hipMemcpyDeviceToHost, b->stream),
-              "read device states");
-    hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-    return h;
-}
+const DeviceState* last_states(const ArmonBatch* b) { return b->states_at(b->cycles_enqueued); }
 
 // The states before the first cycle, then the EOS and CFL minima of the initial fields and the working
 // buffers (launch_begin).
 void begin_fields(ArmonBatch* b, DeviceState* states)
 {
     const int n = (int) b->p.size();
-    std::vector<DeviceState> zero(n);
-    for (auto& s : zero) {
-        memset(&s, 0, sizeof s);
-        for (auto& slot : s.dt_min) slot.bits = kNoBound;
-    }
-    hip_check(hipMemcpyAsync(states, zero.data(), sizeof(DeviceState) * n, hipMemcpyHostToDevice, b->stream),
-              "init device states");
+    launch_clear(states, n, b->stream);
     launch_begin(b->fields(), b->d_domains, n, b->domains[0], b->total, states, b->var.eos, 1.4, b->stream);
     hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
 }
@@ -528,13 +516,14 @@ ARMON_EXPORT ArmonBatch* armon_batch_create(const ArmonParams* common, int n, co
             for (int k = 0; k < 4; k++) boundary_factors(q, sides[k], &D.bc[k][0], &D.bc[k][1]);
             D.x_slots = q.nx + 2 * read_extent(b->var.flux, b->var.proj);
             D.x_inv_slots = 1.0f / (float) D.x_slots;
-            cfg[d] = TimeStepConfig{q.cfl, q.Dt, q.max_time, q.max_cycles, q.cst_dt, q.dt_on_even_cycles};
+            cfg[d] = step_config(q);
         }
         b->domains = dom;
         b->d_domains = device_alloc<BatchDomain>(n, "hipMalloc(domains)");
         b->d_cfgs = device_alloc<TimeStepConfig>(n, "hipMalloc(configs)");
         b->d_states = device_alloc<DeviceState>(2 * (size_t) n, "hipMalloc(states)");
         b->d_tune = device_alloc<DeviceState>(n, "hipMalloc(tune states)");
+        b->reports.create(n);
         hip_check(hipMemcpy(b->d_domains, dom.data(), sizeof(BatchDomain) * n, hipMemcpyHostToDevice), "upload domains");
         hip_check(hipMemcpy(b->d_cfgs, cfg.data(), sizeof(TimeStepConfig) * n, hipMemcpyHostToDevice), "upload configs");
         // default configuration: 256-cell X tiles of one cell per thread, Y tiles or 256-row Y runs by
@@ -753,7 +742,9 @@ ARMON_EXPORT int armon_batch_active(ArmonBatch* b)
 {
     try {
         int k = 0;
-        for (const DeviceState& s : read_states(b)) k += s.active && !s.error;
+        b->reports.post(last_states(b), 0, b->stream);
+        const StepState* s = b->reports.wait(0);
+        for (int d = 0; d < b->reports.size(); d++) k += s[d].running();
         return k;
     } catch (const std::exception& e) {
         fail("armon_batch_active", e);
@@ -766,12 +757,12 @@ ARMON_EXPORT int armon_batch_run(ArmonBatch* b)
     try {
         if (!b->begun || b->finished) throw invalid_argument("armon_batch_begin must come first");
         const int chunk = b->common.graph_chunk > 0 ? b->common.graph_chunk : 16;
-        while (true) {
-            advance(b, chunk);
-            bool any = false;
-            for (const DeviceState& s : read_states(b)) any = any || (s.active && !s.error);
-            if (!any) break;
-        }
+        run_chunks(b->reports, chunk, b->stream,
+                   [&] {
+                       advance(b, chunk);
+                       return last_states(b);
+                   },
+                   [&](int d) { return step_config(b->p[d]); });
         return 0;
     } catch (const std::exception& e) {
         fail("armon_batch_run", e);
@@ -786,10 +777,15 @@ ARMON_EXPORT int armon_batch_finish(ArmonBatch* b)
     try {
         if (!b->begun) throw invalid_argument("armon_batch_begin must come first");
         if (b->finished) return 0;
-        b->final_states = read_states(b);
+        b->reports.post(last_states(b), 0, b->stream);
+        launch_finish(b->fields(), b->d_domains, (int) b->p.size(), b->domains[0], b->total, last_states(b),
+                      b->sweeps_per_cycle, b->var.eos, 1.4, b->stream);
+        hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
+        const StepState* states = b->reports.wait(0);
+        b->final_states.assign(states, states + b->reports.size());
         int status = 0;
         for (int d = 0; d < (int) b->p.size(); d++) {
-            const DeviceState& h = b->final_states[d];
+            const StepState& h = b->final_states[d];
             ArmonParams& q = b->p[d];
             q.cycle = h.cycle;
             q.time = h.time;
@@ -797,9 +793,6 @@ ARMON_EXPORT int armon_batch_finish(ArmonBatch* b)
             q.next_cycle_dt = h.next_dt;
             if (h.error) status = 1;
         }
-        launch_finish(b->fields(), b->d_domains, (int) b->p.size(), b->domains[0], b->total,
-                      b->states_at(b->cycles_enqueued), b->sweeps_per_cycle, b->var.eos, 1.4, b->stream);
-        hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
         b->finished = true;
         b->initialized = false;   // a new run starts from armon_batch_init
         return status;
@@ -812,7 +805,7 @@ ARMON_EXPORT int armon_batch_finish(ArmonBatch* b)
 ARMON_EXPORT int armon_batch_domain_result(ArmonBatch* b, int d, ArmonResult* out)
 {
     if (d < 0 || d >= (int) b->p.size() || !b->finished) return 1;
-    const DeviceState& h = b->final_states[d];
+    const StepState& h = b->final_states[d];
     memset(out, 0, sizeof *out);
     out->status = h.error ? 1 : 0;
     out->cycles = h.cycle;

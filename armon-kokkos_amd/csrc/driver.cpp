@@ -137,6 +137,7 @@ struct ArmonSolver {
 
     // fused engine
     DeviceState* st = nullptr;       // two: the cycles step from one to the other, from st[0]
+    StateReports reports;            // of the state, for the host
     float* f32[10] = {};             // FP32-mixed buffers: A rho,u,v,E | B rho,u,v,E | stale p, c
     int sweeps_per_cycle = 2;
     int64_t cycles_enqueued = 0;
@@ -448,7 +449,7 @@ struct Timer {
 void fused_enqueue_cycle(ArmonSolver* s, int64_t cycle, Timer* timer)
 {
     const ArmonParams& p = s->p;
-    const TimeStepConfig tc{p.cfl, p.Dt, p.max_time, p.max_cycles, p.cst_dt, p.dt_on_even_cycles};
+    const TimeStepConfig tc = step_config(p);
     const DeviceState* prev = s->st + (cycle & 1);
     DeviceState* st = s->st + ((cycle + 1) & 1);
     ArmonParams pc = p;
@@ -538,13 +539,12 @@ void fused_advance(ArmonSolver* s, int64_t n)
     }
 }
 
-DeviceState read_state(ArmonSolver* s)
+const DeviceState* last_state(const ArmonSolver* s) { return s->st + (s->cycles_enqueued & 1); }
+
+StepState read_state(ArmonSolver* s)
 {
-    DeviceState h{};
-    hip_check(hipMemcpyAsync(&h, s->st + (s->cycles_enqueued & 1), sizeof h, hipMemcpyDeviceToHost, s->stream),
-              "read device state");
-    hip_check(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
-    return h;
+    s->reports.post(last_state(s), 0, s->stream);
+    return *s->reports.wait(0);
 }
 
 FieldArrays field_arrays(ArmonSolver* s)
@@ -573,9 +573,7 @@ BatchDomain own_domain(const ArmonSolver* s)
 void fused_begin(ArmonSolver* s)
 {
     ArmonParams& p = s->p;
-    DeviceState h{};
-    for (auto& slot : h.dt_min) slot.bits = kNoBound;
-    hip_check(hipMemcpyAsync(s->st, &h, sizeof h, hipMemcpyHostToDevice, s->stream), "init device state");
+    launch_clear(s->st, 1, s->stream);
     launch_begin(field_arrays(s), nullptr, 1, own_domain(s), s->n, s->st, p.test == 3 ? 1 : 0, 1.4, s->stream);
     hip_check(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
     s->cycles_enqueued = 0;
@@ -586,17 +584,18 @@ void fused_begin(ArmonSolver* s)
 }
 
 // After the loop: put the final state in rho/umat/vmat/Emat and the EOS of the last sweep's
-// input state in pmat/cmat/gmat, as the reference leaves them.
-void fused_finish(ArmonSolver* s)
+// input state in pmat/cmat/gmat, as the reference leaves them. Returns the time-stepping state.
+StepState fused_finish(ArmonSolver* s)
 {
+    s->reports.post(last_state(s), 0, s->stream);
     const ArmonParams& p = s->p;
-    launch_finish(field_arrays(s), nullptr, 1, own_domain(s), s->n, s->st + (s->cycles_enqueued & 1),
-                  s->sweeps_per_cycle, p.test == 3 ? 1 : 0, 1.4, s->stream);
+    launch_finish(field_arrays(s), nullptr, 1, own_domain(s), s->n, last_state(s), s->sweeps_per_cycle, p.test == 3 ? 1 : 0, 1.4, s->stream);
     hip_check(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
+    return *s->reports.wait(0);
 }
 
 // Mass and energy of the fused engine's current state (the buffer written by the last sweep).
-void fused_conservation(ArmonSolver* s, const DeviceState& h, double* mass, double* energy)
+void fused_conservation(ArmonSolver* s, const StepState& h, double* mass, double* energy)
 {
     const ArmonParams& p = s->p;
     const int cur = (int) (((int64_t) h.cycle * s->sweeps_per_cycle) & 1);
@@ -985,6 +984,7 @@ ARMON_EXPORT ArmonSolver* armon_solver_create(const ArmonParams* params)
         void* st = nullptr;
         hip_check(hipMalloc(&st, 2 * sizeof(DeviceState)), "hipMalloc(states)");
         s->st = static_cast<DeviceState*>(st);
+        s->reports.create(1);
         if (s->p.engine == ARMON_ENGINE_FUSED && s->p.precision == ARMON_PREC_FP32_MIXED) {
             for (int k = 0; k < 10; k++) {
                 void* ptr = nullptr;
@@ -1108,7 +1108,7 @@ ARMON_EXPORT int armon_solver_finish(ArmonSolver* s, ArmonResult* out)
         ArmonParams& p = s->p;
         int status = 0;
         if (p.engine == ARMON_ENGINE_FUSED) {
-            const DeviceState h = read_state(s);
+            const StepState h = fused_finish(s);
             p.cycle = h.cycle;
             p.time = h.time;
             p.current_cycle_dt = h.current_dt;
@@ -1123,7 +1123,6 @@ ARMON_EXPORT int armon_solver_finish(ArmonSolver* s, ArmonResult* out)
                 armon_update_axis(&p, axes[n - 1]);
                 p.cycle_dt = p.current_cycle_dt * factors[n - 1];
             }
-            fused_finish(s);
             if (h.error) {
                 char buf[128];
                 snprintf(buf, sizeof buf, "Invalid dt at cycle %d: %f", h.error_cycle, h.error_dt);
@@ -1160,12 +1159,21 @@ ARMON_EXPORT int armon_solver_time_loop(ArmonSolver* s, ArmonResult* out)
     ArmonParams& p = s->p;
     if (p.engine == ARMON_ENGINE_FUSED) {
         try {
-            const int chunk = p.verbose <= 1 ? 1 : (p.graph_chunk > 0 ? p.graph_chunk : 16);
+            const int chunk = p.graph_chunk > 0 ? p.graph_chunk : 16;
+            if (p.verbose > 1) {
+                run_chunks(s->reports, chunk, s->stream,
+                           [&] {
+                               fused_advance(s, chunk);
+                               return last_state(s);
+                           },
+                           [&](int) { return step_config(p); });
+                return armon_solver_finish(s, out);
+            }
             double prev_time = 0.0;
             while (true) {
-                fused_advance(s, chunk);
-                const DeviceState h = read_state(s);
-                if (p.verbose <= 1 && h.active) {
+                fused_advance(s, 1);
+                const StepState h = read_state(s);
+                if (h.active) {
                     // armon_2D.cpp:351-357; the state is in the buffer of the last sweep
                     double m, e;
                     fused_conservation(s, h, &m, &e);

@@ -1,5 +1,6 @@
 // Fused engine, FP64 instantiation of the sweep kernels (sweep_kernels.hpp), plus the kernels of
 // the time step and of what comes before the first cycle and after the last one.
+#include "internal.hpp"
 #include "sweep_kernels.hpp"
 
 #include <cfloat>
@@ -29,6 +30,19 @@ __global__ void k_f2d(const float* in, double* out, int64_t n)
 {
     for (int64_t k = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t) gridDim.x * blockDim.x)
         out[k] = (double) in[k];
+}
+
+__global__ void __launch_bounds__(64) k_clear(DeviceState* states)
+{
+    DeviceState& st = states[blockIdx.x];
+    if (threadIdx.x < kDtSlots) st.dt_min[threadIdx.x].bits = kNoBound;
+    if (threadIdx.x == 63) static_cast<StepState&>(st) = StepState{};
+}
+
+__global__ void __launch_bounds__(64) k_report(const DeviceState* states, int n, StepState* out)
+{
+    const int d = blockIdx.x * blockDim.x + threadIdx.x;
+    if (d < n) out[d] = states[d];
 }
 
 // Domains start on multiples of a wave's 64 elements, so a wave's elements belong to one domain: the
@@ -194,6 +208,47 @@ void launch_finish(const FieldArrays& f, const BatchDomain* domains, int n, cons
     k_finish<<<element_blocks(elements), 256, 0, s>>>(f, domains, n, one, elements, states, sweeps_per_cycle, eos,
                                                       gamma);
     check_launch("finish");
+}
+
+void launch_clear(DeviceState* states, int n, hipStream_t s)
+{
+    k_clear<<<(unsigned) n, 64, 0, s>>>(states);
+    check_launch("clear");
+}
+
+void launch_report(const DeviceState* states, int n, StepState* out, hipStream_t s)
+{
+    k_report<<<(unsigned) ((n + 63) / 64), 64, 0, s>>>(states, n, out);
+    check_launch("report");
+}
+
+StateReports::~StateReports()
+{
+    for (hipEvent_t e : arrived_)
+        if (e) (void) hipEventDestroy(e);
+    if (host_) (void) hipHostFree(host_);
+}
+
+void StateReports::create(int n)
+{
+    void* p = nullptr;
+    hip_check(hipHostMalloc(&p, 2 * sizeof(StepState) * (size_t) n, hipHostMallocDefault), "hipHostMalloc(reports)");
+    host_ = static_cast<StepState*>(p);
+    n_ = n;
+    for (hipEvent_t& e : arrived_)
+        hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+}
+
+void StateReports::post(const DeviceState* states, int k, hipStream_t s)
+{
+    launch_report(states, n_, host_ + (k & 1) * (size_t) n_, s);
+    hip_check(hipEventRecord(arrived_[k & 1], s), "hipEventRecord");
+}
+
+const StepState* StateReports::wait(int k)
+{
+    hip_check(hipEventSynchronize(arrived_[k & 1]), "hipEventSynchronize");
+    return host_ + (k & 1) * (size_t) n_;
 }
 
 void launch_convert_f2d(const float* in, double* out, int64_t n, hipStream_t s)

@@ -1,6 +1,8 @@
 // Fused Lagrange + remap sweeps: device state and launch interface.
 #pragma once
 
+#include "armon/armon.h"
+
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -17,8 +19,13 @@ struct alignas(128) DtSlot {
 };
 constexpr unsigned long long kNoBound = 0x7FEFFFFFFFFFFFFFull;   // DBL_MAX
 
+struct TimeStepConfig {
+    double cfl, Dt, max_time;
+    int max_cycles, cst_dt, dt_on_even_cycles;
+};
+
 // Time-stepping state kept on the device between cycles (armon_2D.cpp:229-252, 347-361).
-struct DeviceState {
+struct StepState {
     double current_dt;
     double next_dt;
     double time;
@@ -27,13 +34,23 @@ struct DeviceState {
     int active;                      // 1 while the current cycle runs
     int error;                       // 1 after an invalid time step
     int error_cycle;
+
+    bool running() const { return active && !error; }
+    // Whether more cycles follow after `n` of this state's time step.
+    bool runs_on(const TimeStepConfig& c, int n) const
+    {
+        return running() && (int64_t) cycle + n < c.max_cycles && time + n * current_dt < c.max_time;
+    }
+};
+
+struct DeviceState : StepState {
     DtSlot dt_min[kDtSlots];
 };
 
-struct TimeStepConfig {
-    double cfl, Dt, max_time;
-    int max_cycles, cst_dt, dt_on_even_cycles;
-};
+inline TimeStepConfig step_config(const ArmonParams& p)
+{
+    return {p.cfl, p.Dt, p.max_time, p.max_cycles, p.cst_dt, p.dt_on_even_cycles};
+}
 
 // A cycle's time step is made from one state into another, in turn between two of them: by a kernel of
 // its own, or by the cycle's first sweep (`prev` set), each of whose waves computes it for itself
@@ -158,6 +175,61 @@ void launch_begin(const FieldArrays& f, const BatchDomain* domains, int n, const
 // cycle are left alone.
 void launch_finish(const FieldArrays& f, const BatchDomain* domains, int n, const BatchDomain& one, int64_t elements,
                    const DeviceState* states, int sweeps_per_cycle, int eos, double gamma, hipStream_t s);
+
+// The states before the first cycle, for launch_begin.
+void launch_clear(DeviceState* states, int n, hipStream_t s);
+
+// ---- the host's view of a run ---------------------------------------------------------------
+
+// Copies the time-stepping part of n states to `out`, which the device can write.
+void launch_report(const DeviceState* states, int n, StepState* out, hipStream_t s);
+
+// Reports of n states in pinned memory that the device writes: two, so that the host reads one while
+// the other is on its way. Whoever holds it calls create() once and uses it from one stream.
+class StateReports {
+public:
+    StateReports() = default;
+    StateReports(const StateReports&) = delete;
+    StateReports& operator=(const StateReports&) = delete;
+    ~StateReports();
+    void create(int n);
+    int size() const { return n_; }
+    // Enqueues report k (the one in the place of report k - 2).
+    void post(const DeviceState* states, int k, hipStream_t s);
+    // Report k, once it has arrived.
+    const StepState* wait(int k);
+
+private:
+    StepState* host_ = nullptr;
+    hipEvent_t arrived_[2] = {};
+    int n_ = 0;
+};
+
+// Runs chunks of `chunk` cycles until no state is running. `enqueue()` enqueues a chunk and returns the
+// states after it; `config(d)` is the configuration of state d.
+//
+// The host learns of a chunk's end a report's round trip later, 20-30 us in which the device would idle
+// (a quarter of a chunk of a 100^2 domain's cycles). So while chunk k runs, chunk k + 1 is enqueued
+// behind it, unless the report of chunk k - 1 says that chunk k will be the last: by the number of
+// cycles left, or by the time left at that report's time step. The guess costs nothing but time
+// where it is wrong: cycles after the end change no state (2 us a launch), and a chunk that was not
+// enqueued ahead is enqueued as soon as its turn is known.
+template <class Enqueue, class Config>
+void run_chunks(StateReports& reports, int chunk, hipStream_t s, Enqueue&& enqueue, Config&& config)
+{
+    const StepState* known = nullptr;   // the report before the newest one
+    reports.post(enqueue(), 0, s);
+    for (int k = 0;; k = (k + 1) & 1) {
+        bool ahead = false;
+        for (int d = 0; known && !ahead && d < reports.size(); d++) ahead = known[d].runs_on(config(d), chunk);
+        if (ahead) reports.post(enqueue(), k ^ 1, s);
+        known = reports.wait(k);
+        bool any = false;
+        for (int d = 0; d < reports.size(); d++) any = any || known[d].runs_on(config(d), 0);
+        if (!any) return;
+        if (!ahead) reports.post(enqueue(), k ^ 1, s);
+    }
+}
 
 // Element-wise conversion of an FP32 working buffer to a reference FP64 array.
 void launch_convert_f2d(const float* in, double* out, int64_t n, hipStream_t s);
