@@ -234,7 +234,7 @@ BatchArgs<T> batch_args(ArmonBatch* b, int parity, double factor, bool reduce, D
     a.prev = prev;
     a.steps = b->d_cfgs;
     a.stencil_width = b->common.stencil_width;
-    a.reduce = reduce ? 1 : 0;
+    a.reduce = reduce ? REDUCE : REDUCE_NO;
     a.gamma = 1.4;
     a.dt_factor = factor;
     return a;

@@ -416,7 +416,7 @@ SweepArgs<T> sweep_args(ArmonSolver* s, int axis, double factor, bool reduce, T*
     boundary_factors(p, axis == ARMON_AXIS_X ? ARMON_SIDE_LEFT : ARMON_SIDE_BOTTOM, &lu, &lv);
     boundary_factors(p, axis == ARMON_AXIS_X ? ARMON_SIDE_RIGHT : ARMON_SIDE_TOP, &hu, &hv);
     a.lo_u = lu; a.lo_v = lv; a.hi_u = hu; a.hi_v = hv;
-    a.reduce = reduce ? 1 : 0;
+    a.reduce = reduce ? REDUCE : REDUCE_NO;
     a.cfl_dx = p.domain_size[0] / (double) p.nx;
     a.cfl_dy = p.domain_size[1] / (double) p.ny;
     return a;

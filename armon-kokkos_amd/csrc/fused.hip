@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(256) k_begin(FieldArrays f, const BatchDomain*
             f.other[3][e] = E;
         }
     }
-    reduce_cfl(states + which, speeds.bound(d.cfl_dx, d.cfl_dy));
+    reduce_cfl(states + which, REDUCE, speeds.bound(d.cfl_dx, d.cfl_dy));
 }
 
 __global__ void __launch_bounds__(256) k_finish(FieldArrays f, const BatchDomain* domains, int n, BatchDomain one,

@@ -59,6 +59,8 @@ inline TimeStepConfig step_config(const ArmonParams& p)
 // sweeps of up to kFoldedCells cells (measured: 1024^2 FP64 1.07x faster a cycle, 2048^2 even).
 constexpr int64_t kFoldedCells = 5 << 19;   // 2.6 M
 
+enum { REDUCE_NO, REDUCE, REDUCE_UNSEEN };   // not, after a look at the accumulator, without one
+
 // Everything a sweep kernel needs. Arrays use the reference layout: row-major with
 // nb_ghosts ghost layers on every side, index(i, j) = index_start + j*row_length + i.
 template <class T>
@@ -73,7 +75,8 @@ struct SweepArgs {
     int seg_len;                          // Y sweep: rows per marching run (set by the launcher)
     int x_slots;                          // X sweep: slots per row, nx + 2 x the ghost layers read
     float x_inv_slots;                    // 1 / x_slots
-    int dx_mode, reduce;                  // dx_mode: DX_POW2 (inv_dx = 1 / dx) or DX_RECIP (inv_dx = RN(1 / dx))
+    int dx_mode;                          // DX_POW2 (inv_dx = 1 / dx) or DX_RECIP (inv_dx = RN(1 / dx))
+    int reduce;                           // whether and how the sweep adds to the CFL accumulators: REDUCE_*
     double gamma, dx, inv_dx, dt_factor;
     double lo_u, lo_v, hi_u, hi_v;        // BC factors: Left/Bottom (lo), Right/Top (hi)
     double cfl_dx, cfl_dy;
