@@ -295,7 +295,7 @@ void enqueue_cycle(ArmonBatch* b, int64_t cycle, Timer* t)
     const int n = armon_split_axes(&pc, axes, factors);
     // the first sweep makes the time step where each of its blocks has one item
     const bool single = axes[0] == ARMON_AXIS_X ? b->tuning.grid_x == 0 : b->y_tiles;
-    const bool folded = n > 1 && single && b->real_cells <= kFoldedCells;
+    const bool folded = n > 1 && single && b->real_cells <= folded_cells(b->fp64() ? 8 : 4);
     if (t) t->begin();
     if (!folded) launch_batch_time_step(prev, states, b->d_cfgs, (int) b->p.size(), b->stream);
     if (t) t->end(2);

@@ -458,7 +458,8 @@ void fused_enqueue_cycle(ArmonSolver* s, int64_t cycle, Timer* timer)
     double factors[3];
     const int n = armon_split_axes(&pc, axes, factors);
     // the last sweep adds to the bounds that the first one clears, so the two must be apart
-    const bool folded = n > 1 && p.y_run_rows <= 0 && (int64_t) p.nx * p.ny <= kFoldedCells;
+    const bool folded = n > 1 && p.y_run_rows <= 0 &&
+                        (int64_t) p.nx * p.ny <= folded_cells(p.precision == ARMON_PREC_FP64 ? 8 : 4);
     if (timer) timer->begin();
     if (!folded) launch_time_step(prev, st, tc, s->stream);
     if (timer) timer->end(2);

@@ -54,10 +54,12 @@ inline TimeStepConfig step_config(const ArmonParams& p)
 
 // A cycle's time step is made from one state into another, in turn between two of them: by a kernel of
 // its own, or by the cycle's first sweep (`prev` set), each of whose waves computes it for itself
-// while one wave writes it down for the sweeps that follow. That saves a launch a cycle, 4.5 us of the
-// 10-20 us of a small domain, for some 30 instructions a wave (7% of a sweep's), so it is done for
-// sweeps of up to kFoldedCells cells (measured: 1024^2 FP64 1.07x faster a cycle, 2048^2 even).
-constexpr int64_t kFoldedCells = 5 << 19;   // 2.6 M
+// while one wave writes it down for the sweeps that follow. That saves a launch a cycle for some 30
+// instructions a wave (7% of a sweep's) and a longer wait before its first stage, so it is done for
+// sweeps of up to folded_cells() cells (0.9 M, 2.1 M). Cycle without -> with it, us: FP64 256^2
+// 12.4 -> 11.0, 512^2 18.8 -> 17.9, 1024x768 37.0 -> 36.8, 1024^2 46.2 -> 46.5, 2048x1280 93.0 -> 95.5;
+// FP32-mixed 512^2 13.2 -> 11.9, 1024^2 25.3 -> 24.4, 2048x1024 39.0 -> 39.1, 2048x1536 52.6 -> 53.4.
+constexpr int64_t folded_cells(size_t element) { return element == 8 ? 7 << 17 : 1 << 21; }
 
 enum { REDUCE_NO, REDUCE, REDUCE_UNSEEN };   // not, after a look at the accumulator, without one
 

@@ -1217,7 +1217,7 @@ template <class T>
 struct YTile {
     static constexpr int cols = y_tile_cols(), rows = y_tile_rows(), threads = sizeof(T) == 8 ? 512 : 256;
     static constexpr int64_t max_cells = y_tile_max_cells(sizeof(T));
-    static_assert(kFoldedCells <= max_cells, "the march makes no time step");
+    static_assert(folded_cells(sizeof(T)) <= max_cells, "the march makes no time step");
 };
 
 template <class T, int FLUX, int PROJ, int EOS, int DXM, bool FOLD>

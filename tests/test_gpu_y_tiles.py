@@ -60,6 +60,17 @@ def test_the_rule_on_the_number_of_cells(armon, ny):
         assert np.array_equal(a[f], b[f]), f
 
 
+# the largest domain whose first sweep makes the time step and the smallest one with a launch for it
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,ny", [(0, 896), (0, 897), (1, 2048), (1, 2049)])
+def test_the_rule_on_the_time_step(armon, precision, ny):
+    kw = dict(nx=1024, ny=ny, max_cycles=4, precision=precision, axis_splitting=1, **GAD2)
+    (a, _, da), (b, _, db) = _run(armon, "Sedov", **kw), _run(armon, "Sedov", y_run_rows=64, **kw)
+    assert da == db
+    for f in FIELDS:
+        assert np.array_equal(a[f], b[f]), f
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("precision,splitting,rows", [(0, 0, 16), (0, 2, 33), (1, 1, 64), (0, 4, 5)])
 def test_batch_tiles_are_its_marches(armon, precision, splitting, rows):
