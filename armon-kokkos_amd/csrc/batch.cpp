@@ -42,12 +42,6 @@ uint64_t splitmix64(uint64_t& s)
 
 double uniform01(uint64_t& s) { return (double) (splitmix64(s) >> 11) * 0x1.0p-53; }
 
-struct StreamScope {
-    void* saved;
-    explicit StreamScope(hipStream_t s) : saved(armon_get_stream()) { armon_set_stream(s); }
-    ~StreamScope() { armon_set_stream(saved); }
-};
-
 template <class T>
 T* device_alloc(size_t count, const char* what)
 {
@@ -69,6 +63,7 @@ struct ArmonBatch {
     double* arr[ARMON_FIELD_COUNT] = {};
     float* f32[10] = {};                 // FP32-mixed: A rho,u,v,E | B rho,u,v,E | stale p, c
     BatchDomain* d_domains = nullptr;
+    BatchInit* d_init = nullptr;
     DeviceState* d_states = nullptr;     // two per domain: the cycles step from one set to the other
     DeviceState* d_tune = nullptr;       // scratch states used while timing candidates
     TimeStepConfig* d_cfgs = nullptr;
@@ -89,10 +84,6 @@ struct ArmonBatch {
     std::vector<StepState> final_states;
 
     ~ArmonBatch();
-    view slice(int field, int d)
-    {
-        return view{arr[field] + offset[d], (int64_t) p[d].nb_cells, nullptr};
-    }
     bool fp64() const { return common.precision == ARMON_PREC_FP64; }
     // the states as of `cycles` enqueued cycles
     DeviceState* states_at(int64_t cycles) const { return d_states + (cycles & 1) * (int64_t) p.size(); }
@@ -116,7 +107,7 @@ ArmonBatch::~ArmonBatch()
         if (a) (void) hipFree(a);
     for (auto* a : f32)
         if (a) (void) hipFree(a);
-    for (void* a : {(void*) d_domains, (void*) d_states, (void*) d_tune, (void*) d_cfgs, (void*) d_items_x,
+    for (void* a : {(void*) d_domains, (void*) d_init, (void*) d_states, (void*) d_tune, (void*) d_cfgs, (void*) d_items_x,
                     (void*) d_items_y})
         if (a) (void) hipFree(a);
     if (stream) (void) hipStreamDestroy(stream);
@@ -493,6 +484,7 @@ ARMON_EXPORT ArmonBatch* armon_batch_create(const ArmonParams* common, int n, co
 
         std::vector<BatchDomain> dom(n);
         std::vector<TimeStepConfig> cfg(n);
+        std::vector<BatchInit> init(n);
         const int sides[4] = {ARMON_SIDE_LEFT, ARMON_SIDE_RIGHT, ARMON_SIDE_TOP, ARMON_SIDE_BOTTOM};
         for (int d = 0; d < n; d++) {
             const ArmonParams& q = b->p[d];
@@ -517,15 +509,20 @@ ARMON_EXPORT ArmonBatch* armon_batch_create(const ArmonParams* common, int n, co
             D.x_slots = q.nx + 2 * read_extent(b->var.flux, b->var.proj);
             D.x_inv_slots = 1.0f / (float) D.x_slots;
             cfg[d] = step_config(q);
+            init[d] = BatchInit{b->offset[d], q.nb_cells, q.row_length, q.nb_ghosts, q.nx, q.ny, q.test,
+                                {q.domain_size[0], q.domain_size[1]}, {q.domain_origin[0], q.domain_origin[1]},
+                                armon_test_option(&q), b->states[d]};
         }
         b->domains = dom;
         b->d_domains = device_alloc<BatchDomain>(n, "hipMalloc(domains)");
         b->d_cfgs = device_alloc<TimeStepConfig>(n, "hipMalloc(configs)");
+        b->d_init = device_alloc<BatchInit>(n, "hipMalloc(initial states)");
         b->d_states = device_alloc<DeviceState>(2 * (size_t) n, "hipMalloc(states)");
         b->d_tune = device_alloc<DeviceState>(n, "hipMalloc(tune states)");
         b->reports.create(n);
         hip_check(hipMemcpy(b->d_domains, dom.data(), sizeof(BatchDomain) * n, hipMemcpyHostToDevice), "upload domains");
         hip_check(hipMemcpy(b->d_cfgs, cfg.data(), sizeof(TimeStepConfig) * n, hipMemcpyHostToDevice), "upload configs");
+        hip_check(hipMemcpy(b->d_init, init.data(), sizeof(BatchInit) * n, hipMemcpyHostToDevice), "upload initial states");
         // default configuration: 256-cell X tiles of one cell per thread, Y tiles or 256-row Y runs by
         // the number of cells, one block per work item
         b->y_tiles = b->real_cells <= y_tile_max_cells(b->fp64() ? 8 : 4);
@@ -559,25 +556,8 @@ ARMON_EXPORT int armon_batch_init(ArmonBatch* b)
 {
     try {
         check_ready(b, false, true);
-        StreamScope scope(b->stream);
-        const uint64_t e0 = report_count();
-        for (int d = 0; d < (int) b->p.size(); d++) {
-            const ArmonParams& q = b->p[d];
-            DomainRange dr = armon_complete_domain(&q);
-            Range range;
-            InnerRange2D inner;
-            armon_domain_iter2D(&dr, &range, &inner);
-            view x = b->slice(ARMON_FIELD_X, d), y = b->slice(ARMON_FIELD_Y, d), rho = b->slice(ARMON_FIELD_RHO, d),
-                 E = b->slice(ARMON_FIELD_EMAT, d), u = b->slice(ARMON_FIELD_UMAT, d), v = b->slice(ARMON_FIELD_VMAT, d),
-                 mask = b->slice(ARMON_FIELD_DOMAIN_MASK, d), pm = b->slice(ARMON_FIELD_PMAT, d),
-                 cm = b->slice(ARMON_FIELD_CMAT, d), gm = b->slice(ARMON_FIELD_GMAT, d),
-                 us = b->slice(ARMON_FIELD_USTAR, d), ps = b->slice(ARMON_FIELD_PSTAR, d);
-            init_test_states(range, inner, q.row_length, q.nb_ghosts, q.nx, q.ny, q.domain_size[0], q.domain_size[1],
-                             q.domain_origin[0], q.domain_origin[1], 0, 0, q.nx, q.ny, x, y, rho, E, u, v, mask, pm, cm,
-                             gm, us, ps, static_cast<Test>(q.test), armon_test_option(&q), b->states[d]);
-        }
+        launch_batch_init(b->d_init, (int) b->p.size(), b->total, b->arr, b->stream);
         hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-        if (report_count() != e0) return 1;
         b->initialized = true;
         b->begun = false;
         b->finished = false;

@@ -45,19 +45,6 @@ __global__ void __launch_bounds__(64) k_report(const DeviceState* states, int n,
     if (d < n) out[d] = states[d];
 }
 
-// Domains start on multiples of a wave's 64 elements, so a wave's elements belong to one domain: the
-// last whose offset is not past them.
-__device__ __forceinline__ int domain_of(const BatchDomain* domains, int n, int64_t element)
-{
-    int lo = 0, hi = n;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (domains[mid].offset <= element) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // Whether element `i` of a domain is one of its real cells.
 __device__ __forceinline__ bool real_cell(const BatchDomain& d, int64_t i)
 {

@@ -116,6 +116,32 @@ struct BatchDomain {
     float x_inv_slots;             // 1 / x_slots
 };
 
+// Domains start on multiples of a wave's 64 elements, so a wave's elements belong to one domain: the
+// last whose offset is not past them.
+template <class Domain>
+__device__ __forceinline__ int domain_of(const Domain* domains, int n, int64_t element)
+{
+    int lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (domains[mid].offset <= element) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// What the initial state of one domain of a batch is made of (init_test_states).
+struct BatchInit {
+    long long offset, cells;       // first element of the domain in the packed arrays, and how many
+    int row_length, nb_ghosts, nx, ny, test;
+    double size[2], origin[2], option;
+    ArmonTestState states;
+};
+
+// The initial state of every domain in one launch, over the whole arrays (ARMON_FIELD_*).
+void launch_batch_init(const BatchInit* domains, int n, int64_t elements, double* const arrays[ARMON_FIELD_COUNT],
+                       hipStream_t s);
+
 // Work items: an X tile (domain; row and slot within that row of the tile's first thread,
 // see sweep_x_tile) or a Y run of one wave (domain, first column, output rows [y0, y1)).
 struct BatchItemX { int domain, row, slot, pad; };
