@@ -174,16 +174,21 @@ constexpr int kBlock = 256;
 // 64-element pieces of `ref` (the array the kernel streams) start on 128-byte lines: a row of
 // the reference layout starts anywhere in a line (its ghost cells come first), and unaligned
 // pieces touch 5 lines instead of 4 (measured on 7-stream kernels: 8% slower). The grid has
-// kAlignSlack more columns than the row (grid_2d).
+// kAlignSlack more columns than the row (grid_2d). The kernels that run down columns shift those of
+// a run by its first row (4096^2, us: second-order advection 279 -> 262, GAD 179 -> 175).
 constexpr int kAlignSlack = 15;
+
+__device__ __forceinline__ int64_t line_shift(const void* ref, int64_t index)
+{
+    return (int64_t) (((uintptr_t) ref / sizeof(flt_t) + (uint64_t) index) & kAlignSlack);
+}
 
 template <class F>
 __device__ __forceinline__ void for_each_2d(const Iter2D& it, const void* ref, F&& f)
 {
     for (int64_t row = it.first_row + blockIdx.y; row <= it.last_row; row += gridDim.y) {
         const int64_t row0 = it.base + row * it.step;    // index of column 0
-        const int64_t shift = (int64_t) (((uintptr_t) ref / sizeof(flt_t) + (uint64_t) row0) & kAlignSlack);
-        const int64_t col = (int64_t) blockIdx.x * blockDim.x + threadIdx.x - shift;
+        const int64_t col = (int64_t) blockIdx.x * blockDim.x + threadIdx.x - line_shift(ref, row0);
         if (col < 0 || col >= it.len) continue;
         const int64_t k = row * it.len + col;
         if (k < it.start || k >= it.end) continue;
@@ -316,14 +321,15 @@ __global__ void __launch_bounds__(kBlock) k_acoustic_GAD_y(Iter2D it, int64_t ru
                                                            const flt_t* __restrict__ pmat,
                                                            const flt_t* __restrict__ cmat)
 {
-    const int64_t col = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= it.len) return;
-    // rows of this column in the range: [r_lo, r_hi]
-    const int64_t r_lo = it.first_row + (col < it.start - it.first_row * it.len ? 1 : 0);
-    const int64_t r_hi = it.last_row - (col > it.end - 1 - it.last_row * it.len ? 1 : 0);
     const int64_t s = it.step;
     const int64_t nruns = (it.last_row - it.first_row + run) / run;
     for (int64_t k = blockIdx.y; k < nruns; k += gridDim.y) {
+        const int64_t col = (int64_t) blockIdx.x * blockDim.x + threadIdx.x -
+                            line_shift(rho, it.base + (it.first_row + k * run) * s);
+        if (col < 0 || col >= it.len) continue;
+        // rows of this column in the range: [r_lo, r_hi]
+        const int64_t r_lo = it.first_row + (col < it.start - it.first_row * it.len ? 1 : 0);
+        const int64_t r_hi = it.last_row - (col > it.end - 1 - it.last_row * it.len ? 1 : 0);
         const int64_t ra = max(it.first_row + k * run, r_lo);
         const int64_t rb = min(it.first_row + (k + 1) * run - 1, r_hi);
         if (ra > rb) continue;
@@ -543,14 +549,15 @@ __global__ void __launch_bounds__(kBlock) k_advection_second_order_y(Iter2D it, 
                                                                     flt_t* __restrict__ a_vrho,
                                                                     flt_t* __restrict__ a_Erho)
 {
-    const int64_t col = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= it.len) return;
-    // rows of this column in the range: [r_lo, r_hi]
-    const int64_t r_lo = it.first_row + (col < it.start - it.first_row * it.len ? 1 : 0);
-    const int64_t r_hi = it.last_row - (col > it.end - 1 - it.last_row * it.len ? 1 : 0);
     const int64_t s = it.step;
     const int64_t nruns = (it.last_row - it.first_row + run) / run;
     for (int64_t k = blockIdx.y; k < nruns; k += gridDim.y) {
+        const int64_t col = (int64_t) blockIdx.x * blockDim.x + threadIdx.x -
+                            line_shift(rho, it.base + (it.first_row + k * run) * s);
+        if (col < 0 || col >= it.len) continue;
+        // rows of this column in the range: [r_lo, r_hi]
+        const int64_t r_lo = it.first_row + (col < it.start - it.first_row * it.len ? 1 : 0);
+        const int64_t r_hi = it.last_row - (col > it.end - 1 - it.last_row * it.len ? 1 : 0);
         const int64_t ra = max(it.first_row + k * run, r_lo);
         const int64_t rb = min(it.first_row + (k + 1) * run - 1, r_hi);
         if (ra > rb) continue;
@@ -1076,7 +1083,7 @@ ARMON_KERNEL_TRY
             const int64_t groups = (it.len + 63) / 64;
             if (groups * ((rows + run - 1) / run) < 8192) run = 4;
             const int64_t nruns = (rows + run - 1) / run;
-            const dim3 g((unsigned) ((it.len + kBlock - 1) / kBlock), (unsigned) (nruns < 65535 ? nruns : 65535));
+            const dim3 g((unsigned) ((it.len + kAlignSlack + kBlock - 1) / kBlock), (unsigned) (nruns < 65535 ? nruns : 65535));
             k_acoustic_GAD_y<LL><<<g, kBlock, 0, stream()>>>(it, run, dt, dx, ustar.data, pstar.data, rho.data,
                                                              u.data, pmat.data, cmat.data);
         } else {
@@ -1256,7 +1263,7 @@ ARMON_KERNEL_TRY
         const int64_t groups = (it.len + 63) / 64;
         if (groups * ((rows + run - 1) / run) < 8192) run = 4;
         const int64_t nruns = (rows + run - 1) / run;
-        const dim3 g((unsigned) ((it.len + kBlock - 1) / kBlock), (unsigned) (nruns < 65535 ? nruns : 65535));
+        const dim3 g((unsigned) ((it.len + kAlignSlack + kBlock - 1) / kBlock), (unsigned) (nruns < 65535 ? nruns : 65535));
         k_advection_second_order_y<<<g, kBlock, 0, stream()>>>(it, run, dx, dt, ustar.data, rho.data, umat.data,
                                                                vmat.data, Emat.data, advection_rho.data,
                                                                advection_urho.data, advection_vrho.data,
