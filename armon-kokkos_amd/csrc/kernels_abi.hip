@@ -175,7 +175,7 @@ constexpr int kBlock = 256;
 // the reference layout starts anywhere in a line (its ghost cells come first), and unaligned
 // pieces touch 5 lines instead of 4 (measured on 7-stream kernels: 8% slower). The grid has
 // kAlignSlack more columns than the row (grid_2d). The kernels that run down columns shift those of
-// a run by its first row (4096^2, us: second-order advection 279 -> 262, GAD 179 -> 175).
+// a run by its first row (run_slack).
 constexpr int kAlignSlack = 15;
 
 __device__ __forceinline__ int64_t line_shift(const void* ref, int64_t index)
@@ -210,6 +210,20 @@ dim3 grid_2d_aligned(const Iter2D& it)
     const int64_t rows = it.last_row - it.first_row + 1;
     const int64_t gx = (it.len + kAlignSlack + kBlock - 1) / kBlock;
     return dim3((unsigned) gx, (unsigned) (rows < 65535 ? rows : 65535), 1);
+}
+
+// How far the kernels that run down columns may shift a run's columns to start on a line: kAlignSlack, or 0
+// for not at all. Aligned, the second-order advection and the GAD fluxes take 11% and 5% less time at
+// 5000^2 (416 -> 368, 263 -> 250 us). Where the row is so close to a whole number of blocks that the shift
+// adds a column of blocks, its cost decides, and with 8 k block columns unshifted the runs above each
+// other share an XCD's L2: advection 1024^2 16.9 -> 17.9, 2048^2 65.5 -> 66.2, 3072^2 161 -> 153, 4096^2
+// 274 -> 254, 6144^2 600 -> 553, 8192^2 1040 -> 1108 us, so from 12 to 24 block columns; GAD 14.6 -> 15.4,
+// 44.6 -> 42.3, 103.5 -> 102.8, 173 -> 169, 380 -> 395, 662 -> 661 us: not.
+int run_slack(int64_t len, bool advection)
+{
+    const int64_t blocks = (len + kBlock - 1) / kBlock;
+    const bool free = (len + kAlignSlack + kBlock - 1) / kBlock == blocks;
+    return free || (advection && blocks >= 12 && blocks <= 24) ? kAlignSlack : 0;
 }
 
 dim3 grid_1d(const Iter1D& it)
@@ -315,7 +329,7 @@ __global__ void __launch_bounds__(kGadTile) k_acoustic_GAD_x(Iter2D it, flt_t dt
 }
 
 template <int L>
-__global__ void __launch_bounds__(kBlock) k_acoustic_GAD_y(Iter2D it, int64_t run, flt_t dt, flt_t dx,
+__global__ void __launch_bounds__(kBlock) k_acoustic_GAD_y(Iter2D it, int64_t run, int slack, flt_t dt, flt_t dx,
                                                            flt_t* __restrict__ ustar, flt_t* __restrict__ pstar,
                                                            const flt_t* __restrict__ rho, const flt_t* __restrict__ u,
                                                            const flt_t* __restrict__ pmat,
@@ -325,7 +339,7 @@ __global__ void __launch_bounds__(kBlock) k_acoustic_GAD_y(Iter2D it, int64_t ru
     const int64_t nruns = (it.last_row - it.first_row + run) / run;
     for (int64_t k = blockIdx.y; k < nruns; k += gridDim.y) {
         const int64_t col = (int64_t) blockIdx.x * blockDim.x + threadIdx.x -
-                            line_shift(rho, it.base + (it.first_row + k * run) * s);
+                            (line_shift(rho, it.base + (it.first_row + k * run) * s) & slack);
         if (col < 0 || col >= it.len) continue;
         // rows of this column in the range: [r_lo, r_hi]
         const int64_t r_lo = it.first_row + (col < it.start - it.first_row * it.len ? 1 : 0);
@@ -538,7 +552,7 @@ __global__ void __launch_bounds__(kAdvTile) k_advection_second_order_x(Iter2D it
     }
 }
 
-__global__ void __launch_bounds__(kBlock) k_advection_second_order_y(Iter2D it, int64_t run, flt_t dx, flt_t dt,
+__global__ void __launch_bounds__(kBlock) k_advection_second_order_y(Iter2D it, int64_t run, int slack, flt_t dx, flt_t dt,
                                                                     const flt_t* __restrict__ ustar,
                                                                     const flt_t* __restrict__ rho,
                                                                     const flt_t* __restrict__ umat,
@@ -553,7 +567,7 @@ __global__ void __launch_bounds__(kBlock) k_advection_second_order_y(Iter2D it, 
     const int64_t nruns = (it.last_row - it.first_row + run) / run;
     for (int64_t k = blockIdx.y; k < nruns; k += gridDim.y) {
         const int64_t col = (int64_t) blockIdx.x * blockDim.x + threadIdx.x -
-                            line_shift(rho, it.base + (it.first_row + k * run) * s);
+                            (line_shift(rho, it.base + (it.first_row + k * run) * s) & slack);
         if (col < 0 || col >= it.len) continue;
         // rows of this column in the range: [r_lo, r_hi]
         const int64_t r_lo = it.first_row + (col < it.start - it.first_row * it.len ? 1 : 0);
@@ -1083,8 +1097,9 @@ ARMON_KERNEL_TRY
             const int64_t groups = (it.len + 63) / 64;
             if (groups * ((rows + run - 1) / run) < 8192) run = 4;
             const int64_t nruns = (rows + run - 1) / run;
-            const dim3 g((unsigned) ((it.len + kAlignSlack + kBlock - 1) / kBlock), (unsigned) (nruns < 65535 ? nruns : 65535));
-            k_acoustic_GAD_y<LL><<<g, kBlock, 0, stream()>>>(it, run, dt, dx, ustar.data, pstar.data, rho.data,
+            const int slack = run_slack(it.len, false);
+            const dim3 g((unsigned) ((it.len + slack + kBlock - 1) / kBlock), (unsigned) (nruns < 65535 ? nruns : 65535));
+            k_acoustic_GAD_y<LL><<<g, kBlock, 0, stream()>>>(it, run, slack, dt, dx, ustar.data, pstar.data, rho.data,
                                                              u.data, pmat.data, cmat.data);
         } else {
             k_acoustic_GAD<LL><<<grid_2d_aligned(it), kBlock, 0, stream()>>>(it, s, dt, dx, ustar.data, pstar.data, rho.data,
@@ -1263,8 +1278,9 @@ ARMON_KERNEL_TRY
         const int64_t groups = (it.len + 63) / 64;
         if (groups * ((rows + run - 1) / run) < 8192) run = 4;
         const int64_t nruns = (rows + run - 1) / run;
-        const dim3 g((unsigned) ((it.len + kAlignSlack + kBlock - 1) / kBlock), (unsigned) (nruns < 65535 ? nruns : 65535));
-        k_advection_second_order_y<<<g, kBlock, 0, stream()>>>(it, run, dx, dt, ustar.data, rho.data, umat.data,
+        const int slack = run_slack(it.len, true);
+        const dim3 g((unsigned) ((it.len + slack + kBlock - 1) / kBlock), (unsigned) (nruns < 65535 ? nruns : 65535));
+        k_advection_second_order_y<<<g, kBlock, 0, stream()>>>(it, run, slack, dx, dt, ustar.data, rho.data, umat.data,
                                                                vmat.data, Emat.data, advection_rho.data,
                                                                advection_urho.data, advection_vrho.data,
                                                                advection_Erho.data);
