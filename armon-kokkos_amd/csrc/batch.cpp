@@ -737,9 +737,9 @@ ARMON_EXPORT int armon_batch_run(ArmonBatch* b)
     try {
         if (!b->begun || b->finished) throw invalid_argument("armon_batch_begin must come first");
         const int chunk = b->common.graph_chunk > 0 ? b->common.graph_chunk : 16;
-        run_chunks(b->reports, chunk, b->stream,
-                   [&] {
-                       advance(b, chunk);
+        run_chunks(b->reports, chunk, b->real_cells, b->stream,
+                   [&](int64_t n) {
+                       advance(b, n);
                        return last_states(b);
                    },
                    [&](int d) { return step_config(b->p[d]); });

@@ -1162,9 +1162,9 @@ ARMON_EXPORT int armon_solver_time_loop(ArmonSolver* s, ArmonResult* out)
         try {
             const int chunk = p.graph_chunk > 0 ? p.graph_chunk : 16;
             if (p.verbose > 1) {
-                run_chunks(s->reports, chunk, s->stream,
-                           [&] {
-                               fused_advance(s, chunk);
+                run_chunks(s->reports, chunk, (int64_t) p.nx * p.ny, s->stream,
+                           [&](int64_t n) {
+                               fused_advance(s, n);
                                return last_state(s);
                            },
                            [&](int) { return step_config(p); });

@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 namespace armon {
@@ -36,10 +37,14 @@ struct StepState {
     int error_cycle;
 
     bool running() const { return active && !error; }
-    // Whether more cycles follow after `n` of this state's time step.
-    bool runs_on(const TimeStepConfig& c, int n) const
+    // How many cycles are left: 0 when the run has ended, else by the count of cycles, or by the time at
+    // this state's time step and one or two more.
+    int64_t left(const TimeStepConfig& c) const
     {
-        return running() && (int64_t) cycle + n < c.max_cycles && time + n * current_dt < c.max_time;
+        if (!running() || !(time < c.max_time) || cycle >= c.max_cycles) return 0;
+        const int64_t count = (int64_t) c.max_cycles - cycle;
+        const double steps = (c.max_time - time) / current_dt;
+        return steps < (double) count ? std::min(count, (int64_t) steps + 2) : count;
     }
 };
 
@@ -236,29 +241,47 @@ private:
     int n_ = 0;
 };
 
-// Runs chunks of `chunk` cycles until no state is running. `enqueue()` enqueues a chunk and returns the
-// states after it; `config(d)` is the configuration of state d.
+// Runs chunks of up to `chunk` cycles until no state is running. `enqueue(n)` enqueues n cycles and returns
+// the states after them; `config(d)` is the configuration of state d.
 //
 // The host learns of a chunk's end a report's round trip later, 20-30 us in which the device would idle
-// (a quarter of a chunk of a 100^2 domain's cycles). So while chunk k runs, chunk k + 1 is enqueued
-// behind it, unless the report of chunk k - 1 says that chunk k will be the last: by the number of
-// cycles left, or by the time left at that report's time step. The guess costs nothing but time
-// where it is wrong: cycles after the end change no state (2 us a launch), and a chunk that was not
-// enqueued ahead is enqueued as soon as its turn is known.
+// (a quarter of a chunk of a 100^2 domain's cycles). So while one chunk runs, the next is enqueued
+// behind it, unless the report before it says that no cycle will be left. Where that guess is wrong,
+// as the time step changes, the run takes a little longer.
+//
+// Cycles after the end change no state, and in small domains whole chunks, each one graph, are the
+// fastest. A large domain's blocks take their time to come and go all the same, 1.2 ns each (an X sweep
+// of 8192^2 160 us, 1.9 ms of a run of 100 cycles in chunks of 16): from kWholeChunks `cells` on, no
+// more cycles are enqueued than the report leaves, the rest of a chunk launch by launch.
+constexpr int64_t kWholeChunks = 1 << 22;
+
 template <class Enqueue, class Config>
-void run_chunks(StateReports& reports, int chunk, hipStream_t s, Enqueue&& enqueue, Config&& config)
+void run_chunks(StateReports& reports, int chunk, int64_t cells, hipStream_t s, Enqueue&& enqueue, Config&& config)
 {
-    const StepState* known = nullptr;   // the report before the newest one
-    reports.post(enqueue(), 0, s);
-    for (int k = 0;; k = (k + 1) & 1) {
-        bool ahead = false;
-        for (int d = 0; known && !ahead && d < reports.size(); d++) ahead = known[d].runs_on(config(d), chunk);
-        if (ahead) reports.post(enqueue(), k ^ 1, s);
+    const int64_t least = cells < kWholeChunks ? chunk : 1;
+    auto left = [&](const StepState* states) {
+        int64_t most = 0;
+        for (int d = 0; d < reports.size(); d++) most = std::max(most, states[d].left(config(d)));
+        return most;
+    };
+    int64_t cycles = least;   // of the chunk that runs
+    for (int d = 0; d < reports.size(); d++) cycles = std::max<int64_t>(cycles, config(d).max_cycles);
+    cycles = std::min<int64_t>(cycles, chunk);
+    const StepState* known = nullptr;   // the report before the chunk that runs
+    reports.post(enqueue(cycles), 0, s);
+    for (int k = 0;; k ^= 1) {
+        int64_t next = known ? left(known) - cycles : 0;
+        const bool ahead = next > 0;
+        next = std::clamp<int64_t>(next, least, chunk);
+        if (ahead) reports.post(enqueue(next), k ^ 1, s);
         known = reports.wait(k);
-        bool any = false;
-        for (int d = 0; d < reports.size(); d++) any = any || known[d].runs_on(config(d), 0);
-        if (!any) return;
-        if (!ahead) reports.post(enqueue(), k ^ 1, s);
+        const int64_t more = left(known);
+        if (more == 0) return;
+        if (!ahead) {
+            next = std::clamp<int64_t>(more, least, chunk);
+            reports.post(enqueue(next), k ^ 1, s);
+        }
+        cycles = next;
     }
 }
 
