@@ -519,7 +519,7 @@ ARMON_EXPORT ArmonBatch* armon_batch_create(const ArmonParams* common, int n, co
         b->d_init = device_alloc<BatchInit>(n, "hipMalloc(initial states)");
         b->d_states = device_alloc<DeviceState>(2 * (size_t) n, "hipMalloc(states)");
         b->d_tune = device_alloc<DeviceState>(n, "hipMalloc(tune states)");
-        b->reports.create(n);
+        b->reports.resize(n);
         hip_check(hipMemcpy(b->d_domains, dom.data(), sizeof(BatchDomain) * n, hipMemcpyHostToDevice), "upload domains");
         hip_check(hipMemcpy(b->d_cfgs, cfg.data(), sizeof(TimeStepConfig) * n, hipMemcpyHostToDevice), "upload configs");
         hip_check(hipMemcpy(b->d_init, init.data(), sizeof(BatchInit) * n, hipMemcpyHostToDevice), "upload initial states");

@@ -985,7 +985,7 @@ ARMON_EXPORT ArmonSolver* armon_solver_create(const ArmonParams* params)
         void* st = nullptr;
         hip_check(hipMalloc(&st, 2 * sizeof(DeviceState)), "hipMalloc(states)");
         s->st = static_cast<DeviceState*>(st);
-        s->reports.create(1);
+        s->reports.resize(1);
         if (s->p.engine == ARMON_ENGINE_FUSED && s->p.precision == ARMON_PREC_FP32_MIXED) {
             for (int k = 0; k < 10; k++) {
                 void* ptr = nullptr;

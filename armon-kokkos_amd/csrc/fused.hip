@@ -216,18 +216,15 @@ StateReports::~StateReports()
     if (host_) (void) hipHostFree(host_);
 }
 
-void StateReports::create(int n)
-{
-    void* p = nullptr;
-    hip_check(hipHostMalloc(&p, 2 * sizeof(StepState) * (size_t) n, hipHostMallocDefault), "hipHostMalloc(reports)");
-    host_ = static_cast<StepState*>(p);
-    n_ = n;
-    for (hipEvent_t& e : arrived_)
-        hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
-}
-
 void StateReports::post(const DeviceState* states, int k, hipStream_t s)
 {
+    if (!host_) {
+        for (hipEvent_t& e : arrived_)
+            if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+        void* p = nullptr;
+        hip_check(hipHostMalloc(&p, 2 * sizeof(StepState) * (size_t) n_, hipHostMallocDefault), "hipHostMalloc(reports)");
+        host_ = static_cast<StepState*>(p);
+    }
     launch_report(states, n_, host_ + (k & 1) * (size_t) n_, s);
     hip_check(hipEventRecord(arrived_[k & 1], s), "hipEventRecord");
 }

@@ -221,14 +221,14 @@ void launch_clear(DeviceState* states, int n, hipStream_t s);
 void launch_report(const DeviceState* states, int n, StepState* out, hipStream_t s);
 
 // Reports of n states in pinned memory that the device writes: two, so that the host reads one while
-// the other is on its way. Whoever holds it calls create() once and uses it from one stream.
+// the other is on its way. Made with the first report; used from one stream.
 class StateReports {
 public:
     StateReports() = default;
     StateReports(const StateReports&) = delete;
     StateReports& operator=(const StateReports&) = delete;
     ~StateReports();
-    void create(int n);
+    void resize(int n) { n_ = n; }   // before the first report
     int size() const { return n_; }
     // Enqueues report k (the one in the place of report k - 2).
     void post(const DeviceState* states, int k, hipStream_t s);
