@@ -38,13 +38,14 @@ struct StepState {
 
     bool running() const { return active && !error; }
     // How many cycles are left: 0 when the run has ended, else by the count of cycles, or by the time at
-    // this state's time step and one or two more.
+    // this state's time step and one or two more. A time step that does not lead to the end (a
+    // constant one may be negative) leaves all of the count.
     int64_t left(const TimeStepConfig& c) const
     {
         if (!running() || !(time < c.max_time) || cycle >= c.max_cycles) return 0;
         const int64_t count = (int64_t) c.max_cycles - cycle;
         const double steps = (c.max_time - time) / current_dt;
-        return steps < (double) count ? std::min(count, (int64_t) steps + 2) : count;
+        return steps >= 0 && steps < (double) count ? std::min(count, (int64_t) steps + 2) : count;
     }
 };
 
