@@ -53,10 +53,13 @@ inline void boundary_factors(const ArmonParams& p, int side, double* uf, double*
 // Library-owned device scratch (reduction partials and scalars), one per device,
 // allocated on first use and kept until the process ends.
 struct Scratch {
-    double* partials = nullptr;       // reduction partials, kPartials entries
+    double* partials = nullptr;       // partial sums of conservation_vars, kPartials entries
+    // Block minima of the CFL bound, kMinima entries: dt_CFL_device returns before they are read, and a
+    // conservation_vars on another stream must not write where they lie.
+    unsigned long long* minima = nullptr;
     double* result = nullptr;         // final results (up to 8 doubles), in pinned host memory that the
                                       // device writes: no copy after the reduction
-    static constexpr int kPartials = 4 * 1024;
+    static constexpr int kPartials = 4 * 1024, kMinima = 1024;
 };
 Scratch& scratch();
 

@@ -73,11 +73,12 @@ Scratch& scratch()
     if (!s.partials) {
         void* p = nullptr;
         void* h = nullptr;
-        hip_check(hipMalloc(&p, sizeof(double) * Scratch::kPartials), "hipMalloc(scratch)");
+        hip_check(hipMalloc(&p, sizeof(double) * (Scratch::kPartials + Scratch::kMinima)), "hipMalloc(scratch)");
         hipError_t e = hipHostMalloc(&h, sizeof(double) * 8, hipHostMallocMapped);
         if (e != hipSuccess) (void) hipFree(p);
         hip_check(e, "hipHostMalloc(scratch)");
         s.partials = static_cast<double*>(p);
+        s.minima = reinterpret_cast<unsigned long long*>(s.partials + Scratch::kPartials);
         s.result = static_cast<double*>(h);
     }
     return s;
@@ -842,6 +843,7 @@ __global__ void __launch_bounds__(kBlock) k_batch_init(const armon::BatchInit* _
 // ---- reductions -------------------------------------------------------------------------
 
 constexpr int kRedBlocks = 1024;
+static_assert(kRedBlocks <= Scratch::kMinima && 4 * kRedBlocks <= Scratch::kPartials);
 
 __device__ __forceinline__ double wave_min(double v)
 {
@@ -1496,16 +1498,15 @@ static void launch_dt_CFL(const Range& range, const InnerRange1D& inner_range, f
     check_view(domain_mask, "domain_mask", sp);
     Scratch& sc = armon::scratch();
     const double init = (sizeof(flt_t) == 8) ? DBL_MAX : (double) FLT_MAX;
-    auto* minima = reinterpret_cast<unsigned long long*>(sc.partials);
     int64_t g = 0;
     if (!empty_1d(it)) {
         g = (it.end - it.start + kBlock - 1) / kBlock;
         if (g > kRedBlocks) g = kRedBlocks;
         k_dt_CFL<<<(unsigned) g, kBlock, 0, stream()>>>(it, dx, dy, umat.data, vmat.data, cmat.data, domain_mask.data,
-                                                         minima);
+                                                         sc.minima);
         after_launch("dt_CFL");
     }
-    k_dt_final<<<1, kBlock, 0, stream()>>>(minima, (int) g, init, dt_device);
+    k_dt_final<<<1, kBlock, 0, stream()>>>(sc.minima, (int) g, init, dt_device);
     after_launch("dt_CFL(result)");
 }
 

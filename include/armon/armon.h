@@ -52,7 +52,8 @@ ARMON_EXPORT const char* armon_version(void);
 /* ---- device-resident CFL reduction -------------------------------------- */
 
 /* Same reduction as dt_CFL (reductions.cpp:8-24) but asynchronous: the minimum is
- * written to *dt_device (a device address) on the library stream. */
+ * written to *dt_device (a device address) on the library stream. Calls of dt_CFL and dt_CFL_device
+ * that overlap on one device (on different streams) share the library's block minima and race. */
 ARMON_EXPORT void dt_CFL_device(ARMON_CREF(Range) range, ARMON_CREF(InnerRange1D) inner_range, flt_t dx, flt_t dy,
                                 ARMON_CREF(view) umat, ARMON_CREF(view) vmat, ARMON_CREF(view) cmat,
                                 ARMON_CREF(mask_view) domain_mask, double* dt_device);
