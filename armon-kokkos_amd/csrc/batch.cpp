@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -52,6 +53,9 @@ T* device_alloc(size_t count, const char* what)
 
 }  // namespace
 
+// The field fills a gap before the doubles: the struct keeps its size and the other fields their places.
+static_assert(offsetof(ArmonBatchTuning, ms_x) == 24 && sizeof(ArmonBatchTuning) == 48);
+
 struct ArmonBatch {
     ArmonParams common{};
     std::vector<ArmonParams> p;          // per domain, through armon_params_init
@@ -72,7 +76,6 @@ struct ArmonBatch {
     BatchItemX* d_items_x = nullptr;
     BatchItemY* d_items_y = nullptr;
     ArmonBatchTuning tuning{};
-    bool y_tiles = false;                // the Y items are LDS tiles, not the tuning's marching runs
     SweepVariant var{};
     int sweeps_per_cycle = 2;
     int64_t cycles_enqueued = 0;
@@ -154,7 +157,7 @@ void build_items(ArmonBatch* b, int run)
             const int64_t s0 = t * W;
             b->items_x.push_back(BatchItemX{d, (int) (s0 / slots), (int) (s0 % slots), 0});
         }
-        if (b->y_tiles) {
+        if (b->tuning.y_tiles) {
             const int rows = y_tile_outputs(b->var);
             for (int y0 = 0; y0 < q.ny; y0 += rows)
                 for (int x0 = 0; x0 < q.nx; x0 += y_tile_cols()) b->items_y.push_back(BatchItemY{d, x0, y0, 0});
@@ -239,7 +242,7 @@ void launch_one_sweep(ArmonBatch* b, int axis, int parity, double factor, bool r
     const void* items = x ? (const void*) b->d_items_x : (const void*) b->d_items_y;
     const int nitems = x ? (int) b->items_x.size() : (int) b->items_y.size();
     const int grid = x ? blocks_x(b, b->tuning.grid_x) : blocks_y(b, b->tuning.grid_y);
-    const int tile = x ? b->tuning.tile_x : b->y_tiles ? 1 : 0;
+    const int tile = x ? b->tuning.tile_x : b->tuning.y_tiles ? 1 : 0;
     if (b->fp64())
         launch_batch_sweep<double>(axis, b->var, batch_args<double>(b, parity, factor, reduce, states, prev), items,
                                    nitems, grid, tile, b->tuning.x_cells_per_thread, b->stream);
@@ -285,7 +288,7 @@ void enqueue_cycle(ArmonBatch* b, int64_t cycle, Timer* t)
     double factors[3];
     const int n = armon_split_axes(&pc, axes, factors);
     // the first sweep makes the time step where each of its blocks has one item
-    const bool single = axes[0] == ARMON_AXIS_X ? b->tuning.grid_x == 0 : b->y_tiles;
+    const bool single = axes[0] == ARMON_AXIS_X ? b->tuning.grid_x == 0 : b->tuning.y_tiles != 0;
     const bool folded = n > 1 && single && b->real_cells <= folded_cells(b->fp64() ? 8 : 4);
     if (t) t->begin();
     if (!folded) launch_batch_time_step(prev, states, b->d_cfgs, (int) b->p.size(), b->stream);
@@ -525,7 +528,7 @@ ARMON_EXPORT ArmonBatch* armon_batch_create(const ArmonParams* common, int n, co
         hip_check(hipMemcpy(b->d_init, init.data(), sizeof(BatchInit) * n, hipMemcpyHostToDevice), "upload initial states");
         // default configuration: 256-cell X tiles of one cell per thread, Y tiles or 256-row Y runs by
         // the number of cells, one block per work item
-        b->y_tiles = b->real_cells <= y_tile_max_cells(b->fp64() ? 8 : 4);
+        b->tuning.y_tiles = b->real_cells <= y_tile_max_cells(b->fp64() ? 8 : 4);
         b->tuning.tile_x = 256;
         b->tuning.x_cells_per_thread = 1;
         b->tuning.grid_x = 0;
@@ -591,7 +594,7 @@ ARMON_EXPORT int armon_batch_set_tuning(ArmonBatch* b, const ArmonBatchTuning* t
         b->tuning.x_cells_per_thread = cpt;
         b->tuning.grid_x = std::max(0, t->grid_x);
         b->tuning.grid_y = std::max(0, t->grid_y);
-        b->y_tiles = false;
+        b->tuning.y_tiles = t->y_tiles != 0;
         build_items(b, t->y_run_rows);
         return 0;
     } catch (const std::exception& e) {
@@ -624,7 +627,7 @@ ARMON_EXPORT int armon_batch_autotune(ArmonBatch* b, ArmonBatchTuning* out)
         // X: tile width (128, 256, 512 cells, one per thread) x (persistent grids of 1, 2, 4
         // resident rounds | one block per tile), then tiles of 256 and 512 cells at two cells
         // per thread (one block per tile)
-        b->y_tiles = false;
+        b->tuning.y_tiles = 0;
         double best_x = 1e300;
         int grid_x = 0, tile_x = 256, cpt_x = 1;
         const int run0 = b->tuning.y_run_rows;
@@ -664,15 +667,15 @@ ARMON_EXPORT int armon_batch_autotune(ArmonBatch* b, ArmonBatchTuning* out)
                 if (ms < best_y) { best_y = ms; grid_y = g; run_y = run; }
             }
         }
-        // Y tiles beside the marches: the fastest march stays in the tuning, for a batch that takes it
-        b->y_tiles = true;
+        // Y tiles beside the marches: the fastest march stays in the tuning, for set_tuning without y_tiles
+        b->tuning.y_tiles = 1;
         build_items(b, run_y);
         const double ms_tiles = time_sweep(b, ARMON_AXIS_Y, reps);
         b->tuning.grid_y = grid_y;
         if (ms_tiles < best_y) {
             best_y = ms_tiles;
         } else {
-            b->y_tiles = false;
+            b->tuning.y_tiles = 0;
             build_items(b, run_y);
         }
         b->tuning.ms_x = best_x;

@@ -254,7 +254,7 @@ ARMON_EXPORT int armon_run(ArmonParams* p, ArmonResult* out);
 
 /* ---- batched ensemble ------------------------------------------------------
  * Many independent domains of different sizes advanced together: every sweep of a cycle
- * is ONE persistent launch over the work items (row tiles for X, column runs for Y) of all
+ * is ONE launch over the work items (row tiles for X, column runs or tiles for Y) of all
  * domains, each domain with its own dt, time, cycle count and end time, all on the device;
  * cycles are replayed from a captured hipGraph. Each domain follows exactly the reference
  * time loop (armon_2D.cpp:327-386) on its own parameters, so a domain's result is the
@@ -279,11 +279,14 @@ ARMON_EXPORT int armon_batch_random_specs(uint64_t seed, int n, int64_t min_area
 /* Launch configuration of the batched sweeps, chosen by armon_batch_autotune: the tile shape
  * and the cells each thread computes (an X tile is tile_x cells along a row, computed by
  * tile_x / x_cells_per_thread threads; a Y item is a wave of 64 columns, each thread marching
- * y_run_rows cells down its column) and the launch grids. */
+ * y_run_rows cells down its column, or with y_tiles an LDS tile of 16 columns x 32 rows) and the
+ * launch grids. A batch of up to a few million cells starts with y_tiles. */
 typedef struct ArmonBatchTuning {
-    int y_run_rows;           /* rows a wave marches per Y work item (64 columns wide) */
-    int grid_x, grid_y;       /* blocks of the X and Y launches (persistent when below the item count) */
+    int y_run_rows;           /* rows a wave marches per Y work item (64 columns wide); > 0, not used with y_tiles */
+    int grid_x, grid_y;       /* blocks of the X and Y launches (persistent when below the item count; Y tiles:
+                                 always one block each) */
     int items_x, items_y;     /* work items per X / Y sweep (outputs) */
+    int y_tiles;              /* nonzero: the Y items are tiles, else marches */
     double ms_x, ms_y;        /* measured time per X / Y sweep of this configuration (autotune output) */
     int tile_x;               /* cells per X tile: 128, 256 or 512 (0 in set_tuning: 256) */
     int x_cells_per_thread;   /* cells per thread of the X tile: 1, or 2 for tiles of 256 or 512 cells
@@ -305,10 +308,11 @@ ARMON_EXPORT void* armon_batch_stream(ArmonBatch* b);
 /* init_test_states of every domain (armon_2D.cpp:112-127). */
 ARMON_EXPORT int armon_batch_init(ArmonBatch* b);
 /* Times the sweeps over the initial state for the candidate configurations (X tile width, Y
- * run length, persistent or one-block-per-item grids) and keeps the fastest. After init, before
- * begin. */
+ * run length or Y tiles, persistent or one-block-per-item grids) and keeps the fastest. After init,
+ * before begin. */
 ARMON_EXPORT int armon_batch_autotune(ArmonBatch* b, ArmonBatchTuning* out);
-/* Sets the configuration by hand (grid_x/grid_y <= 0: one block per item); before begin. */
+/* Sets the configuration by hand (grid_x/grid_y <= 0: one block per item), or again as
+ * armon_batch_get_tuning or armon_batch_autotune returned it; before begin. */
 ARMON_EXPORT int armon_batch_set_tuning(ArmonBatch* b, const ArmonBatchTuning* t);
 ARMON_EXPORT int armon_batch_get_tuning(const ArmonBatch* b, ArmonBatchTuning* out);
 ARMON_EXPORT int armon_batch_begin(ArmonBatch* b);
