@@ -79,6 +79,7 @@ struct ArmonBatch {
     SweepVariant var{};
     int sweeps_per_cycle = 2;
     int64_t cycles_enqueued = 0;
+    int64_t ended_at = -1;               // cycles_enqueued when armon_batch_run found no domain left to run
     hipStream_t stream = nullptr;
     hipGraphExec_t graph[2] = {};        // graph_chunk cycles from an even (0) or odd (1) cycle
     hipGraph_t graph_def[2] = {};
@@ -696,6 +697,7 @@ ARMON_EXPORT int armon_batch_begin(ArmonBatch* b)
         check_ready(b, true, true);
         begin_fields(b, b->d_states);
         b->cycles_enqueued = 0;
+        b->ended_at = -1;
         // both graphs now, so that no later advance pays for a capture
         if (b->common.graph_chunk > 0)
             for (int parity = 0; parity < 2; parity++)
@@ -727,6 +729,8 @@ ARMON_EXPORT int armon_batch_active(ArmonBatch* b)
         int k = 0;
         b->reports.post(last_states(b), 0, b->stream);
         const StepState* s = b->reports.wait(0);
+        // a run ends without a cycle after the last, so its states are those of cycles that ran
+        if (b->cycles_enqueued == b->ended_at) return 0;
         for (int d = 0; d < b->reports.size(); d++) k += s[d].running();
         return k;
     } catch (const std::exception& e) {
@@ -746,6 +750,7 @@ ARMON_EXPORT int armon_batch_run(ArmonBatch* b)
                        return last_states(b);
                    },
                    [&](int d) { return step_config(b->p[d]); });
+        b->ended_at = b->cycles_enqueued;
         return 0;
     } catch (const std::exception& e) {
         fail("armon_batch_run", e);

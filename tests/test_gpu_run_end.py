@@ -35,3 +35,33 @@ def test_batch_with_a_negative_constant_time_step_runs_every_cycle(armon):
     assert b.finish() == 0, armon.errors()
     assert [b.result(d).cycles for d in range(b.n)] == [40] * 3
     b.close()
+
+
+# 16 and 32 cycles are whole chunks; 4.2 M cells enqueue no more cycles than are left
+@pytest.mark.gpu
+@pytest.mark.parametrize("cycles", [1, 16, 20, 32])
+@pytest.mark.parametrize("areas", [(16 * 16, 32 * 32), (2060 * 2060, 2070 * 2070)])
+def test_no_domain_is_active_after_a_run(armon, cycles, areas):
+    b = armon.Batch(armon.batch_params(**dict(SCHEME, max_cycles=cycles)), armon.random_specs(3, 2, *areas))
+    b.init()
+    b.begin()
+    b.advance(cycles + 1)
+    b.finish()
+    want = [b.result(d).cycles for d in range(2)]   # a small domain may reach its end time first
+    assert max(want) == cycles
+    for _ in range(2):
+        b.init()
+        b.begin()
+        b.run()
+        assert b.active() == 0
+        b.advance(1)   # nothing left to do
+        assert b.active() == 0
+        assert b.finish() == 0, armon.errors()
+        assert b.active() == 0
+        assert [b.result(d).cycles for d in range(2)] == want
+    b.init()
+    b.begin()
+    b.advance(1)
+    assert b.active() == 2
+    b.finish()
+    b.close()
