@@ -345,12 +345,14 @@ void advance(ArmonBatch* b, int64_t n)
 const DeviceState* last_states(const ArmonBatch* b) { return b->states_at(b->cycles_enqueued); }
 
 // The states before the first cycle, then the EOS and CFL minima of the initial fields and the working
-// buffers (launch_begin).
-void begin_fields(ArmonBatch* b, DeviceState* states)
+// buffers (launch_begin). `keep_eos`: the fields of the EOS stay as they are (the autotuner's).
+void begin_fields(ArmonBatch* b, DeviceState* states, bool keep_eos = false)
 {
     const int n = (int) b->p.size();
+    FieldArrays f = b->fields();
+    if (keep_eos) f.g = nullptr;
     launch_clear(states, n, b->stream);
-    launch_begin(b->fields(), b->d_domains, n, b->domains[0], b->total, states, b->var.eos, 1.4, b->stream);
+    launch_begin(f, b->d_domains, n, b->domains[0], b->total, states, b->var.eos, 1.4, b->stream);
     hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
 }
 
@@ -608,7 +610,7 @@ ARMON_EXPORT int armon_batch_autotune(ArmonBatch* b, ArmonBatchTuning* out)
 {
     try {
         check_ready(b, true, true);
-        begin_fields(b, b->d_tune);
+        begin_fields(b, b->d_tune, true);
         // every domain active with a small positive dt: the work of a real cycle
         std::vector<DeviceState> tune(b->p.size());
         for (auto& s : tune) {

@@ -75,9 +75,11 @@ __global__ void __launch_bounds__(256) k_begin(FieldArrays f, const BatchDomain*
         double p, c, g;
         if (real_cell(d, e - d.offset)) {
             full_eos(eos, gamma, rho, u, v, E, p, c, g);
-            f.p[e] = p;
-            f.c[e] = c;
-            f.g[e] = g;
+            if (f.g) {
+                f.p[e] = p;
+                f.c[e] = c;
+                f.g[e] = g;
+            }
             speeds.add(u, v, c);
         } else if (f.f32[0]) {
             p = f.p[e];

@@ -202,7 +202,7 @@ struct FieldArrays {
 
 // What the first cycle finds: the EOS of the real cells into p, c and g, the CFL minimum of each
 // domain's real cells into its state's accumulators (which must be clear), and a copy of every cell
-// (ghosts included) in the cycles' buffers. One pass over memory and one launch for all domains;
+// (ghosts included) in the cycles' buffers. With a null g, the fields p, c and g stay as they are. One pass over memory and one launch for all domains;
 // `n` domains from `domains`, or the one of `one` when n is 1. `elements`: length of the arrays.
 void launch_begin(const FieldArrays& f, const BatchDomain* domains, int n, const BatchDomain& one, int64_t elements,
                   DeviceState* states, int eos, double gamma, hipStream_t s);

@@ -52,3 +52,18 @@ def test_tiles_by_hand_have_the_bits_of_marches(armon, precision):
         return out
 
     assert all(np.array_equal(x, y) for x, y in zip(run(True), run(False)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [0, 1])
+def test_autotune_leaves_the_initial_fields(armon, precision):
+    """The fields between init and begin are init's, tuned or not; only the work arrays are the tuner's."""
+    b = armon.Batch(armon.batch_params(precision=precision, **SCHEME), armon.random_specs(4, 3, 20 * 20, 60 * 60))
+    b.init()
+    fields = [f for f in armon.FIELD if not f.startswith("work")]
+    before = [[b.read(d, f) for f in fields] for d in range(b.n)]
+    b.autotune()
+    for d in range(b.n):
+        for f, x in zip(fields, before[d]):
+            assert np.array_equal(b.read(d, f), x, equal_nan=True), (d, f)
+    b.close()
