@@ -529,9 +529,11 @@ ARMON_EXPORT ArmonBatch* armon_batch_create(const ArmonParams* common, int n, co
         hip_check(hipMemcpy(b->d_domains, dom.data(), sizeof(BatchDomain) * n, hipMemcpyHostToDevice), "upload domains");
         hip_check(hipMemcpy(b->d_cfgs, cfg.data(), sizeof(TimeStepConfig) * n, hipMemcpyHostToDevice), "upload configs");
         hip_check(hipMemcpy(b->d_init, init.data(), sizeof(BatchInit) * n, hipMemcpyHostToDevice), "upload initial states");
-        // default configuration: 256-cell X tiles of one cell per thread, Y tiles or 256-row Y runs by
-        // the number of cells, one block per work item
-        b->tuning.y_tiles = b->real_cells <= y_tile_max_cells(b->fp64() ? 8 : 4);
+        // default configuration: 256-cell X tiles of one cell per thread, Y tiles or 256-row Y runs,
+        // one block per work item
+        YSweepWork work;
+        for (const ArmonParams& q : b->p) work.add(b->var, q.nx, q.ny, 256);
+        b->tuning.y_tiles = y_takes_tiles(work, b->fp64() ? 8 : 4);
         b->tuning.tile_x = 256;
         b->tuning.x_cells_per_thread = 1;
         b->tuning.grid_x = 0;

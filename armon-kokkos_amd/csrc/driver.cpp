@@ -457,14 +457,16 @@ void fused_enqueue_cycle(ArmonSolver* s, int64_t cycle, Timer* timer)
     int axes[3];
     double factors[3];
     const int n = armon_split_axes(&pc, axes, factors);
-    // the last sweep adds to the bounds that the first one clears, so the two must be apart
-    const bool folded = n > 1 && p.y_run_rows <= 0 &&
-                        (int64_t) p.nx * p.ny <= folded_cells(p.precision == ARMON_PREC_FP64 ? 8 : 4);
+    const SweepVariant var = variant_of(p);
+    const size_t element = p.precision == ARMON_PREC_FP64 ? 8 : 4;
+    // the last sweep adds to the bounds that the first one clears, so the two must be apart; the march
+    // makes no time step
+    const bool folded = n > 1 && p.y_run_rows <= 0 && (int64_t) p.nx * p.ny <= folded_cells(element) &&
+                        (axes[0] == ARMON_AXIS_X || y_takes_tiles(var, element, p.nx, p.ny));
     if (timer) timer->begin();
     if (!folded) launch_time_step(prev, st, tc, s->stream);
     if (timer) timer->end(2);
 
-    const SweepVariant var = variant_of(p);
     // buffer parity at the start of this cycle
     int64_t parity = (cycle * s->sweeps_per_cycle) & 1;
     for (int k = 0; k < n; k++) {

@@ -164,6 +164,19 @@ template int batch_resident_blocks<double>(int, const SweepVariant&, int);
 
 int x_tile_outputs(const SweepVariant& v, int tile) { return tile - 2 * read_extent(v.flux, v.proj); }
 
+bool y_takes_tiles(const YSweepWork& w, size_t element)
+{
+    if (w.cells > y_tile_max_cells(element)) return false;
+    return (double) w.slots <= 0.85 * (double) w.marched * (1.0 + (double) device_simds() / (double) w.waves);
+}
+
+bool y_takes_tiles(const SweepVariant& v, size_t element, int nx, int ny)
+{
+    YSweepWork w;
+    w.add(v, nx, ny, y_run_rows(nx, ny, read_extent(v.flux, v.proj)));
+    return y_takes_tiles(w, element);
+}
+
 void launch_time_step(const DeviceState* prev, DeviceState* st, const TimeStepConfig& c, hipStream_t s)
 {
     k_time_step<<<1, 64, 0, s>>>(prev, st, c);

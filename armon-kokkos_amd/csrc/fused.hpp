@@ -186,6 +186,29 @@ constexpr int y_tile_rows() { return 32; }
 inline int y_tile_outputs(const SweepVariant& v) { return y_tile_rows() - 2 * read_extent(v.flux, v.proj); }
 constexpr int64_t y_tile_max_cells(size_t element) { return element == 8 ? 5 << 19 : 7 << 19; }   // 2.6 M, 3.7 M
 
+// What a Y sweep computes either way, in lanes' cells, summed over its domains: as tiles all of their
+// slots, as marches (runs of `run` rows, one wave per 64 columns) the rows with their warm-up.
+struct YSweepWork {
+    int64_t cells = 0, slots = 0, marched = 0, waves = 0;
+    void add(const SweepVariant& v, int nx, int ny, int run)
+    {
+        const int64_t W = y_tile_outputs(v), groups = (nx + 63) / 64, runs = (ny + run - 1) / run;
+        cells += (int64_t) nx * ny;
+        slots += (int64_t) ((nx + y_tile_cols() - 1) / y_tile_cols()) * ((ny + W - 1) / W) * y_tile_cols() * y_tile_rows();
+        marched += groups * 64 * (ny + 2 * read_extent(v.flux, v.proj) * runs);
+        waves += groups * runs;
+    }
+};
+
+// Whether it takes tiles: up to y_tile_max_cells() cells, where the tiles' rows are filled. A flat domain
+// leaves most of a tile's 24 to 28 output rows empty, where a march has no row too many, so the slots
+// must stay below 0.85 of what the march costs, its rate growing with the waves w as w / (w + SIMDs)
+// (y_run_rows). Y sweep with GAD and second order, us (in brackets slots / cost), march / tile: FP64
+// 100 000 x 8 (1.21) 36.8 / 55.1, 325 000 x 8 (1.66) 73 / 158, 56 000 x 25 (0.98) 53.5 / 68.1, 28 000 x 50
+// (0.74) 54 / 52; FP32 100 000 x 8 21.9 / 26.2, 66 666 x 12 (0.81) 24.2 / 22.2. Squares: 0.67 at most.
+bool y_takes_tiles(const YSweepWork& w, size_t element);
+bool y_takes_tiles(const SweepVariant& v, size_t element, int nx, int ny);   // one domain's, against its best march
+
 // The time step of every domain (one wave each), per-domain configuration.
 void launch_batch_time_step(const DeviceState* prev, DeviceState* states, const TimeStepConfig* cfgs, int n,
                             hipStream_t s);

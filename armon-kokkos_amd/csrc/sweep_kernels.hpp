@@ -1212,12 +1212,10 @@ __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, Begin&& begi
 // 1.5 us each; a tile has a thread per cell or two. The march is the cheaper per cell (its runs are
 // longer than 24 rows, and nothing passes through LDS) once its waves fill the chip: us per Y sweep,
 // march / tile, FP64 512^2 24.7 / 12.1, 1024^2 35.9 / 27.8, 2048^2 86 / 92; FP32 512^2 16.9 / 10.5,
-// 1024^2 23 / 16.9, 2048^2 40 / 41. `max_cells` (2.6 M, 3.7 M): the domains that take tiles.
+// 1024^2 23 / 16.9, 2048^2 40 / 41. y_takes_tiles() has the rule.
 template <class T>
 struct YTile {
     static constexpr int cols = y_tile_cols(), rows = y_tile_rows(), threads = sizeof(T) == 8 ? 512 : 256;
-    static constexpr int64_t max_cells = y_tile_max_cells(sizeof(T));
-    static_assert(folded_cells(sizeof(T)) <= max_cells, "the march makes no time step");
 };
 
 template <class T, int FLUX, int PROJ, int EOS, int DXM, bool FOLD>
@@ -1484,7 +1482,7 @@ void launch_variant(int axis, const SweepArgs<T>& a, hipStream_t s)
     } else {
         using Y = YTile<T>;
         // a run length that the caller gives is a march's
-        if (a.seg_len <= 0 && (int64_t) a.nx * a.ny <= Y::max_cells) {
+        if (a.seg_len <= 0 && y_takes_tiles(SweepVariant{F, P, E}, sizeof(T), a.nx, a.ny)) {
             constexpr int W = Y::rows - 2 * R;
             const int nc = (a.nx + Y::cols - 1) / Y::cols, nb = (a.ny + W - 1) / W;
             const dim3 grid((unsigned) (nc * nb)), block(Y::threads);
@@ -1495,6 +1493,7 @@ void launch_variant(int axis, const SweepArgs<T>& a, hipStream_t s)
             check_launch("sweep_y_tile");
             return;
         }
+        if (a.prev) throw std::logic_error("the march makes no time step");
         // Each block marches down a run of rows of its 256 columns (the warm-up is paid once
         // per run); blocks are numbered row band by row band (segment-major).
         const int ncolblk = (a.nx + kYBlock - 1) / kYBlock;
