@@ -809,14 +809,26 @@ struct MarchLds {
 // fewer: with register windows the unrolled march does not fit the 168 of 3 waves per SIMD; 48 KB
 // with the rest, 3 blocks a CU); in FP32 in registers, where the march has them (100 VGPRs) and is
 // 4% faster so (494 -> 472 us at 8192^2).
-template <class T>
+//
+// E2: whether the projection is of second order. In first order only the fluxes wait, 28 KB in all, and the
+// registers allow 4 waves per SIMD; a block takes 40 KB, for 4 blocks a CU. With 3 (48 KB) GAD's Y sweeps
+// took 5-11% longer: 60 M cells in 7745 columns 799 us and 746 with 4, 6 M in 2450 columns 133 and 120.
+// With 5 Godunov's, bound by memory, took up to 20% longer in 60 M cells (4000 columns 720 us with 3 or 4
+// and 870); with 4 no size lost and the mean gained 7%.
+template <class T, bool E2>
 struct MarchWindows;
 
-template <>
-struct MarchWindows<double> {
-    struct Lds {
+template <bool E2>
+struct MarchWindows<double, E2> {
+    struct SecondOrder {
         double yL[2][kYBlock];
-        Pair<double> cell[2][kYBlock], slope[2][kYBlock], flux[2][kYBlock];
+        Pair<double> cell[2][kYBlock], slope[2][kYBlock];
+    };
+    struct FirstOrder {
+        double unused[6 * kYBlock];
+    };
+    struct Lds : std::conditional_t<E2, SecondOrder, FirstOrder> {
+        Pair<double> flux[2][kYBlock];
     };
     Lds* lds;
     static __device__ __forceinline__ void swap(Pair<double> (&at)[2][kYBlock], const double (&put)[4], double (&got)[4])
@@ -844,8 +856,8 @@ struct MarchWindows<double> {
     }
 };
 
-template <>
-struct MarchWindows<float> {
+template <bool E2>
+struct MarchWindows<float, E2> {
     struct Lds {};
     float cell_[4], flux_[4], slope_[4], yL_[2];
     static __device__ __forceinline__ void swap(float (&at)[4], const float (&put)[4], float (&got)[4])
@@ -881,10 +893,10 @@ struct MarchWindows<float> {
 };
 
 // A block's LDS: one in a kernel, also where that holds two copies of the march.
-template <class T>
+template <class T, bool E2>
 struct MarchBlockLds {
     MarchLds<T> keep;
-    typename MarchWindows<T>::Lds windows;
+    typename MarchWindows<T, E2>::Lds windows;
 };
 
 // The march state of one column of a Y run: sliding windows of the stage results along y. Each row's
@@ -915,9 +927,9 @@ struct YColumn {
     unsigned column;                      // byte offset of the column within a row
     bool lane_ok;                         // false for lanes past the domain
     CflSpeeds speeds;                     // of the column's outputs
-    MarchWindows<T> windows;
+    MarchWindows<T, PROJ == 2> windows;
 
-    __device__ __forceinline__ void init(int x, bool ok, typename MarchWindows<T>::Lds* lds)
+    __device__ __forceinline__ void init(int x, bool ok, typename MarchWindows<T, PROJ == 2>::Lds* lds)
     {
         windows.init(lds);
         column = (unsigned) x * (unsigned) sizeof(T);
@@ -1014,7 +1026,7 @@ struct YColumn {
         u += dtdm_U * (ps[0] - ps[1]);
         E += dtdm_U * (ps[0] * us[2] - ps[1] * us[3]);
         T older[4];                       // cell U-2
-        windows.cell(q[1], older);
+        if constexpr (E2) windows.cell(q[1], older);
 #pragma unroll
         for (int k = 0; k < 4; k++) q[0][k] = q[1][k];
         q[1][0] = rho; q[1][1] = u; q[1][2] = rest.x; q[1][3] = E;
@@ -1097,8 +1109,8 @@ struct YColumn {
 // hold live runs of equal length (most blocks, as the runs are listed longest first) and the
 // independent march otherwise.
 template <class T, int FLUX, int PROJ, int EOS, int DXM, bool STALE, bool SYNC = false>
-__device__ __forceinline__ void sweep_y_run(const SweepArgs<T>& a, T dt, int x, int y0, int y1, MarchBlockLds<T>& lds,
-                                            bool idle = false)
+__device__ __forceinline__ void sweep_y_run(const SweepArgs<T>& a, T dt, int x, int y0, int y1,
+                                            MarchBlockLds<T, PROJ == 2>& lds, bool idle = false)
 {
     using Col = YColumn<T, FLUX, PROJ, EOS, DXM, STALE>;
     constexpr int R = Col::R;
@@ -1146,7 +1158,7 @@ __global__ void __launch_bounds__(kYBlock) ARMON_Y_OCCUPANCY k_sweep_y(SweepArgs
     const int x = (bid - seg * ncolblk) * kYBlock + threadIdx.x;
     const bool idle = x - (int) (threadIdx.x & 63) >= a.nx;   // a wave past the last column
     const int y0 = seg * a.seg_len;
-    __shared__ MarchBlockLds<T> lds;
+    __shared__ MarchBlockLds<T, PROJ == 2> lds;
     sweep_y_run<T, FLUX, PROJ, EOS, DXM, STALE, true>(a, dt, x, y0, min(y0 + a.seg_len, a.ny), lds, idle);
 }
 
@@ -1330,7 +1342,7 @@ template <class T, int FLUX, int PROJ, int EOS, bool STALE>
 __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)))
         k_batch_y(BatchArgs<T> b, const BatchItemY* __restrict__ items, int nitems)
 {
-    __shared__ MarchBlockLds<T> lds;
+    __shared__ MarchBlockLds<T, PROJ == 2> lds;
     const int lane = threadIdx.x & 63;
     const int nwaves = (gridDim.x * blockDim.x) >> 6;
     // the item index is uniform across the wave: keep it (and what is loaded through it) scalar
@@ -1356,7 +1368,7 @@ template <class T, int FLUX, int PROJ, int EOS, bool STALE>
 __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)))
         k_batch_y1(BatchArgs<T> b, const BatchItemY* __restrict__ items, int nitems)
 {
-    __shared__ MarchBlockLds<T> lds;
+    __shared__ MarchBlockLds<T, PROJ == 2> lds;
     const int lane = threadIdx.x & 63;
     const int it = __builtin_amdgcn_readfirstlane((int) ((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
     BatchItemY item{0, 0, 0, 0};
