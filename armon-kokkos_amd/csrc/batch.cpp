@@ -532,7 +532,7 @@ ARMON_EXPORT ArmonBatch* armon_batch_create(const ArmonParams* common, int n, co
         // default configuration: 256-cell X tiles of one cell per thread, Y tiles or 256-row Y runs,
         // one block per work item
         YSweepWork work;
-        for (const ArmonParams& q : b->p) work.add(b->var, q.nx, q.ny, 256);
+        for (const ArmonParams& q : b->p) work.add(b->var, q.nx, q.ny, 256, kWave);
         b->tuning.y_tiles = y_takes_tiles(work, b->fp64() ? 8 : 4);
         b->tuning.tile_x = 256;
         b->tuning.x_cells_per_thread = 1;

@@ -166,14 +166,16 @@ int x_tile_outputs(const SweepVariant& v, int tile) { return tile - 2 * read_ext
 
 bool y_takes_tiles(const YSweepWork& w, size_t element)
 {
-    if (w.cells > y_tile_max_cells(element)) return false;
-    return (double) w.slots <= 0.85 * (double) w.marched * (1.0 + (double) device_simds() / (double) w.waves);
+    const double slots = (double) w.slots, marched = (double) w.marched;
+    if (slots <= (element == 8 ? 0.7 : 0.35) * marched) return true;
+    return w.cells <= y_tile_max_cells(element) &&
+           slots <= 0.85 * marched * (1.0 + (double) device_simds() / (double) w.waves);
 }
 
 bool y_takes_tiles(const SweepVariant& v, size_t element, int nx, int ny)
 {
     YSweepWork w;
-    w.add(v, nx, ny, y_run_rows(nx, ny, read_extent(v.flux, v.proj)));
+    w.add(v, nx, ny, y_run_rows(nx, ny, read_extent(v.flux, v.proj)), kYBlock);
     return y_takes_tiles(w, element);
 }
 

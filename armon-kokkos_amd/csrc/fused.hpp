@@ -187,25 +187,32 @@ inline int y_tile_outputs(const SweepVariant& v) { return y_tile_rows() - 2 * re
 constexpr int64_t y_tile_max_cells(size_t element) { return element == 8 ? 5 << 19 : 7 << 19; }   // 2.6 M, 3.7 M
 
 // What a Y sweep computes either way, in lanes' cells, summed over its domains: as tiles all of their
-// slots, as marches (runs of `run` rows, one wave per 64 columns) the rows with their warm-up.
+// slots, as marches (runs of `run` rows; blocks of `cols` columns, one wave per 64) the rows with their
+// warm-up.
 struct YSweepWork {
     int64_t cells = 0, slots = 0, marched = 0, waves = 0;
-    void add(const SweepVariant& v, int nx, int ny, int run)
+    void add(const SweepVariant& v, int nx, int ny, int run, int cols)
     {
-        const int64_t W = y_tile_outputs(v), groups = (nx + 63) / 64, runs = (ny + run - 1) / run;
+        const int64_t W = y_tile_outputs(v), runs = (ny + run - 1) / run;
         cells += (int64_t) nx * ny;
         slots += (int64_t) ((nx + y_tile_cols() - 1) / y_tile_cols()) * ((ny + W - 1) / W) * y_tile_cols() * y_tile_rows();
-        marched += groups * 64 * (ny + 2 * read_extent(v.flux, v.proj) * runs);
-        waves += groups * runs;
+        marched += (int64_t) ((nx + cols - 1) / cols) * cols * (ny + 2 * read_extent(v.flux, v.proj) * runs);
+        waves += (nx + 63) / 64 * runs;
     }
 };
 
-// Whether it takes tiles: up to y_tile_max_cells() cells, where the tiles' rows are filled. A flat domain
-// leaves most of a tile's 24 to 28 output rows empty, where a march has no row too many, so the slots
-// must stay below 0.85 of what the march costs, its rate growing with the waves w as w / (w + SIMDs)
-// (y_run_rows). Y sweep with GAD and second order, us (in brackets slots / cost), march / tile: FP64
-// 100 000 x 8 (1.21) 36.8 / 55.1, 325 000 x 8 (1.66) 73 / 158, 56 000 x 25 (0.98) 53.5 / 68.1, 28 000 x 50
-// (0.74) 54 / 52; FP32 100 000 x 8 21.9 / 26.2, 66 666 x 12 (0.81) 24.2 / 22.2. Squares: 0.67 at most.
+// Whether it takes tiles.
+//  * Up to y_tile_max_cells() cells, where the tiles' rows are filled: a flat domain leaves most of a tile's
+//    24 to 28 output rows empty, where a march has no row too many, so the slots must stay below 0.85 of
+//    what the march costs, its rate growing with the waves w as w / (w + SIMDs) (y_run_rows). Y sweep with
+//    GAD and second order, us (in brackets slots / cost), march / tile: FP64 100 000 x 8 (1.21) 36.8 / 55.1,
+//    325 000 x 8 (1.66) 73 / 158, 56 000 x 25 (0.98) 53.5 / 68.1, 28 000 x 50 (0.74) 54 / 52; FP32
+//    100 000 x 8 21.9 / 26.2, 66 666 x 12 (0.81) 24.2 / 22.2. Squares: 0.67 at most.
+//  * Of any size, where a march's blocks have many columns past the domain, whose waves hold registers and
+//    LDS to the end: slots below 0.7 (FP64) or 0.35 (FP32) of the march's lanes; a full width has 1.2. 20 M
+//    cells, march / tile, FP64: Godunov and first order 4 columns 7785 / 1090, 64 (0.25) 551 / 320, 130
+//    (0.57) 409 / 317; GAD and second order 100 (0.52) 653 / 486, 130 (0.67) 602 / 499, 180 (0.84) 449 / 473.
+//    FP32: 64 (0.30) 317 / 225; Godunov and first order 100 (0.44) 185 / 194, 130 (0.57) 172 / 211.
 bool y_takes_tiles(const YSweepWork& w, size_t element);
 bool y_takes_tiles(const SweepVariant& v, size_t element, int nx, int ny);   // one domain's, against its best march
 

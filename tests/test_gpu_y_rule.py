@@ -54,3 +54,20 @@ def test_batch_starts_with_what_its_sizes_fill(armon, sizes, tiles):
 
     for x, y in zip(run(), run(y_run_rows=32, y_tiles=not tiles)):
         assert np.array_equal(x, y)
+
+
+# narrow domains take tiles above the limit on cells too: 2.7 M and 3.9 M cells
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nx,ny,scheme", [(5, 780001, GAD2), (64, 61000, GOD1), (130, 30007, GAD2), (257, 15200, GOD1)])
+def test_narrow_domains_above_the_limit(armon, nx, ny, scheme, precision):
+    test_flat_and_narrow_domains_have_the_bits_of_marches(armon, nx, ny, scheme, precision, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny,tiles", [(5, 780001, 1), (40, 100000, 0), (64, 61000, 0), (1000, 3900, 0)])
+def test_batch_of_a_narrow_domain(armon, nx, ny, tiles):
+    spec = armon.ArmonDomainSpec(test=armon.TESTS["Sod"], nx=nx, ny=ny, state=armon.reference_state("Sod"))
+    b = armon.Batch(armon.batch_params(max_cycles=4, verbose=5, **GAD2), [spec])
+    assert b.tuning().y_tiles == tiles
+    b.close()
