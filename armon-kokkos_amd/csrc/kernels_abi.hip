@@ -629,16 +629,21 @@ __global__ void __launch_bounds__(kBlock) k_advection_second_order_y(Iter2D it, 
     }
 }
 
-// Ghost layers [w0, w1), one per blockIdx.y: a layer's cells are written from real cells that no layer
-// writes (disp is not 0), so the layers need not wait for each other (one thread doing 4 of them in
-// turn took 8 us, mostly latency; 3.5 us so).
+// Ghost layers [w0, w1), dealt to threadIdx.x and blockIdx.y, of the border's elements, dealt to
+// threadIdx.y and blockIdx.x: a layer's cells are written from real cells that no layer writes (disp is
+// not 0), so the layers need not wait for each other (one thread doing 4 of them in turn took 8 us,
+// mostly latency; 3.5 us so). Layers that adjoin in their rows (disp 1 or -1) share lines, so they go to
+// neighbouring lanes of one wave: one layer a block, different XCDs wrote parts of the same lines (4
+// layers of 30 000 rows 26-28 us, now 5.5-6; of a million rows of 7 cells 580-1210, now 172-368).
 __global__ void __launch_bounds__(kBlock) k_boundary_conditions(Iter1D it, int64_t w0, int64_t w1, int64_t disp,
                                                                 flt_t u_factor, flt_t v_factor, flt_t* rho,
                                                                 flt_t* umat, flt_t* vmat, flt_t* pmat, flt_t* cmat,
                                                                 flt_t* gmat, flt_t* Emat)
 {
-    for (int64_t w = w0 + blockIdx.y; w < w1; w += gridDim.y)
-        for_each_1d(it, [&](int64_t, int64_t border) {
+    for (int64_t w = w0 + (int64_t) blockIdx.y * blockDim.x + threadIdx.x; w < w1; w += (int64_t) gridDim.y * blockDim.x)
+        for (int64_t k = it.start + (int64_t) blockIdx.x * blockDim.y + threadIdx.y; k < it.end;
+             k += (int64_t) gridDim.x * blockDim.y) {
+            const int64_t border = k * it.step + it.base;
             const int64_t i = border - w * disp, ip = border + (w + 1) * disp;
             const flt_t r = rho[ip], u = umat[ip], v = vmat[ip], p = pmat[ip], c = cmat[ip], g = gmat[ip],
                         E = Emat[ip];
@@ -649,7 +654,7 @@ __global__ void __launch_bounds__(kBlock) k_boundary_conditions(Iter1D it, int64
             cmat[i] = c;
             gmat[i] = g;
             Emat[i] = E;
-        });
+        }
 }
 
 // Element k of a border's range, for each k once. A border is a few columns of many rows: its
@@ -1319,13 +1324,14 @@ ARMON_KERNEL_TRY
     if (empty_1d(it) || stencil_width <= 0) return;
     // a displacement of 0 maps every layer to the border itself: one layer after the other
     const int64_t together = disp != 0 ? stencil_width : 1;
-    for (int64_t w = 0; w < stencil_width; w += together) {
-        dim3 grid = grid_1d(it);
-        grid.y = (unsigned) (together < 65535 ? together : 65535);
-        k_boundary_conditions<<<grid, kBlock, 0, stream()>>>(it, w, w + together, disp, u_factor, v_factor, rho.data,
-                                                             umat.data, vmat.data, pmat.data, cmat.data, gmat.data,
-                                                             Emat.data);
-    }
+    const unsigned lanes = disp == 1 || disp == -1 ? (unsigned) (together < 16 ? together : 16) : 1;
+    const dim3 block(lanes, kBlock / lanes);
+    const int64_t gx = (it.end - it.start + block.y - 1) / block.y, gy = (together + lanes - 1) / lanes;
+    const dim3 grid((unsigned) (gx < 65536 ? gx : 65536), (unsigned) (gy < 65535 ? gy : 65535));
+    for (int64_t w = 0; w < stencil_width; w += together)
+        k_boundary_conditions<<<grid, block, 0, stream()>>>(it, w, w + together, disp, u_factor, v_factor, rho.data,
+                                                            umat.data, vmat.data, pmat.data, cmat.data, gmat.data,
+                                                            Emat.data);
     after_launch("boundary_conditions");
 }
 ARMON_KERNEL_CATCH("boundary_conditions")
