@@ -214,17 +214,20 @@ dim3 grid_2d_aligned(const Iter2D& it)
 }
 
 // How far the kernels that run down columns may shift a run's columns to start on a line: kAlignSlack, or 0
-// for not at all. Aligned, the second-order advection and the GAD fluxes take 11% and 5% less time at
-// 5000^2 (416 -> 368, 263 -> 250 us). Where the row is so close to a whole number of blocks that the shift
-// adds a column of blocks, its cost decides, and with 8 k block columns unshifted the runs above each
-// other share an XCD's L2: advection 1024^2 16.9 -> 17.9, 2048^2 65.5 -> 66.2, 3072^2 161 -> 153, 4096^2
-// 274 -> 254, 6144^2 600 -> 553, 8192^2 1040 -> 1108 us, so from 12 to 24 block columns; GAD 14.6 -> 15.4,
-// 44.6 -> 42.3, 103.5 -> 102.8, 173 -> 169, 380 -> 395, 662 -> 661 us: not.
-int run_slack(int64_t len, bool advection)
+// for not at all. Where no column of blocks is added the shift costs nothing and gains 5-11% (5000^2:
+// second-order advection 416 -> 368 us, GAD 263 -> 250). Where the row is so close to a whole number of
+// blocks that one is added, the advection still gains more than that costs from 12 columns of blocks on,
+// unless its 9 arrays stay in the Infinity Cache. Time with the shift over that without, on the same
+// buffers, three placements: FP64 squares of 8 columns of blocks 0.93-1.00, 10 0.95-0.97, 11 0.98, 12
+// 0.94-0.95, 13 0.97-0.99, 16 0.93-0.94, 20 0.92-0.93, 25 0.98, 28 0.92-0.95, 32 0.98-1.01, 33 0.90-0.94;
+// 4096 x 9000 0.93-0.94, 16384 x 1500 0.92-0.95, 3328 x 9000 1.01; float the same within 0.03, but in the
+// cache (4096 x 1000, 147 MB) 1.07-1.09. GAD: not, in float it loses up to 5% below 20 columns of blocks.
+int run_slack(int64_t len, int64_t rows, bool advection)
 {
+    constexpr int64_t kInfinityCache = 256 << 20;
     const int64_t blocks = (len + kBlock - 1) / kBlock;
-    const bool free = (len + kAlignSlack + kBlock - 1) / kBlock == blocks;
-    return free || (advection && blocks >= 12 && blocks <= 24) ? kAlignSlack : 0;
+    if ((len + kAlignSlack + kBlock - 1) / kBlock == blocks) return kAlignSlack;
+    return advection && blocks >= 12 && 9 * (int64_t) sizeof(flt_t) * len * rows > kInfinityCache ? kAlignSlack : 0;
 }
 
 dim3 grid_1d(const Iter1D& it)
@@ -1104,7 +1107,7 @@ ARMON_KERNEL_TRY
             const int64_t groups = (it.len + 63) / 64;
             if (groups * ((rows + run - 1) / run) < 8192) run = 4;
             const int64_t nruns = (rows + run - 1) / run;
-            const int slack = run_slack(it.len, false);
+            const int slack = run_slack(it.len, rows, false);
             const dim3 g((unsigned) ((it.len + slack + kBlock - 1) / kBlock), (unsigned) (nruns < 65535 ? nruns : 65535));
             k_acoustic_GAD_y<LL><<<g, kBlock, 0, stream()>>>(it, run, slack, dt, dx, ustar.data, pstar.data, rho.data,
                                                              u.data, pmat.data, cmat.data);
@@ -1285,7 +1288,7 @@ ARMON_KERNEL_TRY
         const int64_t groups = (it.len + 63) / 64;
         if (groups * ((rows + run - 1) / run) < 8192) run = 4;
         const int64_t nruns = (rows + run - 1) / run;
-        const int slack = run_slack(it.len, true);
+        const int slack = run_slack(it.len, rows, true);
         const dim3 g((unsigned) ((it.len + slack + kBlock - 1) / kBlock), (unsigned) (nruns < 65535 ? nruns : 65535));
         k_advection_second_order_y<<<g, kBlock, 0, stream()>>>(it, run, slack, dx, dt, ustar.data, rho.data, umat.data,
                                                                vmat.data, Emat.data, advection_rho.data,
