@@ -291,9 +291,11 @@ void enqueue_cycle(ArmonBatch* b, int64_t cycle, Timer* t)
     // the first sweep makes the time step where each of its blocks has one item
     const bool single = axes[0] == ARMON_AXIS_X ? b->tuning.grid_x == 0 : b->tuning.y_tiles != 0;
     const bool folded = n > 1 && single && b->real_cells <= folded_cells(b->fp64() ? 8 : 4);
-    if (t) t->begin();
-    if (!folded) launch_batch_time_step(prev, states, b->d_cfgs, (int) b->p.size(), b->stream);
-    if (t) t->end(2);
+    if (!folded) {
+        if (t) t->begin();
+        launch_batch_time_step(prev, states, b->d_cfgs, (int) b->p.size(), b->stream);
+        if (t) t->end(2);
+    }
     int parity = (int) ((cycle * b->sweeps_per_cycle) & 1);
     for (int k = 0; k < n; k++) {
         if (t) t->begin();

@@ -463,9 +463,11 @@ void fused_enqueue_cycle(ArmonSolver* s, int64_t cycle, Timer* timer)
     // makes no time step
     const bool folded = n > 1 && p.y_run_rows <= 0 && (int64_t) p.nx * p.ny <= folded_cells(element) &&
                         (axes[0] == ARMON_AXIS_X || y_takes_tiles(var, element, p.nx, p.ny));
-    if (timer) timer->begin();
-    if (!folded) launch_time_step(prev, st, tc, s->stream);
-    if (timer) timer->end(2);
+    if (!folded) {
+        if (timer) timer->begin();
+        launch_time_step(prev, st, tc, s->stream);
+        if (timer) timer->end(2);
+    }
 
     // buffer parity at the start of this cycle
     int64_t parity = (cycle * s->sweeps_per_cycle) & 1;

@@ -208,7 +208,8 @@ typedef struct ArmonResult {
 } ArmonResult;
 
 typedef struct ArmonKernelTimes {
-    int launches[4];      /* [0] X sweeps, [1] Y sweeps, [2] time-step kernels, [3] other */
+    int launches[4];      /* [0] X sweeps, [1] Y sweeps, [2] time-step kernels (none where a cycle's first
+                             sweep makes the time step), [3] other */
     double total_ms[4];   /* summed HIP-event durations per kernel class */
 } ArmonKernelTimes;
 
