@@ -578,8 +578,11 @@ BatchDomain own_domain(const ArmonSolver* s)
 void fused_begin(ArmonSolver* s)
 {
     ArmonParams& p = s->p;
-    launch_clear(s->st, 1, s->stream);
-    launch_begin(field_arrays(s), nullptr, 1, own_domain(s), s->n, s->st, p.test == 3 ? 1 : 0, 1.4, s->stream);
+    {
+        Stage st(s->clock, "EOS_init", nullptr);   // the graphs below are not part of it
+        launch_clear(s->st, 1, s->stream);
+        launch_begin(field_arrays(s), nullptr, 1, own_domain(s), s->n, s->st, p.test == 3 ? 1 : 0, 1.4, s->stream);
+    }
     hip_check(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
     s->cycles_enqueued = 0;
     // both graphs now, so that no later advance pays for a capture
@@ -1060,7 +1063,6 @@ ARMON_EXPORT int armon_solver_begin(ArmonSolver* s)
         s->compare_stop = false;
         armon_update_axis(&p, ARMON_AXIS_X);
         if (p.engine == ARMON_ENGINE_FUSED) {
-            Stage st(s->clock, "EOS_init", nullptr);
             fused_begin(s);
         } else {
             { Stage st(s->clock, "EOS_init", nullptr); staged_update_EOS(s); }
