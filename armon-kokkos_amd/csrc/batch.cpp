@@ -125,12 +125,6 @@ void fail(const char* where, const std::exception& e)
     else report_std(where, e);
 }
 
-// Work lists. X: every tile of every domain's stream of padded rows (the tile mapping of
-// sweep_x_tile: tiles of W outputs overlapping by 2R slots). Y: every (64-column group, run of
-// at most `run` rows) of every domain, band by band, so that the waves of a block march
-// neighbouring column groups of one band (measured 2% faster in FP64 and 12% in FP32-mixed
-// than column group by column group); then longest runs first (a stable sort) so that a
-// grid-stride walk over them balances well. Y tiles: band by band too.
 // Destroys the captured graphs: they hold the work lists' addresses and the launch grids.
 void drop_graphs(ArmonBatch* b)
 {
@@ -142,6 +136,12 @@ void drop_graphs(ArmonBatch* b)
     }
 }
 
+// Work lists. X: every tile of every domain's stream of padded rows (the tile mapping of
+// sweep_x_tile: tiles of W outputs overlapping by 2R slots). Y: every (64-column group, run of
+// at most `run` rows) of every domain, band by band, so that the waves of a block march
+// neighbouring column groups of one band (measured 2% faster in FP64 and 12% in FP32-mixed
+// than column group by column group); then longest runs first (a stable sort) so that a
+// grid-stride walk over them balances well. Y tiles: band by band too.
 void build_items(ArmonBatch* b, int run)
 {
     drop_graphs(b);

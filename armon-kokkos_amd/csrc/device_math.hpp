@@ -513,7 +513,7 @@ template <class T> __device__ __forceinline__ void perfect_gas_pc(T gamma, T rho
 
 // bizarrium without g, with y = shared_recip(rho): the quotients by rho and by 1 - s x go through two
 // shared reciprocals, the one by the constant rho0 through its own (div_by_recip); 5 divisions fewer.
-// Each f is part of the next, so a NaN from any of them reaches f3.
+// Each f is part of the next, so a NaN from any of them reaches f2.
 __device__ __forceinline__ void bizarrium_pc(double rho, double E, double u, double v, double y, double& p, double& c)
 {
     const double rho0 = 1e4, K0 = 1e11, Cv0 = 1e3, T0 = 300, eps0 = 0;

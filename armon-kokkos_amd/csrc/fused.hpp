@@ -280,10 +280,14 @@ private:
 // behind it, unless the report before it says that no cycle will be left. Where that guess is wrong,
 // as the time step changes, the run takes a little longer.
 //
-// Cycles after the end change no state, and in small domains whole chunks, each one graph, are the
-// fastest. A large domain's blocks take their time to come and go all the same, 1.2 ns each (an X sweep
-// of 8192^2 160 us, 1.9 ms of a run of 100 cycles in chunks of 16): from kWholeChunks `cells` on, no
-// more cycles are enqueued than the report leaves, the rest of a chunk launch by launch.
+// Cycles after the end change no state, but their blocks take their time to come and go, 1.3 ns each: such an
+// X sweep takes 352 us at 8192^2 in FP64 (270 900 blocks) and 177 in FP32 (133 300, two cells a thread), 95 and
+// 41 at 4096^2, 24 and 14 at 2048^2. From kWholeChunks `cells` on, no more cycles are enqueued than the
+// report leaves, the rest of a chunk launch by launch: 100 cycles of 8192^2 in chunks of 16, of which 12 are
+// past the end, 190 -> 187 ms in FP64 and 94 -> 90 in FP32, 33 cycles of 4096^2 18.6 -> 17.0 and 9.6 -> 9.0.
+// Smaller domains enqueue whole chunks, though the rest one by one would be the faster there too (100 cycles
+// of 128^2 1.13 -> 1.10 ms, of 1024^2 4.83 -> 4.70, of 2048^2 14.9 -> 14.6): a run's graph launches, which
+// the table of stage times counts, are then whole ones (20 cycles in chunks of 8 are 3).
 constexpr int64_t kWholeChunks = 1 << 22;
 
 template <class Enqueue, class Config>

@@ -122,6 +122,9 @@ struct LoadedCell {
 // Cell `k` (along the sweep axis, `n` real cells) of the pencil whose cell 0 lies `first` elements
 // past `base` (the same for the whole wave) and whose cells lie `stride` apart. Real cells are
 // loaded; ghost layers 1..stencil_width mirror real cells; deeper ghost layers are read as they are.
+// The byte offsets fit 32 bits: a row has fewer than 2^23 real cells (the fused engine takes no longer
+// ones) and at most 8.4 M with its ghosts, as a domain's index allows 2^31 - 1 cells in all; an X tile
+// stays within one such row or some short ones, a Y tile within 31 rows of its base, 2.1 GB in FP64.
 template <class T>
 __device__ __forceinline__ LoadedCell<T> fetch_cell(const SweepArgs<T>& a, int64_t base, int first, int k, int stride,
                                                     int n)
@@ -173,8 +176,9 @@ __device__ __forceinline__ Cell<T> make_cell(const SweepArgs<T>& a, int64_t base
     return cell;
 }
 
-// The Y march loads a row's state one row before it makes the cell: where row `k` comes from (the same for the whole wave: the row it is read at, the mirror side
-// or staleness), then the cell from the loaded state.
+// The Y march loads a row's state one row before it makes the cell: where row `k` comes from (the same
+// for the whole wave: the row it is read at, the mirror side or staleness), then the cell from the loaded
+// state.
 struct RowSource {
     int row;
     int mirror;
@@ -677,8 +681,9 @@ __device__ __forceinline__ void tile_sweep(T dx, T inv_dx, T dt, SchemeLds<T, FL
 }
 
 // One X tile of the domain described by `a`; `begin(dt)` gives the cycle's dt, or false where the cycle
-// does not run (the same for the whole block). Called by all TILE / CPT threads of a block; each thread computes CPT cells of the tile, at slots t, t + TILE / CPT, ...
-// (consecutive lanes on consecutive slots for every load and store).
+// does not run (the same for the whole block). Called by all TILE / CPT threads of a block; each thread
+// computes CPT cells of the tile, at slots t, t + TILE / CPT, ... (consecutive lanes on consecutive slots
+// for every load and store).
 //
 // The rows of the domain are laid end to end as a stream of slots, each row taking
 // x_slots = nx + 2R slots (its R ghost cells on each side, then the next row). A tile covers
@@ -1407,7 +1412,6 @@ inline unsigned grid_for(int64_t n, int block, int64_t max_blocks)
     return (unsigned) g;
 }
 
-// Blocks of `block` threads of `kernel` resident on the whole device at once.
 // How the tiles of a single domain add to its CFL accumulators (see reduce_cfl): up to 4096 waves without
 // a look. Cycle with -> without it, us: 128^2 FP64 10.2 -> 9.9, 512^2 FP32 (2816 waves) 13.1 -> 12.0,
 // 512^2 FP64 (5632) 17.8 -> 18.1, 1024^2 FP64 (22 016) 45.6 -> 50.5.
@@ -1416,6 +1420,7 @@ inline int reduce_mode(int reduce, int64_t blocks, int threads)
     return reduce && blocks * (threads / 64) <= 4096 ? REDUCE_UNSEEN : reduce;
 }
 
+// Blocks of `block` threads of `kernel` resident on the whole device at once.
 inline int resident_blocks(const void* kernel, int block)
 {
     int dev = 0, per_cu = 0, cus = 0;
