@@ -46,22 +46,15 @@ constexpr int kTile = 256;    // X sweep: cells per tile (FP64 single-domain swe
 constexpr int kYBlock = 256;  // Y sweep: columns per block
 
 // Y march: rows per unrolled loop body (FP64: 4 rows spill, 1 row moves its windows, 982 -> 992 us at
-// 8192^2) and the minimum waves per SIMD the register allocation must allow (0: the compiler's choice).
+// 8192^2) and the minimum waves per SIMD the register allocation must allow.
 #ifndef ARMON_Y_UNROLL_FP64
 #define ARMON_Y_UNROLL_FP64 2
 #endif
 #ifndef ARMON_Y_UNROLL_FP32
 #define ARMON_Y_UNROLL_FP32 2
 #endif
-#ifndef ARMON_Y_WAVES_PER_EU
-#define ARMON_Y_WAVES_PER_EU 3   // the FP64 march's occupancy (168 VGPRs); 0: no hint
-#endif
 constexpr int kYUnrollFp64 = ARMON_Y_UNROLL_FP64, kYUnrollFp32 = ARMON_Y_UNROLL_FP32;
-#if ARMON_Y_WAVES_PER_EU > 0
-#define ARMON_Y_OCCUPANCY __attribute__((amdgpu_waves_per_eu(ARMON_Y_WAVES_PER_EU)))
-#else
-#define ARMON_Y_OCCUPANCY
-#endif
+constexpr int kYWaves = 3, kYWavesFirstOrder = 4;   // 168 and 128 VGPRs
 
 template <class T>
 struct Cell {
@@ -803,10 +796,12 @@ __device__ __forceinline__ void push(T (&w)[N], T v)
 // What a thread of the march keeps in LDS until a later row, off the arithmetic's dependency chains
 // (a slot is read before the row that wraps round to it writes it): the parts of a cell that the
 // faces do not read and, for the CFL bound, its sound speed.
-template <class T>
+// The update takes them two rows later with GAD, else one; the bound R rows later, with GAD 3 or 4.
+template <class T, int FLUX, int PROJ>
 struct MarchLds {
-    Pair<T> ut_E[2][kYBlock];
-    T dtdm[2][kYBlock], c[4][kYBlock];
+    static constexpr int kRows = FLUX > 0 ? 2 : 1, kBounds = FLUX > 0 ? 4 : PROJ == 2 ? 3 : 2;
+    Pair<T> ut_E[kRows][kYBlock];
+    T dtdm[kRows][kYBlock], c[kBounds][kYBlock];
 };
 
 // What else waits for the next row or two: the reciprocal of an updated cell's length, its slopes and
@@ -815,11 +810,7 @@ struct MarchLds {
 // with the rest, 3 blocks a CU); in FP32 in registers, where the march has them (100 VGPRs) and is
 // 4% faster so (494 -> 472 us at 8192^2).
 //
-// E2: whether the projection is of second order. In first order only the fluxes wait, 28 KB in all, and the
-// registers allow 4 waves per SIMD; a block takes 40 KB, for 4 blocks a CU. With 3 (48 KB) GAD's Y sweeps
-// took 5-11% longer: 60 M cells in 7745 columns 799 us and 746 with 4, 6 M in 2450 columns 133 and 120.
-// With 5 Godunov's, bound by memory, took up to 20% longer in 60 M cells (4000 columns 720 us with 3 or 4
-// and 870); with 4 no size lost and the mean gained 7%.
+// E2: whether the projection is of second order; in first order only the fluxes wait.
 template <class T, bool E2>
 struct MarchWindows;
 
@@ -829,9 +820,7 @@ struct MarchWindows<double, E2> {
         double yL[2][kYBlock];
         Pair<double> cell[2][kYBlock], slope[2][kYBlock];
     };
-    struct FirstOrder {
-        double unused[6 * kYBlock];
-    };
+    struct FirstOrder {};
     struct Lds : std::conditional_t<E2, SecondOrder, FirstOrder> {
         Pair<double> flux[2][kYBlock];
     };
@@ -897,12 +886,28 @@ struct MarchWindows<float, E2> {
     }
 };
 
-// A block's LDS: one in a kernel, also where that holds two copies of the march.
-template <class T, bool E2>
-struct MarchBlockLds {
-    MarchLds<T> keep;
-    typename MarchWindows<T, E2>::Lds windows;
+template <size_t BYTES>
+struct Unused {
+    char bytes[BYTES];
 };
+template <>
+struct Unused<0> {};
+
+// A block's LDS: one in a kernel, also where that holds two copies of the march. In FP64 GAD and second order
+// take 48 KB, for 3 blocks a CU, as their registers allow; the others 40 KB, for 4, with what they need
+// (18 to 40 KB) and some unused. With 3 blocks they took 8% longer on the mean of 50 sizes of 6 M to 60 M
+// cells (GAD and first order 60 M in 7745 columns 792 us and 745 with 4; Godunov and second order in 520
+// columns 1023 and 898). With 5 Godunov and first order, bound by memory, took up to 20% longer in 60 M
+// cells (4000 columns 720 us with 3 or 4 and 870).
+template <class T, int FLUX, int PROJ>
+struct MarchParts {
+    MarchLds<T, FLUX, PROJ> keep;
+    typename MarchWindows<T, PROJ == 2>::Lds windows;
+};
+template <class T, int FLUX, int PROJ>
+struct MarchBlockLds : MarchParts<T, FLUX, PROJ>,
+                       Unused<sizeof(T) == 8 && sizeof(MarchParts<T, FLUX, PROJ>) < 40960
+                                      ? 40960 - sizeof(MarchParts<T, FLUX, PROJ>) : 0> {};
 
 // The march state of one column of a Y run: sliding windows of the stage results along y. Each row's
 // state is loaded one row before it is used (with STALE = false, when the stencil width covers the
@@ -974,7 +979,7 @@ struct YColumn {
 
     // Row n of a run that outputs rows [y0, y1).
     __device__ __forceinline__ void step(const SweepArgs<T>& a, T dt, T dx, T inv_dx, int n, int y0, int y1,
-                                         MarchLds<T>& keep)
+                                         MarchLds<T, FLUX, PROJ>& keep)
     {
         const int t = threadIdx.x;
         // Keeps the column's offset out of the loop-invariant addresses that the compiler would make
@@ -993,14 +998,17 @@ struct YColumn {
         p = cn.p;
         T dtdm = mass_quotient<DXM>(dt, dm[2], cn.y, inv_dx);
         if (__builtin_expect(unusable(dtdm), 0)) dtdm = dv<T>(dt, dm[2]);
-        // what is left of cell U (the one before n, or two before it) and the sound speed of cell n-4
+        // what is left of cell U (the one before n, or two before it) and the sound speed of cell n-R
         constexpr int W = GAD ? 0 : 1;    // window index of cell U among n-2, n-1, n
-        const Pair<T> rest = keep.ut_E[(n + W) & 1][t];
-        const T dtdm_U = keep.dtdm[(n + W) & 1][t];
-        const T c_P = keep.c[(n - R) & 3][t];
-        keep.ut_E[n & 1][t] = {cn.ut, cn.E};
-        keep.dtdm[n & 1][t] = dtdm;
-        keep.c[n & 3][t] = cn.c;
+        constexpr unsigned kBounds = MarchLds<T, FLUX, PROJ>::kBounds;
+        const int row = GAD ? n & 1 : 0;
+        const unsigned bound = (unsigned) (n + 4) % kBounds, bound_P = (unsigned) (n + 4 + (int) kBounds - R) % kBounds;
+        const Pair<T> rest = keep.ut_E[row][t];
+        const T dtdm_U = keep.dtdm[row][t];
+        const T c_P = keep.c[bound_P][t];
+        keep.ut_E[row][t] = {cn.ut, cn.E};
+        keep.dtdm[row][t] = dtdm;
+        keep.c[bound][t] = cn.c;
 
         // Godunov at face n (cells n-1 | n).
         T gu, gp;
@@ -1115,7 +1123,7 @@ struct YColumn {
 // independent march otherwise.
 template <class T, int FLUX, int PROJ, int EOS, int DXM, bool STALE, bool SYNC = false>
 __device__ __forceinline__ void sweep_y_run(const SweepArgs<T>& a, T dt, int x, int y0, int y1,
-                                            MarchBlockLds<T, PROJ == 2>& lds, bool idle = false)
+                                            MarchBlockLds<T, FLUX, PROJ>& lds, bool idle = false)
 {
     using Col = YColumn<T, FLUX, PROJ, EOS, DXM, STALE>;
     constexpr int R = Col::R;
@@ -1154,7 +1162,8 @@ __device__ __forceinline__ void sweep_y_run(const SweepArgs<T>& a, T dt, int x, 
 }
 
 template <class T, int FLUX, int PROJ, int EOS, int DXM, bool STALE>
-__global__ void __launch_bounds__(kYBlock) ARMON_Y_OCCUPANCY k_sweep_y(SweepArgs<T> a, int ncolblk)
+__global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(PROJ == 2 ? kYWaves : kYWavesFirstOrder)))
+        k_sweep_y(SweepArgs<T> a, int ncolblk)
 {
     if (!a.st->active) return;
     const T dt = (T) (a.st->current_dt * a.dt_factor);
@@ -1163,7 +1172,7 @@ __global__ void __launch_bounds__(kYBlock) ARMON_Y_OCCUPANCY k_sweep_y(SweepArgs
     const int x = (bid - seg * ncolblk) * kYBlock + threadIdx.x;
     const bool idle = x - (int) (threadIdx.x & 63) >= a.nx;   // a wave past the last column
     const int y0 = seg * a.seg_len;
-    __shared__ MarchBlockLds<T, PROJ == 2> lds;
+    __shared__ MarchBlockLds<T, FLUX, PROJ> lds;
     sweep_y_run<T, FLUX, PROJ, EOS, DXM, STALE, true>(a, dt, x, y0, min(y0 + a.seg_len, a.ny), lds, idle);
 }
 
@@ -1347,7 +1356,7 @@ template <class T, int FLUX, int PROJ, int EOS, bool STALE>
 __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)))
         k_batch_y(BatchArgs<T> b, const BatchItemY* __restrict__ items, int nitems)
 {
-    __shared__ MarchBlockLds<T, PROJ == 2> lds;
+    __shared__ MarchBlockLds<T, FLUX, PROJ> lds;
     const int lane = threadIdx.x & 63;
     const int nwaves = (gridDim.x * blockDim.x) >> 6;
     // the item index is uniform across the wave: keep it (and what is loaded through it) scalar
@@ -1370,10 +1379,10 @@ __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)
 // block marches them with the block barrier of sweep_y_run (same trip count for every wave),
 // which keeps their accesses of a row together in DRAM.
 template <class T, int FLUX, int PROJ, int EOS, bool STALE>
-__global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(PROJ == 2 ? kYWaves : kYWavesFirstOrder)))
         k_batch_y1(BatchArgs<T> b, const BatchItemY* __restrict__ items, int nitems)
 {
-    __shared__ MarchBlockLds<T, PROJ == 2> lds;
+    __shared__ MarchBlockLds<T, FLUX, PROJ> lds;
     const int lane = threadIdx.x & 63;
     const int it = __builtin_amdgcn_readfirstlane((int) ((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
     BatchItemY item{0, 0, 0, 0};
@@ -1382,12 +1391,14 @@ __global__ void __launch_bounds__(kYBlock) __attribute__((amdgpu_waves_per_eu(3)
         item = items[it];
         live = b.states[item.domain].active != 0;
     }
-    __shared__ int rows_of_wave[kYBlock / 64];
+    // in the march's LDS: 16 bytes more would leave room for a block less
+    int* rows_of_wave = reinterpret_cast<int*>(&lds);
     if (lane == 0) rows_of_wave[threadIdx.x >> 6] = live ? item.y1 - item.y0 : -1;
     __syncthreads();
     bool sync = true;
 #pragma unroll
     for (int w = 0; w < kYBlock / 64; w++) sync = sync && rows_of_wave[w] == rows_of_wave[0] && rows_of_wave[w] >= 0;
+    __syncthreads();
     if (!live) return;   // the whole wave; never in a synchronised block
     const DeviceState* st = b.states + item.domain;
     const SweepArgs<T> a = batch_domain_args(b, item.domain, 1);
